@@ -67,6 +67,8 @@ static void release(Ctx& c)
   if (c.partials) hipFree(c.partials);
   if (c.ke_part) hipFree(c.ke_part);
   c.ke_part = nullptr;
+  if (c.red_part) hipFree(c.red_part);
+  c.red_part = nullptr;
   if (c.low_part) hipFree(c.low_part);
   if (c.low_red) hipFree(c.low_red);
   if (c.low_coef) hipFree(c.low_coef);
@@ -217,6 +219,7 @@ int cup_create(const cup_grid_desc* d, cup_ctx** out)
                         "hipHostMalloc")))
       break;
     if ((rc = ensure_partials(c, 20 * (size_t)c.nb + 1024))) break;
+    if ((rc = check_hip(c, hipMalloc(&c.red_part, REDUCE_CHUNKS * 32 * sizeof(double)), "hipMalloc reduction"))) break;
     if ((rc = check_hip(c, hipMalloc(&c.ke_part, 4 * (size_t)c.nb * sizeof(double)), "hipMalloc ke"))) break;
     if ((rc = check_hip(c, hipMemsetAsync(c.ke_part, 0, 4 * (size_t)c.nb * sizeof(double), c.stream), "memset ke")))
       break;

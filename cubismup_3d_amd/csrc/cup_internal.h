@@ -72,6 +72,7 @@ struct DevScalars {
   unsigned long long umax_slots[2][256];
 };
 constexpr int UMAX_SLOTS = 256;
+constexpr int REDUCE_CHUNKS = 256;  // workgroups per component of a large reduction (launch_reduce)
 
 // Radix plan of a transform length that is not a power of two (FFT passes with the length
 // known at run time): n = r[0] r[1] ... r[ns-1], radices 8, 4, 2, 3, 5.
@@ -169,6 +170,7 @@ struct Ctx {
   void* ghat = nullptr;   // (padded grid) the Green's function's spectrum, FP64 complex
   double* partials = nullptr;
   size_t partials_cap = 0;  // doubles
+  double* red_part = nullptr;  // launch_reduce's first stage: [REDUCE_CHUNKS][up to 32 components]
   double* ke_part = nullptr;  // [nb][4] partial sums |u|^2 of the fused step's velocity (per wave)
   DevScalars* sc = nullptr;
   DevScalars* sc_host = nullptr;  // pinned

@@ -7,6 +7,7 @@
 // BlockLab::load with periodic wrap), then computes 2 cells per thread.
 #include "cup_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -1518,24 +1519,50 @@ int launch_gradp_fused(Ctx& c, const double uinf[3], const int* skip_slot, bool 
 
 // ------------------------------------------------------------------- reductions
 
-// One workgroup per component; component i of partial j at part[j*width + i].
+// Component i of partial j at part[j*width + i]; grid (width, nchunk): workgroup (i, c) reduces
+// component i of chunk c of the partials into out[c*width + i]. Each thread keeps 8 loads in
+// flight (a single workgroup is bound by the latency of its loads, about 1 ns per partial one
+// load at a time); the lanes' and chunks' order is fixed, so the result is deterministic.
 __global__ __launch_bounds__(NT) void k_reduce(const double* __restrict__ part, int n, int width, unsigned maxmask,
                                                double* __restrict__ out)
 {
+  constexpr int U = 8;
   const int i = blockIdx.x;
   const bool ismax = (maxmask >> i) & 1;
-  double a[1] = {ismax ? -INFINITY : 0.0};
-  for (int j = threadIdx.x; j < n; j += NT) {
-    const double x = part[(size_t)j * width + i];
-    a[0] = ismax ? fmax(a[0], x) : a[0] + x;
+  const double none = ismax ? -INFINITY : 0.0;
+  const int per = (n + gridDim.y - 1) / gridDim.y, j0 = blockIdx.y * per, j1 = min(n, j0 + per);
+  double acc[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) acc[k] = none;
+  for (int j = j0 + threadIdx.x; j < j1; j += U * NT) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const double x = j + k * NT < j1 ? part[(size_t)(j + k * NT) * width + i] : none;
+      acc[k] = ismax ? fmax(acc[k], x) : acc[k] + x;
+    }
   }
-  block_reduce<1>(a, ismax ? 1u : 0u, out + i);
+  double a[1] = {acc[0]};
+#pragma unroll
+  for (int k = 1; k < U; ++k) a[0] = ismax ? fmax(a[0], acc[k]) : a[0] + acc[k];
+  block_reduce<1>(a, ismax ? 1u : 0u, out + (size_t)blockIdx.y * width + i);
 }
+
+// Above REDUCE_ONE partials a component is reduced by several workgroups of half as many
+// partials each (more with REDUCE_CHUNKS of them), whose results a second launch reduces: one workgroup
+// took 150 us over the 131072 energy partials of 256^3 and 1.7 ms over the 1048576 of 512^3.
+// Below, the second launch costs more than the one workgroup's few rounds of loads.
+constexpr int REDUCE_ONE = 8192;
 
 int launch_reduce(Ctx& c, int n, int width, unsigned maxmask, double* out_dev, const double* part)
 {
-  hipLaunchKernelGGL(k_reduce, dim3(width), dim3(NT), 0, c.stream, part ? part : c.partials, n, width, maxmask,
-                     out_dev);
+  if (!part) part = c.partials;
+  if (n > REDUCE_ONE) {
+    const int chunks = std::min(REDUCE_CHUNKS, (n + REDUCE_ONE / 2 - 1) / (REDUCE_ONE / 2));
+    hipLaunchKernelGGL(k_reduce, dim3(width, chunks), dim3(NT), 0, c.stream, part, n, width, maxmask, c.red_part);
+    part = c.red_part;
+    n = chunks;
+  }
+  hipLaunchKernelGGL(k_reduce, dim3(width), dim3(NT), 0, c.stream, part, n, width, maxmask, out_dev);
   return check_hip(c, hipGetLastError(), "k_reduce");
 }
 
