@@ -443,8 +443,7 @@ int cup_poisson_mixed(cup_ctx* ctx)
   CUP_GUARD(ctx);
   if (c.decomposition != CUP_PLAIN)
     return set_error(c, CUP_E_STATE, "poisson_mixed: takes the CUP_PLAIN decomposition's RHS buffer");
-  if (int rc = launch_poisson_mixed(c)) return rc;
-  return launch_copy(c, c.f[CUP_P], c.rbuf, c.ncell);  // PoissonSolver::_fftw2cub
+  return launch_poisson_mixed(c);
 }
 
 int cup_poisson_unbounded(cup_ctx* ctx)

@@ -1050,41 +1050,161 @@ int launch_fft_inverse_field(Ctx& c, void* spec, void* real_blocks)
 // ------------------------------------------------------- PoissonSolverMixed
 // PoissonSolverMixed::solve (PoissonSolverMixed.cpp:66-103, _solve PoissonSolverMixed.h:27-80):
 // FFTW r2r transforms per axis, R2HC / HC2R on periodic axes and REDFT10 / REDFT01 (DCT-II /
-// DCT-III) on the others (PoissonSolverMixed.cpp:37-42), here as dense N x N matrices applied
-// to each line in LDS (N^2 work per line: the path for non-periodic boxes, not a benchmark
-// path); the coefficient (i, j, k) times norm / (denX_i + denY_j + denZ_k) in FP64, the first
-// one zeroed. Works on the RHS buffer in block layout.
+// DCT-III) on the others (PoissonSolverMixed.cpp:37-42), here as dense N x N matrices, a
+// contraction over each line on the matrix cores; the coefficient (i, j, k) times
+// norm / (denX_i + denY_j + denZ_k) in FP64, the first one zeroed.
+//
+// One workgroup transforms LN lines of N cells: it stages them in LDS as X[j][line] and forms
+// Y = M X in 16 x 16 tiles of the 16x16x4 matrix instruction (M's fragments from the cache, 16
+// columns of j in flight; X's from LDS, two line groups per fragment of M), then stores each tile
+// back over its lines. What bounds it is the latency of M's fragments in the cache, not the
+// matrix units (2 us a pass at their rate) or the field's traffic: on 128 x 96 x 64 cells in FP64
+// a pass takes 9 to 14 us, against 50 us with one thread per output walking its line, where every
+// line read the whole matrix.
 template <typename T>
-__global__ __launch_bounds__(NT) void k_r2r_axis(T* __restrict__ a, const T* __restrict__ mt, GridArgs g, int axis)
-{
-  extern __shared__ __align__(16) unsigned char r2r_lds[];
-  T* line = reinterpret_cast<T*>(r2r_lds);
-  const int n = axis == 0 ? g.Nx : (axis == 1 ? g.Ny : g.Nz);
-  const int n1 = axis == 0 ? g.Ny : g.Nx;  // the first of the other two axes
-  const int p = blockIdx.x, o1 = p % n1, o2 = p / n1;
-  auto at = [&](int k) -> size_t {
-    return axis == 0 ? cell_index(g, k, o1, o2) : (axis == 1 ? cell_index(g, o1, k, o2) : cell_index(g, o1, o2, k));
-  };
-  for (int j = threadIdx.x; j < n; j += NT) line[j] = a[at(j)];
-  __syncthreads();
-  for (int k = threadIdx.x; k < n; k += NT) {
-    T acc = 0;
-    for (int j = 0; j < n; ++j) acc += mt[(size_t)j * n + k] * line[j];
-    a[at(k)] = acc;
+struct MatTile;
+template <>
+struct MatTile<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mma(double a, double b, acc c)
+  {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
+  // the tile row of a lane's v-th accumulator (its column is lane % 16)
+  static __device__ __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
+};
+template <>
+struct MatTile<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mma(float a, float b, acc c)
+  {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
+};
+
+constexpr int R2R_STAGE = 17;  // row pitch of a wave's 16 x 16 staging tile
+// Row pitch of X: the four rows a fragment reads fall on distinct banks.
+constexpr int r2r_pitch(int ln) { return ln == 16 ? 16 : ln + 16; }
+template <typename T, int LN, int AXIS>
+inline size_t r2r_lds(int n)
+{
+  return ((size_t)n * r2r_pitch(LN) + (AXIS == 0 ? NT / 64 * 16 * R2R_STAGE : 0)) * sizeof(T);
 }
 
-template <typename T>
-__global__ void k_mixed_divide(T* __restrict__ a, GridArgs g, double norm, const double* __restrict__ dx,
-                               const double* __restrict__ dy, const double* __restrict__ dz)
+// src and dst may be the same field: a workgroup reads its lines before it writes them. dx, dy,
+// dz: the symbol's terms when this pass (along z) also divides, else null.
+template <typename T, int LN, int AXIS>
+__global__ __launch_bounds__(NT) void k_r2r_axis(const T* src, T* dst, const T* __restrict__ mt, GridArgs g,
+                                                 double norm, const double* __restrict__ dx,
+                                                 const double* __restrict__ dy, const double* __restrict__ dz)
 {
-  const size_t n = (size_t)g.nb * BS3;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const int b = (int)(i / BS3), c = (int)(i % BS3);
-    const int x = (b % g.nbx) * BS + (c & 7), y = ((b / g.nbx) % g.nby) * BS + ((c >> 3) & 7),
-              z = (b / (g.nbx * g.nby)) * BS + (c >> 6);
-    if (x == 0 && y == 0 && z == 0) a[i] = 0;
-    else a[i] = (T)((double)a[i] * (norm / (dx[x] + dy[y] + dz[z])));
+  using MT = MatTile<T>;
+  using V2 = typename Vec2<T>::type;
+  using V4 = typename Vec4<T>::type;
+  constexpr int PX = r2r_pitch(LN), SUB = 64 / LN, NG = LN / 16, GI = NG > 1 ? 2 : 1;
+  extern __shared__ __align__(32) unsigned char r2r_lds_buf[];
+  T* X = reinterpret_cast<T*>(r2r_lds_buf);
+  const int n = AXIS == 0 ? g.Nx : (AXIS == 1 ? g.Ny : g.Nz);
+  const int sub = blockIdx.x % SUB, o = blockIdx.x / SUB;  // LN of the 64 lines through a row of blocks
+  const int n1 = AXIS == 0 ? g.nby : g.nbx, o1 = o % n1, o2 = o / n1;
+  auto block = [&](int q) -> size_t {  // the q-th block along the lines
+    return AXIS == 0 ? q + (size_t)g.nbx * (o1 + (size_t)g.nby * o2)
+                     : (AXIS == 1 ? o1 + (size_t)g.nbx * (q + (size_t)g.nby * o2)
+                                  : o1 + (size_t)g.nbx * (o2 + (size_t)g.nby * q));
+  };
+  // Pairs of x-adjacent cells; line = (iz, iy) for x, (iz, ix) for y, (iy, ix) for z, the first
+  // index from sub * LN/8 on. Each wave reads whole 64-byte sectors and writes runs of lines.
+  for (int r = threadIdx.x; r < n * LN / 2; r += NT) {
+    const int q = r / (LN * 4), p = r % (LN * 4);
+    int cell, j, line;
+    if (AXIS == 0) {
+      line = (p >> 6) * 16 + (p & 15);
+      const int xp = (p >> 4) & 3;
+      cell = (sub * LN + line) * BS + 2 * xp;
+      j = q * BS + 2 * xp;
+    } else if (AXIS == 1) {
+      const int xp = p & 3, iz = (p >> 6) * 2 + ((p >> 2) & 1), iy = (p >> 3) & 7;
+      line = iz * BS + 2 * xp;
+      cell = ((sub * (LN / BS) + iz) * BS + iy) * BS + 2 * xp;
+      j = q * BS + iy;
+    } else {
+      line = 2 * (p % (LN / 2));
+      const int iz = p / (LN / 2);
+      cell = iz * BS * BS + sub * LN + line;
+      j = q * BS + iz;
+    }
+    const V2 v = *reinterpret_cast<const V2*>(src + block(q) * BS3 + cell);
+    if (AXIS == 0) {
+      X[j * PX + line] = v.x;
+      X[(j + 1) * PX + line] = v.y;
+    } else {
+      *reinterpret_cast<V2*>(&X[j * PX + line]) = v;
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lc = lane & 15, lr = lane >> 4;
+  const int items = (n + 15) / 16 * (NG / GI);
+  for (int item = wv; item < items; item += NT / 64) {
+    const int i0 = item / (NG / GI) * 16, g0 = item % (NG / GI) * GI;
+    const int ai = min(i0 + lc, n - 1);  // the last tile's rows past n are not stored
+    typename MT::acc acc[GI];
+#pragma unroll
+    for (int q = 0; q < GI; ++q) acc[q] = typename MT::acc{0, 0, 0, 0};
+    T a[4], an[4];
+    auto fetch = [&](T (&f)[4], int j0) {  // n is a multiple of 8: the last 16 columns may be half empty
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = j0 + 4 * q + lr;
+        f[q] = j < n ? mt[(size_t)j * n + ai] : (T)0;
+      }
+    };
+    fetch(a, 0);
+    for (int j0 = 0; j0 < n; j0 += 16) {
+      if (j0 + 16 < n) fetch(an, j0 + 16);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = min(j0 + 4 * q + lr, n - 1);
+#pragma unroll
+        for (int k = 0; k < GI; ++k) acc[k] = MT::mma(a[q], X[j * PX + (g0 + k) * 16 + lc], acc[k]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[q] = an[q];
+    }
+#pragma unroll
+    for (int k = 0; k < GI; ++k) {
+      const int line = (g0 + k) * 16 + lc;
+      if (AXIS == 0) {
+        // through the wave's staging tile, so that a line's cells leave as whole vectors
+        T* st = X + (size_t)n * PX + wv * 16 * R2R_STAGE;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) st[MT::row(lane, v) * R2R_STAGE + lc] = acc[k][v];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int sl = lane >> 2, i = 4 * (lane & 3);
+        const V4 w = {st[i * R2R_STAGE + sl], st[(i + 1) * R2R_STAGE + sl], st[(i + 2) * R2R_STAGE + sl],
+                      st[(i + 3) * R2R_STAGE + sl]};
+        if (i0 + i < n)
+          *reinterpret_cast<V4*>(dst + block((i0 + i) >> 3) * BS3 + (sub * LN + (g0 + k) * 16 + sl) * BS +
+                                 ((i0 + i) & 7)) = w;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = i0 + MT::row(lane, v);
+          if (i >= n) continue;
+          const int cell = AXIS == 1 ? ((sub * (LN / BS) + (line >> 3)) * BS + (i & 7)) * BS + (line & 7)
+                                     : (i & 7) * BS * BS + sub * LN + line;
+          T out = acc[k][v];
+          if (AXIS == 2 && dx) {
+            const int x = o1 * BS + (line & 7), y = o2 * BS + sub * (LN / BS) + (line >> 3);
+            out = (x | y | i) ? (T)((double)out * (norm / (dx[x] + dy[y] + dz[i]))) : (T)0;
+          }
+          dst[block(i >> 3) * BS3 + cell] = out;
+        }
+      }
+    }
   }
 }
 
@@ -1131,25 +1251,37 @@ static int mixed_setup(Ctx& c)
   return CUP_OK;
 }
 
+// Lines per workgroup: more of them share each fragment of the matrix, as long as the tile keeps
+// two workgroups on a CU (64 KiB) and the launch has two for every CU; 16 at least.
+template <typename T, int AXIS>
+static void r2r_pass(Ctx& c, const T* src, T* dst, int q, double norm, bool divide)
+{
+  const int n = c.N[AXIS], rows = (int)(c.ncell / (size_t)n / 64);
+  auto go = [&](auto kern, int ln, size_t lds) {
+    hipLaunchKernelGGL(kern, dim3(rows * (64 / ln)), dim3(NT), lds, c.stream, src, dst, (const T*)c.r2r[AXIS][q],
+                       c.grid(), norm, (const double*)(divide ? c.mden[0] : nullptr), (const double*)c.mden[1],
+                       (const double*)c.mden[2]);
+  };
+  constexpr size_t cap = 64 * 1024;
+  if (rows >= 512 && r2r_lds<T, 64, AXIS>(n) <= cap) go(k_r2r_axis<T, 64, AXIS>, 64, r2r_lds<T, 64, AXIS>(n));
+  else if (rows >= 256 && r2r_lds<T, 32, AXIS>(n) <= cap) go(k_r2r_axis<T, 32, AXIS>, 32, r2r_lds<T, 32, AXIS>(n));
+  else go(k_r2r_axis<T, 16, AXIS>, 16, r2r_lds<T, 16, AXIS>(n));
+}
+
+// The RHS stays in rbuf; the transforms work in the spectrum's buffer and end in p.
 template <typename T>
 static int poisson_mixed_t(Ctx& c)
 {
   if (int rc = mixed_setup<T>(c)) return rc;
-  T* a = (T*)c.rbuf;
-  const GridArgs g = c.grid();
-  auto axis_pass = [&](int d, int q) {
-    const int n = c.N[d], lines = (int)(c.ncell / (size_t)n);
-    hipLaunchKernelGGL((k_r2r_axis<T>), dim3(lines), dim3(NT), (size_t)n * sizeof(T), c.stream, a,
-                       (const T*)c.r2r[d][q], g, d);
-  };
-  for (int d = 0; d < 3; ++d) axis_pass(d, 0);
+  T* a = (T*)c.spec;
   double norm = 1 / c.h;
   for (int d = 0; d < 3; ++d) norm *= (c.bc[d] == CUP_BC_PERIODIC ? 1.0 : 0.5) / c.N[d];
-  size_t gsz = (c.ncell + NT - 1) / NT;
-  if (gsz > 65536) gsz = 65536;
-  hipLaunchKernelGGL((k_mixed_divide<T>), dim3((unsigned)gsz), dim3(NT), 0, c.stream, a, g, norm,
-                     (const double*)c.mden[0], (const double*)c.mden[1], (const double*)c.mden[2]);
-  for (int d = 0; d < 3; ++d) axis_pass(d, 1);
+  r2r_pass<T, 0>(c, (const T*)c.rbuf, a, 0, norm, false);
+  r2r_pass<T, 1>(c, a, a, 0, norm, false);
+  r2r_pass<T, 2>(c, a, a, 0, norm, true);
+  r2r_pass<T, 2>(c, a, a, 1, norm, false);
+  r2r_pass<T, 1>(c, a, a, 1, norm, false);
+  r2r_pass<T, 0>(c, a, (T*)c.f[CUP_P], 1, norm, false);
   return check_hip(c, hipGetLastError(), "poisson_mixed");
 }
 

@@ -41,6 +41,18 @@ __device__ __forceinline__ void load2_nt(const T* p, T& a, T& b)
   b = v.y;
 }
 
+// Two-wide vector of the context precision.
+template <typename T>
+struct Vec2;
+template <>
+struct Vec2<float> {
+  using type = float2;
+};
+template <>
+struct Vec2<double> {
+  using type = double2;
+};
+
 // Four-wide vector of the context precision (16- or 32-byte loads of 4 consecutive cells).
 template <typename T>
 struct Vec4;
@@ -343,7 +355,7 @@ int launch_count_nan(Ctx& c, long long out[4]);  // NaN cells of u, v, w, p (syn
 int free_error(int code, const std::string& msg);
 int launch_reset_umax(Ctx& c);  // clears both banks
 int launch_inflow_correction(Ctx& c);  // UpdateAndCorrectInflow on the open faces of u
-int launch_poisson_mixed(Ctx& c);      // PoissonSolverMixed: rbuf (RHS) -> rbuf (solution)
+int launch_poisson_mixed(Ctx& c);      // PoissonSolverMixed: rbuf (RHS) -> p
 int launch_poisson_unbounded(Ctx& c);  // PoissonSolverUnbounded: rbuf (RHS) -> p
 void unbounded_free(Ctx& c);
 // Device address of bank k of the max |u| slots (host pointer arithmetic, no access).

@@ -17,17 +17,6 @@ namespace cup {
 constexpr int L1 = 10;
 constexpr int L1C = L1 * L1 * L1;
 
-template <typename T>
-struct Vec2;
-template <>
-struct Vec2<float> {
-  using type = float2;
-};
-template <>
-struct Vec2<double> {
-  using type = double2;
-};
-
 
 // kinds[f] (HaloKind) says how field f's halo forms at a wall face; periodic grids ignore it.
 template <typename T, int NF>
