@@ -196,8 +196,19 @@ __device__ __forceinline__ void lab_put(const LabRegs<T, NF>& r, T (*lab)[LabGeo
 // The pipelined kernels' walk: workgroup w takes nbw blocks stacked in z,
 // b_j = bxy + nxy*(zg*nbw + j) with bxy = w % nxy, zg = w / nxy (nxy = nbx*nby), so that each
 // block after the first finds its lower z-face in the block just loaded (still in L2).
-// nbw = 4 when the blocks along z allow it.
-inline int blocks_per_wg(int nbz) { return nbz % 4 == 0 ? 4 : (nbz % 2 == 0 ? 2 : 1); }
+// nbw = 4 where the blocks along z allow it and at least 1024 workgroups remain (walk_blocks).
+//
+// A walk's length trades the halo faces it saves against workgroups: with fewer than a few per CU
+// a launch lasts as long as its longest chain of blocks. Gradient, FP32, 1 / 2 / 4 blocks:
+// 8.3 / 8.8 / 10.8 us on 64^3, 10.6 / 10.9 / 11.5 on 96^3, 17.3 / 16.0 / 16.1 on 128^3,
+// 88.0 / 84.5 / 83.1 on 256^3.
+// The largest of most, most/2, .. 1 blocks that divides n and leaves at least wgs workgroups.
+inline int walk_blocks(int n, int nb, int most, int wgs)
+{
+  while (most > 1 && (n % most || nb / most < wgs)) most /= 2;
+  return most;
+}
+inline int blocks_per_wg(const Ctx& c) { return walk_blocks(c.bpd[2], c.nb, 4, 1024); }
 
 __device__ __forceinline__ int walk_first(const GridArgs& g, int w, int nbw)
 {
@@ -548,10 +559,14 @@ static int advdiff_t(Ctx& c, double nu, const double uinf[3], const StepFold* fo
       fd.f[2 * a + 1] = (T)(1 - fac * hi * hi);
     }
   }
-  const int nbx = c.bpd[0];
-  if (nbx % 8 == 0) launch_advdiff_xwalk<T, 8>(c, nu, uinf, fold, fd);
-  else if (nbx % 4 == 0) launch_advdiff_xwalk<T, 4>(c, nu, uinf, fold, fd);
-  else if (nbx % 2 == 0) launch_advdiff_xwalk<T, 2>(c, nu, uinf, fold, fd);
+  // Blocks per walk. FP32, 1 / 2 / 4 / 8: 9.4 / 9.2 / 11.2 / 13.8 us on 64^3, 17.1 / 16.2 / 18.9
+  // on 160 x 96 x 120, 18.5 / 15.8 / 15.6 / 16.5 on 128^3, 130 / 106 / 100 / 106 on 256^3. FP64,
+  // whose x faces cost more sectors: 12.1 / 12.4 / 13.1 / 16.6 on 64^3, 19.1 / 17.7 / 14.8 on
+  // 96^3, 33.8 / 26.4 / 24.9 / 23.4 on 128^3.
+  const int nbw = sizeof(T) == 4 ? walk_blocks(c.bpd[0], c.nb, 4, 1024) : walk_blocks(c.bpd[0], c.nb, 8, 256);
+  if (nbw == 8) launch_advdiff_xwalk<T, 8>(c, nu, uinf, fold, fd);
+  else if (nbw == 4) launch_advdiff_xwalk<T, 4>(c, nu, uinf, fold, fd);
+  else if (nbw == 2) launch_advdiff_xwalk<T, 2>(c, nu, uinf, fold, fd);
   else launch_advdiff_xwalk<T, 1>(c, nu, uinf, fold, fd);
   return check_hip(c, hipGetLastError(), "k_advdiff_xwalk");
 }
@@ -827,10 +842,13 @@ static void up3_walk_launch(Ctx& c, int src0, int base0, int out0, double nu, co
 template <typename T>
 static int up3_stage(Ctx& c, int src0, int base0, int out0, double nu, const double uinf[3], double mult)
 {
+  // Blocks per walk, both stages of the midpoint form. FP32, 1 / 2 / 4 / 8: 14.9 / 15.7 / 22.8 /
+  // 31.8 us on 64^3, 42 / 41 / 45 / 43 on 128^3, 119 / 108 / 123 / 114 on 192^3, 291 / 254 / 276 /
+  // 255 on 256^3; FP64: 17 / 18 / 23 / 35 on 64^3, 77 / 64 / 71 / 62 on 128^3, 246 / 200 / 193 /
+  // 187 on 192^3.
   const int nbx = c.bpd[0];
-  if (nbx % 8 == 0) up3_walk_launch<T, 8>(c, src0, base0, out0, nu, uinf, mult);
-  else if (nbx % 4 == 0) up3_walk_launch<T, 4>(c, src0, base0, out0, nu, uinf, mult);
-  else if (nbx % 2 == 0) up3_walk_launch<T, 2>(c, src0, base0, out0, nu, uinf, mult);
+  if (nbx % 8 == 0 && c.nb / 8 >= (sizeof(T) == 4 ? 2048 : 512)) up3_walk_launch<T, 8>(c, src0, base0, out0, nu, uinf, mult);
+  else if (nbx % 2 == 0 && c.nb / 2 >= 512) up3_walk_launch<T, 2>(c, src0, base0, out0, nu, uinf, mult);
   else up3_walk_launch<T, 1>(c, src0, base0, out0, nu, uinf, mult);
   return check_hip(c, hipGetLastError(), "k_advdiff_up3_xwalk");
 }
@@ -1254,7 +1272,7 @@ static int gradp_t(Ctx& c, bool fused, const double uinf[3], const int* skip, bo
   const T* p = (const T*)c.f[CUP_P];
   const int s = fused ? c.ustar : CUP_U;
   const C2<T>* tx = (const C2<T>*)c.tw[0];
-  const int nbw = blocks_per_wg(c.bpd[2]);
+  const int nbw = blocks_per_wg(c);
   const dim3 grid(c.nb / nbw);
   const T* xf = (const T*)c.xface;
   if (fused && force && xface)
@@ -1294,7 +1312,7 @@ static int gradp_t(Ctx& c, bool fused, const double uinf[3], const int* skip, bo
 // projection's last pass.
 int launch_gradp_inplace(Ctx& c, int field0)
 {
-  const int nbw = blocks_per_wg(c.bpd[2]);
+  const int nbw = blocks_per_wg(c);
   const dim3 grid(c.nb / nbw);
   if (c.precision == 4) {
     float* f[3] = {(float*)c.f[field0], (float*)c.f[field0 + 1], (float*)c.f[field0 + 2]};
