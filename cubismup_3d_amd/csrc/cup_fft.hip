@@ -157,7 +157,8 @@ __device__ __forceinline__ void dft5(C2<T>* v)
 template <int R, int DIR, typename T>
 __device__ __forceinline__ void dftR(C2<T>* v)
 {
-  if constexpr (R == 8) dft8<DIR>(v);
+  if constexpr (R == 16) dft16<DIR>(v);
+  else if constexpr (R == 8) dft8<DIR>(v);
   else if constexpr (R == 4) dft4<DIR>(v[0], v[1], v[2], v[3]);
   else if constexpr (R == 5) dft5<DIR>(v);
   else if constexpr (R == 3) dft3<DIR>(v);
@@ -486,96 +487,224 @@ __global__ __launch_bounds__(NT) void k_fft_x_inv(const C2<T>* __restrict__ S, T
 
 // ------------------------------------------------------------------ y / z passes
 
-template <typename T, int N>
-struct ColTile {
-  // columns per workgroup: LDS tile at most 64 KiB, at most 16 columns; a length known at run
-  // time (N = 0, at most FFT_MAX_N) takes 4 (FP32) or 2 (FP64) columns, 32 KiB at most
-  static constexpr int raw = N > 0 ? 65536 / (N * (int)sizeof(C2<T>)) : (sizeof(T) == 4 ? 4 : 2);
-  static constexpr int TK = raw >= 16 ? 16 : (raw < 1 ? 1 : raw);
-};
-
 enum ZMode { ZM_FWD = 0, ZM_INV = 1, ZM_POISSON = 2 };
 
-// Column FFT along y (AXIS=1) or z (AXIS=2). grid = (ceil(ncols/TK), other axis).
-// MODE: forward, inverse, or (z only) forward + grid-consistent division + inverse.
-template <typename T, int N, int AXIS, int MODE, bool FORCE = false>
-__global__ __launch_bounds__(NT) void k_fft_col(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw, int ncols,
-                                                int Ny, int Nz, double norm, const double* __restrict__ cx,
-                                                const double* __restrict__ cy, const double* __restrict__ cz,
-                                                const LowModes* __restrict__ lmp, const double* __restrict__ coef,
-                                                FftPlan pl)
-{
-  constexpr int TK = ColTile<T, N>::TK;
-  static_assert(TK % 2 == 0, "columns move in pairs");
-  const int n = N > 0 ? N : pl.n;
-  C2<T>* buf = lds_tile<T, N * TK>();
-  const int kx0 = blockIdx.x * TK, other = blockIdx.y;
-  const int nc = min(TK, ncols - kx0);
-  // element (f, n): AXIS=1: S[(other*Ny + n)*ncols + kx0 + f]; AXIS=2: S[(n*Ny + other)*ncols + kx0 + f].
-  // Columns move in pairs (ncols, TK and so nc are even): one 2-element vector access each.
-  using V4 = typename Vec4<T>::type;
-  for (int t = threadIdx.x; t < n * TK / 2; t += NT) {
-    const int f = 2 * (t % (TK / 2)), e = t / (TK / 2);
-    V4 a = {0, 0, 0, 0};
-    if (f < nc) {
-      const size_t gi = AXIS == 1 ? ((size_t)other * Ny + e) * ncols + kx0 + f : ((size_t)e * Ny + other) * ncols + kx0 + f;
-      a = *reinterpret_cast<const V4*>(S + gi);
-    }
-    *reinterpret_cast<V4*>(buf + f + e * TK) = a;
+// Column passes of the lengths without a register four-step form below: 512 and 1024 (N > 0, radices
+// known at compile time) and every length that is not a power of two, or below 64 (N = 0, the plan's
+// radices). M bounds the length. A workgroup of BT threads takes TK columns, at most 16 elements per
+// thread, in Stockham stages whose butterflies a thread holds in registers: the first stage reads its
+// inputs j + r n/R from global memory, the last writes its outputs (the same indices) there, and
+// only the stages between exchange through LDS. The z pass's division happens on the last forward
+// stage's registers, which are also the inputs of the first inverse stage when the inverse takes the
+// radices in reverse order. Against a tile staged in LDS at both ends this halves the LDS traffic:
+// on 512^3 FP32 (1 GiB of traffic) a y pass went from 325 to 215 us, the rate of a large copy, and the
+// z pass from 614 to 370; on 160 x 96 x 120 from 20 to 8 and from 28 to 15 us.
+template <typename T, int M>
+struct ColTile {
+  // 16 columns (8 for 1024) in FP32, 64 KiB of LDS at most: 128-byte segments, or 64 at 1024
+  static constexpr int TK = sizeof(T) == 4 ? (M <= 512 ? 16 : 8) : (M <= 256 ? 16 : (M <= 512 ? 8 : 4));
+  static constexpr int BT = TK * M / 16;
+  static constexpr int E = 16;  // elements per thread
+};
+
+// k = j % Ns for j < 2^20 and Ns <= 1024 (rNs = 1/Ns rounded): the quotient's estimate is below the
+// next integer by at least 1/(2 Ns), more than the product's rounding.
+__device__ __forceinline__ int mod_ns(int j, int Ns, float rNs) { return j - Ns * (int)(((float)j + 0.5f) * rNs); }
+
+template <typename T, int N, int M>
+struct ColStages {
+  using CT = ColTile<T, M>;
+  static constexpr int TK = CT::TK, BT = CT::BT;
+  C2<T>* S;
+  C2<T>* buf;
+  const C2<T>* tw;
+  size_t base, stride;  // element e of column f is S[base + f + e stride]
+  bool inv;             // an inverse transform: the forward one with the real and imaginary parts swapped
+  int n, nc;            // length, live columns
+  int kx0, ky, Ny;      // the z pass's symbol and forcing modes
+  double norm;
+  const double *cx, *cy, *cz;
+  const LowModes* lmp;  // null: no forcing
+  const double* coef;
+
+  __device__ __forceinline__ C2<T> load(int f, int e) const
+  {
+    const C2<T> a = f < nc ? S[base + f + e * stride] : C2<T>{0, 0};
+    return inv ? C2<T>{a.y, a.x} : a;
   }
-  __syncthreads();
-  if (MODE == ZM_INV) {
-    if constexpr (N > 0) lds_fft<N, TK, +1>(buf, tw);
-    else lds_fft_rt<TK, +1>(buf, tw, pl);
-  } else {
-    if constexpr (N > 0) lds_fft<N, TK, -1>(buf, tw);
-    else lds_fft_rt<TK, -1>(buf, tw, pl);
-  }
-  if (FORCE) {
-    // fused forcing: add the forcing's RHS modes (coefficients from k_forcing_reduce)
-    const LowModes& lm = *lmp;
-    for (int e = threadIdx.x; e < lm.npos; e += NT) {
-      const int slot = lm.pos[e][0], ky = lm.pos[e][1], kz = lm.pos[e][2], mc = lm.pos[e][3];
-      if (ky != other || slot < kx0 || slot >= kx0 + nc) continue;
-      const double* cm = coef + 8 * (mc >> 1);
-      const double ci = (mc & 1) ? -cm[1] : cm[1];
-      C2<T>& v = buf[(slot - kx0) + kz * TK];
-      v.x = (T)((double)v.x + cm[0]);
-      v.y = (T)((double)v.y + ci);
-    }
-    __syncthreads();
-  }
-  if (MODE == ZM_POISSON) {
-    // PoissonSolverPeriodic::_solve grid-consistent branch (PoissonSolverPeriodic.cpp:23-61):
-    // multiply by norm/(2D-6), D = cos(4 pi kx/Nx) + cos(4 pi ky/Ny) + cos(4 pi kz/Nz),
-    // in FP64; zero the modes with every index in {0, N/2} (kx slot 0 carries kx=0 and Nx/2).
-    const int ky = other;
-    for (int t = threadIdx.x; t < n * TK; t += NT) {
-      const int f = t % TK, kz = t / TK;
-      const int kx = kx0 + f;
-      if (f < nc) {
-        const double D = cx[kx] + cy[ky] + cz[kz];
-        double fac = norm / (2 * D - 6);
-        const bool zero = kx == 0 && (ky == 0 || 2 * ky == Ny) && (kz == 0 || 2 * kz == n);
-        if (zero) fac = 0;
-        C2<T> v = buf[f + kz * TK];
-        v.x = (T)((double)v.x * fac);
-        v.y = (T)((double)v.y * fac);
-        if (zero) v = C2<T>{0, 0};
-        buf[f + kz * TK] = v;
+
+  // the spectral division of the outputs kz = j + r n/R of column kx0 + f, after the forcing's modes
+  template <int R>
+  __device__ __forceinline__ void divide(C2<T> (&v)[R], int f, int j) const
+  {
+    const int m = n / R;
+    if (lmp && kx0 == 0) {
+      const LowModes& lm = *lmp;
+      for (int e = 0; e < lm.npos; ++e) {
+        const int slot = lm.pos[e][0], kye = lm.pos[e][1], kz = lm.pos[e][2], mc = lm.pos[e][3];
+        if (kye != ky || slot != f) continue;
+        const double* cm = coef + 8 * (mc >> 1);
+        const double ci = (mc & 1) ? -cm[1] : cm[1];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (kz == j + r * m) {
+            v[r].x = (T)((double)v[r].x + cm[0]);
+            v[r].y = (T)((double)v[r].y + ci);
+          }
       }
     }
-    __syncthreads();
-    if constexpr (N > 0) lds_fft<N, TK, +1>(buf, tw);
-    else lds_fft_rt<TK, +1>(buf, tw, pl);
-  }
-  for (int t = threadIdx.x; t < n * TK / 2; t += NT) {
-    const int f = 2 * (t % (TK / 2)), n = t / (TK / 2);
-    if (f < nc) {
-      const size_t gi = AXIS == 1 ? ((size_t)other * Ny + n) * ncols + kx0 + f : ((size_t)n * Ny + other) * ncols + kx0 + f;
-      *reinterpret_cast<V4*>(S + gi) = *reinterpret_cast<const V4*>(buf + f + n * TK);
+    // PoissonSolverPeriodic::_solve's grid-consistent branch (PoissonSolverPeriodic.cpp:23-61):
+    // norm/(2D-6), D = cos(4 pi kx/Nx) + cos(4 pi ky/Ny) + cos(4 pi kz/Nz), in FP64; the modes with
+    // every index in {0, N/2} are zeroed (kx slot 0 carries kx = 0 and Nx/2)
+    const int kx = kx0 + f;
+    const double dxy = f < nc ? cx[kx] + cy[ky] : 0.0;
+    const bool zxy = kx == 0 && (ky == 0 || 2 * ky == Ny);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int kz = j + r * m;
+      const double D = dxy + cz[kz];
+      double fac = norm / (2 * D - 6);
+      const bool zero = zxy && (kz == 0 || 2 * kz == n);
+      if (zero) fac = 0;
+      v[r].x = (T)((double)v[r].x * fac);
+      v[r].y = (T)((double)v[r].y * fac);
+      if (zero) v[r] = C2<T>{0, 0};
     }
   }
+
+  // One stage of radix R after Ns = the product of the earlier radices. FIRST and LAST: it reads
+  // from and writes to global memory. MID: the forward transform's last stage, the division and the
+  // inverse transform's first stage, after which the parts are swapped.
+  template <int R, bool FIRST, bool LAST, bool MID>
+  __device__ __forceinline__ void stage(int Ns)
+  {
+    constexpr int IT = (CT::E + R - 1) / R;
+    const int m = n / R, NB = TK * m, st = n / (Ns * R);
+    const float rNs = 1.0f / (float)Ns;
+    C2<T> v[IT][R];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int t = threadIdx.x + it * BT;
+      if (t >= NB) continue;
+      const int f = t % TK, j = t / TK;
+      if (FIRST) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[it][r] = load(f, j + r * m);
+      } else {
+        const int k = N > 0 ? j % Ns : mod_ns(j, Ns, rNs);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          v[it][r] = buf[f + (j + r * m) * TK];
+          if (r) v[it][r] = cmul(v[it][r], tw[r * k * st]);
+        }
+      }
+      dftR<R, -1>(v[it]);
+      if (MID) {
+        divide<R>(v[it], f, j);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[it][r] = C2<T>{v[it][r].y, v[it][r].x};
+        dftR<R, -1>(v[it]);
+      }
+    }
+    if (!FIRST && !LAST) __syncthreads();  // the stage's reads are done
+    const bool swap = LAST && (MID || inv);
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int t = threadIdx.x + it * BT;
+      if (t >= NB) continue;
+      const int f = t % TK, j = t / TK;
+      if (LAST) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (f < nc) S[base + f + (j + r * m) * stride] = swap ? C2<T>{v[it][r].y, v[it][r].x} : v[it][r];
+      } else {
+        // MID's outputs are those of the inverse's first stage: k = 0, from j R on
+        const int k = MID || FIRST ? 0 : (N > 0 ? j % Ns : mod_ns(j, Ns, rNs));
+        const int o = MID || FIRST ? j * R : (j - k) * R + k, step = MID ? 1 : Ns;
+#pragma unroll
+        for (int r = 0; r < R; ++r) buf[f + (o + r * step) * TK] = v[it][r];
+      }
+    }
+    if (!LAST) __syncthreads();
+  }
+
+  template <bool LAST, bool MID>
+  __device__ __forceinline__ void stage_rt(int R, int Ns)
+  {
+    if (R == 8) stage<8, false, LAST, MID>(Ns);
+    else if (R == 4) stage<4, false, LAST, MID>(Ns);
+    else if (R == 5) stage<5, false, LAST, MID>(Ns);
+    else if (R == 3) stage<3, false, LAST, MID>(Ns);
+    else stage<2, false, LAST, MID>(Ns);
+  }
+
+  // The plan's radices; the first is 8 (a length is 8 x blocks), and the only one at length 8.
+  template <bool POISSON>
+  __device__ __forceinline__ void run_rt(const FftPlan& pl)
+  {
+    const int last = pl.ns - 1;
+    if (last == 0) {
+      stage<8, true, true, POISSON>(1);
+      return;
+    }
+    stage<8, true, false, false>(1);
+    int Ns = 8;
+    for (int s = 1; s < last; ++s) {
+      stage_rt<false, false>(pl.r[s], Ns);
+      Ns *= pl.r[s];
+    }
+    if constexpr (!POISSON) {
+      stage_rt<true, false>(pl.r[last], Ns);
+      return;
+    }
+    stage_rt<false, true>(pl.r[last], Ns);
+    inv = true;
+    Ns = pl.r[last];
+    for (int s = last - 1; s > 0; --s) {
+      stage_rt<false, false>(pl.r[s], Ns);
+      Ns *= pl.r[s];
+    }
+    stage<8, false, true, false>(Ns);
+  }
+
+  // 512 = 8 8 8 and 1024 = 16 8 8: three stages each
+  template <bool POISSON>
+  __device__ __forceinline__ void run_ct()
+  {
+    constexpr int R0 = N / 64;
+    stage<R0, true, false, false>(1);
+    stage<8, false, false, false>(R0);
+    if constexpr (!POISSON) {
+      stage<8, false, true, false>(8 * R0);
+    } else {
+      stage<8, false, false, true>(8 * R0);
+      inv = true;
+      stage<8, false, false, false>(8);
+      stage<R0, false, true, false>(64);
+    }
+  }
+};
+
+// Column FFT along y (axis 1) or z (axis 2). grid = (ceil(ncols/TK), other axis). POISSON (z only):
+// forward transform, grid-consistent division and inverse transform.
+template <typename T, int N, int M, bool POISSON>
+__global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw,
+                                                               int ncols, int axis, int inv, int Ny, double norm,
+                                                               const double* __restrict__ cx,
+                                                               const double* __restrict__ cy,
+                                                               const double* __restrict__ cz,
+                                                               const LowModes* __restrict__ lmp,
+                                                               const double* __restrict__ coef, FftPlan pl)
+{
+  using CS = ColStages<T, N, M>;
+  C2<T>* buf = lds_tile<T, N * CS::TK>();
+  const int kx0 = blockIdx.x * CS::TK, o = blockIdx.y;
+  const size_t base = (axis == 1 ? (size_t)o * Ny : (size_t)o) * ncols + kx0;
+  const size_t stride = axis == 1 ? (size_t)ncols : (size_t)Ny * ncols;
+  CS cs{S,   buf, tw, base, stride, inv != 0, N > 0 ? N : pl.n, min(CS::TK, ncols - kx0), kx0, o, Ny, norm,
+        cx,  cy,  cz, lmp,  coef};
+  if constexpr (N > 0) cs.template run_ct<POISSON>();
+  else cs.template run_rt<POISSON>(pl);
 }
 
 // ------------------------------------------- y / z passes, register four-step form
@@ -856,26 +985,30 @@ struct ColPass {
         hipLaunchKernelGGL((k_fft_colr<T, N, 2, ZM_POISSON, false>), grid, dim3(NT), 0, c.stream, spec, tw, ncols,
                            c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr,
                            ex);
-      return;
+    } else if constexpr (N >= 512) {
+      launch<N, N>(c, spec, mode, norm, force);
+    } else {
+      const int n = c.N[AXIS];
+      if (n <= 256) launch<0, 256>(c, spec, mode, norm, force);
+      else if (n <= 512) launch<0, 512>(c, spec, mode, norm, force);
+      else launch<0, FFT_MAX_N>(c, spec, mode, norm, force);
     }
-    constexpr int TK = ColTile<T, N>::TK;
+  }
+  template <int NN, int M>
+  static void launch(Ctx& c, C2<T>* spec, int mode, double norm, bool force)
+  {
+    using CT = ColTile<T, M>;
     const int ncols = c.N[0] / 2;
-    const int other = AXIS == 1 ? c.N[2] : c.N[1];
-    dim3 grid((ncols + TK - 1) / TK, other);
-    const C2<T>* tw = (const C2<T>*)c.tw[AXIS];
-    const size_t lds = N > 0 ? 0 : (size_t)c.N[AXIS] * TK * sizeof(C2<T>);
-    if (mode == ZM_FWD)
-      hipLaunchKernelGGL((k_fft_col<T, N, AXIS, ZM_FWD>), grid, dim3(NT), lds, c.stream, spec, tw, ncols, c.N[1], c.N[2],
-                         norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr, c.plan[AXIS]);
-    else if (mode == ZM_INV)
-      hipLaunchKernelGGL((k_fft_col<T, N, AXIS, ZM_INV>), grid, dim3(NT), lds, c.stream, spec, tw, ncols, c.N[1], c.N[2],
-                         norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr, c.plan[AXIS]);
-    else if (AXIS == 2 && force)
-      hipLaunchKernelGGL((k_fft_col<T, N, 2, ZM_POISSON, true>), grid, dim3(NT), lds, c.stream, spec, tw, ncols, c.N[1],
-                         c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)c.low_coef, c.plan[AXIS]);
-    else if (AXIS == 2)
-      hipLaunchKernelGGL((k_fft_col<T, N, 2, ZM_POISSON, false>), grid, dim3(NT), lds, c.stream, spec, tw, ncols, c.N[1],
-                         c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr, c.plan[AXIS]);
+    const dim3 grid((ncols + CT::TK - 1) / CT::TK, AXIS == 1 ? c.N[2] : c.N[1]), bt(CT::BT);
+    const size_t lds = NN > 0 ? 0 : (size_t)c.N[AXIS] * CT::TK * sizeof(C2<T>);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, bt, lds, c.stream, spec, (const C2<T>*)c.tw[AXIS], ncols, AXIS,
+                         mode == ZM_INV ? 1 : 0, c.N[1], norm, (const double*)c.cos4[0], (const double*)c.cos4[1],
+                         (const double*)c.cos4[2], (const LowModes*)(force ? c.low_dev : nullptr),
+                         (const double*)c.low_coef, c.plan[AXIS]);
+    };
+    if (mode == ZM_POISSON) go(k_fft_col<T, NN, M, true>);
+    else go(k_fft_col<T, NN, M, false>);
   }
 };
 
