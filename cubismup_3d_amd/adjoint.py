@@ -14,9 +14,49 @@ velocity is not differentiated). No counterpart in the reference.
 """
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from .grid import Grid
+
+
+def _checkpoints(grid: Grid, nsteps: int, every: int):
+    """{step: buffer} of the steps whose velocity the forward keeps, 0, every, 2 every, ..., with the
+    present velocity in the first."""
+    steps = range(0, max(nsteps, 1), every)
+    ckpts = dict(zip(steps, grid.velocity_buffers(len(steps))))
+    grid.keep_velocity(ckpts[0])
+    return ckpts
+
+
+@contextlib.contextmanager
+def _settled(grid: Grid):
+    """Waits for the grid's stream on the way out, also after an error: the copies into and out of
+    torch's buffers are done before torch may hand their memory on."""
+    try:
+        yield
+    finally:
+        grid.synchronize()
+
+
+def _backward_steps(grid: Grid, ckpts, nsteps: int, every: int, step, adjoint):
+    """The backward's walk over the segments, last first: each one's states recomputed from its
+    checkpoint by step(n), then adjoint(n) with the velocity of step n in place. The adjoint fields
+    stay on the grid throughout (the forward steps do not touch them), and the states in the grid's
+    own block order on its own stream."""
+    spare = grid.velocity_buffers(max(0, min(every, nsteps) - 1))
+    with _settled(grid):
+        for s0 in sorted(ckpts, reverse=True):
+            s1 = min(s0 + every, nsteps)
+            states = [ckpts[s0]] + spare[:max(0, s1 - 1 - s0)]
+            grid.restore_velocity(ckpts[s0])
+            for n in range(s0, s1 - 1):
+                step(n)
+                grid.keep_velocity(states[n + 1 - s0])
+            for n in reversed(range(s0, s1)):
+                grid.restore_velocity(states[n - s0])
+                adjoint(n)
 
 
 class Rollout(torch.autograd.Function):
@@ -26,18 +66,24 @@ class Rollout(torch.autograd.Function):
         """dts: fixed timesteps, or None for CFL timesteps (appended to dts_out); forcing:
         (tke_target, injection_rate), both 0 for none."""
         grid.set_torch_velocity(u0.detach())
-        ckpts = {0: u0.detach().clone()}
+        ckpts = _checkpoints(grid, nsteps, every)
         used = []
         fkw = dict(spectral_forcing=any(f > 0 for f in forcing), tke_target=forcing[0], injection_rate=forcing[1])
-        for n in range(nsteps):
-            if dts is None:
-                grid.run_steps(1, CFL=CFL, nu=nu, uinf=uinf, scheme=scheme, **fkw)
-                used.append(grid.step_state()["last_dt"])
-            else:
-                grid.run_steps(1, nu=nu, uinf=uinf, fixed_dt=dts[n], scheme=scheme, **fkw)
-                used.append(float(dts[n]))
-            if (n + 1) % every == 0 and n + 1 < nsteps:
-                ckpts[n + 1] = grid.get_torch_velocity()
+        n = 0
+        with _settled(grid):
+            while n < nsteps:
+                if n and n in ckpts:
+                    grid.keep_velocity(ckpts[n])
+                m = 1
+                if dts is None:
+                    grid.run_steps(1, CFL=CFL, nu=nu, uinf=uinf, scheme=scheme, **fkw)
+                    used.append(grid.step_state()["last_dt"])
+                else:  # equal timesteps up to the next checkpoint in one call
+                    while n + m < nsteps and n + m not in ckpts and dts[n + m] == dts[n]:
+                        m += 1
+                    grid.run_steps(m, nu=nu, uinf=uinf, fixed_dt=dts[n], scheme=scheme, **fkw)
+                    used.extend([float(dts[n])] * m)
+                n += m
         dts_out.extend(used)
         ctx.grid, ctx.nsteps, ctx.nu, ctx.uinf, ctx.dts, ctx.every = grid, nsteps, nu, uinf, used, every
         ctx.scheme = scheme
@@ -48,21 +94,18 @@ class Rollout(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        grid, every = ctx.grid, ctx.every
-        lam = g.detach().contiguous().to(grid._torch_dtype())
-        for s0 in sorted(ctx.ckpts, reverse=True):
-            s1 = min(s0 + every, ctx.nsteps)
-            states = [ctx.ckpts[s0]]
-            grid.set_torch_velocity(ctx.ckpts[s0])
-            for n in range(s0, s1 - 1):
-                grid.run_steps(1, nu=ctx.nu, uinf=ctx.uinf, fixed_dt=ctx.dts[n], scheme=ctx.scheme, **ctx.fkw)
-                states.append(grid.get_torch_velocity())
-            for n in reversed(range(s0, s1)):
-                grid.set_torch_velocity(states[n - s0])
-                grid.set_torch_adjoint(lam)
-                grid.adjoint_step(ctx.dts[n], ctx.nu, ctx.uinf, scheme=ctx.scheme, tke_target=ctx.forcing[0],
-                                  injection_rate=ctx.forcing[1])
-                lam = grid.get_torch_adjoint()
+        grid = ctx.grid
+        grid.set_torch_adjoint(g.detach().contiguous().to(grid._torch_dtype()))
+
+        def step(n):
+            grid.run_steps(1, nu=ctx.nu, uinf=ctx.uinf, fixed_dt=ctx.dts[n], scheme=ctx.scheme, **ctx.fkw)
+
+        def adjoint(n):
+            grid.adjoint_step(ctx.dts[n], ctx.nu, ctx.uinf, scheme=ctx.scheme, tke_target=ctx.forcing[0],
+                              injection_rate=ctx.forcing[1])
+
+        _backward_steps(grid, ctx.ckpts, ctx.nsteps, ctx.every, step, adjoint)
+        lam = grid.get_torch_adjoint()
         ctx.ckpts = None
         return lam.to(ctx.u0_dtype), None, None, None, None, None, None, None, None, None, None
 
@@ -106,13 +149,14 @@ class PenalizedRollout(torch.autograd.Function):
             grid.chi_from_sphere(body[0], body[1], mollify=body[2])
         grid.set_torch_velocity(u0.detach())
         T = float(sum(dts))
-        ckpts = {0: u0.detach().clone()}
+        ckpts = _checkpoints(grid, nsteps, every)
         J = 0.0
-        for n in range(nsteps):
-            grid.run_steps(1, nu=nu, uinf=uinf, fixed_dt=dts[n], sphere=sphere, **fkw)
-            J += dts[n] / T * grid.last_body_force()[0]
-            if (n + 1) % every == 0 and n + 1 < nsteps:
-                ckpts[n + 1] = grid.get_torch_velocity()
+        with _settled(grid):
+            for n in range(nsteps):
+                if n and n in ckpts:
+                    grid.keep_velocity(ckpts[n])
+                grid.run_steps(1, nu=nu, uinf=uinf, fixed_dt=dts[n], sphere=sphere, **fkw)
+                J += dts[n] / T * grid.last_body_force()[0]
         ctx.grid, ctx.nsteps, ctx.nu, ctx.uinf, ctx.dts, ctx.every = grid, nsteps, nu, uinf, list(dts), every
         ctx.sphere, ctx.T, ctx.ckpts, ctx.u0_dtype, ctx.vdev, ctx.body = sphere, T, ckpts, u0.dtype, vel.device, body
         ctx.cdev = centre.device if centre is not None else None
@@ -122,34 +166,31 @@ class PenalizedRollout(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gJ):
-        grid, every, sphere = ctx.grid, ctx.every, ctx.sphere
+        grid, sphere = ctx.grid, ctx.sphere
         want_c = ctx.body is not None and ctx.needs_input_grad[2]
         want_w = ctx.wdev is not None and ctx.needs_input_grad[3]
         if ctx.body is not None:
             grid.chi_from_sphere(ctx.body[0], ctx.body[1], mollify=ctx.body[2])
         g = float(gJ)
-        lam = torch.zeros((3,) + grid.shape, dtype=grid._torch_dtype(), device="cuda")
+        grid.set_torch_adjoint(torch.zeros((3,) + grid.shape, dtype=grid._torch_dtype(), device="cuda"))
         dV = torch.zeros(3, dtype=torch.float64)
         dc = torch.zeros(3, dtype=torch.float64)
         dW = torch.zeros(3, dtype=torch.float64)
-        for s0 in sorted(ctx.ckpts, reverse=True):
-            s1 = min(s0 + every, ctx.nsteps)
-            states = [ctx.ckpts[s0]]
-            grid.set_torch_velocity(ctx.ckpts[s0])
-            for n in range(s0, s1 - 1):
-                grid.run_steps(1, nu=ctx.nu, uinf=ctx.uinf, fixed_dt=ctx.dts[n], sphere=sphere, **ctx.fkw)
-                states.append(grid.get_torch_velocity())
-            for n in reversed(range(s0, s1)):
-                grid.set_torch_velocity(states[n - s0])
-                grid.set_torch_adjoint(lam)
-                out = grid.adjoint_step_body(ctx.dts[n], ctx.nu, ctx.uinf, sphere, g * ctx.dts[n] / ctx.T,
-                                             centre=want_c, rotation=True, scheme=ctx.scheme,
-                                             tke_target=ctx.forcing[0], injection_rate=ctx.forcing[1])
-                dV += torch.from_numpy(out[0])
-                dW += torch.from_numpy(out[1])
-                if want_c:
-                    dc += torch.from_numpy(out[2])
-                lam = grid.get_torch_adjoint()
+
+        def step(n):
+            grid.run_steps(1, nu=ctx.nu, uinf=ctx.uinf, fixed_dt=ctx.dts[n], sphere=sphere, **ctx.fkw)
+
+        def adjoint(n):
+            out = grid.adjoint_step_body(ctx.dts[n], ctx.nu, ctx.uinf, sphere, g * ctx.dts[n] / ctx.T, centre=want_c,
+                                         rotation=True, scheme=ctx.scheme, tke_target=ctx.forcing[0],
+                                         injection_rate=ctx.forcing[1])
+            dV.add_(torch.from_numpy(out[0]))
+            dW.add_(torch.from_numpy(out[1]))
+            if want_c:
+                dc.add_(torch.from_numpy(out[2]))
+
+        _backward_steps(grid, ctx.ckpts, ctx.nsteps, ctx.every, step, adjoint)
+        lam = grid.get_torch_adjoint()
         ctx.ckpts = None
         return (lam.to(ctx.u0_dtype), dV.to(ctx.vdev), dc.to(ctx.cdev) if want_c else None,
                 dW.to(ctx.wdev) if want_w else None, None, None, None, None, None, None, None, None, None, None,
@@ -197,13 +238,14 @@ class BodiesRollout(torch.autograd.Function):
             grid.body_velocity(k, bodies[k]["trans_vel"], bodies[k]["ang_vel"])
         grid.set_torch_velocity(u0.detach())
         T = float(sum(dts))
-        ckpts = {0: u0.detach().clone()}
+        ckpts = _checkpoints(grid, nsteps, every)
         J = 0.0
-        for s in range(nsteps):
-            grid.run_steps(1, nu=nu, uinf=uinf, fixed_dt=dts[s], sphere=sphere, **fkw)
-            J += dts[s] / T * sum(weights[k] * grid.last_body_force_body(k)[0] for k in range(n))
-            if (s + 1) % every == 0 and s + 1 < nsteps:
-                ckpts[s + 1] = grid.get_torch_velocity()
+        with _settled(grid):
+            for s in range(nsteps):
+                if s and s in ckpts:
+                    grid.keep_velocity(ckpts[s])
+                grid.run_steps(1, nu=nu, uinf=uinf, fixed_dt=dts[s], sphere=sphere, **fkw)
+                J += dts[s] / T * sum(weights[k] * grid.last_body_force_body(k)[0] for k in range(n))
         ctx.grid, ctx.nsteps, ctx.nu, ctx.uinf, ctx.dts, ctx.every = grid, nsteps, nu, uinf, list(dts), every
         ctx.sphere, ctx.bodies, ctx.weights, ctx.fkw, ctx.forcing, ctx.scheme = \
             sphere, bodies, list(weights), fkw, forcing, scheme
@@ -212,28 +254,25 @@ class BodiesRollout(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gJ):
-        grid, every, n = ctx.grid, ctx.every, len(ctx.bodies)
+        grid, n = ctx.grid, len(ctx.bodies)
         g = float(gJ)
-        lam = torch.zeros((3,) + grid.shape, dtype=grid._torch_dtype(), device="cuda")
+        grid.set_torch_adjoint(torch.zeros((3,) + grid.shape, dtype=grid._torch_dtype(), device="cuda"))
         dV = torch.zeros((n, 3), dtype=torch.float64)
         dW = torch.zeros((n, 3), dtype=torch.float64)
-        for s0 in sorted(ctx.ckpts, reverse=True):
-            s1 = min(s0 + every, ctx.nsteps)
-            states = [ctx.ckpts[s0]]
-            grid.set_torch_velocity(ctx.ckpts[s0])
-            for s in range(s0, s1 - 1):
-                grid.run_steps(1, nu=ctx.nu, uinf=ctx.uinf, fixed_dt=ctx.dts[s], sphere=ctx.sphere, **ctx.fkw)
-                states.append(grid.get_torch_velocity())
-            for s in reversed(range(s0, s1)):
-                grid.set_torch_velocity(states[s - s0])
-                grid.set_torch_adjoint(lam)
-                w = [g * ctx.dts[s] / ctx.T * wk for wk in ctx.weights]
-                dv, dw = grid.adjoint_step_bodies(ctx.dts[s], ctx.nu, ctx.uinf, ctx.bodies, ctx.sphere["lambda_"],
-                                                  ctx.sphere["implicit"], w, scheme=ctx.scheme,
-                                                  tke_target=ctx.forcing[0], injection_rate=ctx.forcing[1])
-                dV += torch.from_numpy(dv)
-                dW += torch.from_numpy(dw)
-                lam = grid.get_torch_adjoint()
+
+        def step(s):
+            grid.run_steps(1, nu=ctx.nu, uinf=ctx.uinf, fixed_dt=ctx.dts[s], sphere=ctx.sphere, **ctx.fkw)
+
+        def adjoint(s):
+            w = [g * ctx.dts[s] / ctx.T * wk for wk in ctx.weights]
+            dv, dw = grid.adjoint_step_bodies(ctx.dts[s], ctx.nu, ctx.uinf, ctx.bodies, ctx.sphere["lambda_"],
+                                              ctx.sphere["implicit"], w, scheme=ctx.scheme, tke_target=ctx.forcing[0],
+                                              injection_rate=ctx.forcing[1])
+            dV.add_(torch.from_numpy(dv))
+            dW.add_(torch.from_numpy(dw))
+
+        _backward_steps(grid, ctx.ckpts, ctx.nsteps, ctx.every, step, adjoint)
+        lam = grid.get_torch_adjoint()
         ctx.ckpts = None
         return (lam.to(ctx.u0_dtype), dV.to(ctx.vdev), dW.to(ctx.vdev), None, None, None, None, None, None, None,
                 None, None, None, None)

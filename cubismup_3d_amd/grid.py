@@ -141,6 +141,24 @@ class Grid:
         import torch
         return torch.stack([self.get_torch(n) for n in "uvw"])
 
+    # The velocity kept aside in the grid's own block order, for callers that restore it (the
+    # rollouts' checkpoints): device copies ordered on the grid's stream alone. The buffers are
+    # torch's, so whoever holds them synchronizes torch's stream after making them and the grid
+    # before letting them go.
+    def velocity_buffers(self, n: int):
+        import torch
+        out = [torch.empty((3, int(np.prod(self.shape))), dtype=self._torch_dtype(), device="cuda") for _ in range(n)]
+        torch.cuda.current_stream().synchronize()
+        return out
+
+    def keep_velocity(self, buf):
+        for q, n in enumerate("uvw"):
+            self._c(L.lib().cup_get_field_device(self._h, L.FIELD_IDS[n], C.c_void_p(buf[q].data_ptr())))
+
+    def restore_velocity(self, buf):
+        for q, n in enumerate("uvw"):
+            self._c(L.lib().cup_set_field_device(self._h, L.FIELD_IDS[n], C.c_void_p(buf[q].data_ptr())))
+
     def set_torch_adjoint(self, lam):
         for q, n in enumerate(("adjU", "adjV", "adjW")):
             self.set_torch(n, lam[q])
