@@ -67,7 +67,6 @@ static void release(Ctx& c)
   if (c.partials) hipFree(c.partials);
   if (c.ke_part) hipFree(c.ke_part);
   c.ke_part = nullptr;
-  if (c.red_part) hipFree(c.red_part);
   c.red_part = nullptr;
   if (c.low_part) hipFree(c.low_part);
   if (c.low_red) hipFree(c.low_red);
@@ -219,8 +218,10 @@ int cup_create(const cup_grid_desc* d, cup_ctx** out)
                         "hipHostMalloc")))
       break;
     if ((rc = ensure_partials(c, 20 * (size_t)c.nb + 1024))) break;
-    if ((rc = check_hip(c, hipMalloc(&c.red_part, REDUCE_CHUNKS * 32 * sizeof(double)), "hipMalloc reduction"))) break;
-    if ((rc = check_hip(c, hipMalloc(&c.ke_part, 4 * (size_t)c.nb * sizeof(double)), "hipMalloc ke"))) break;
+    if ((rc = check_hip(c, hipMalloc(&c.ke_part, (4 * (size_t)c.nb + REDUCE_CHUNKS * 32) * sizeof(double)),
+                        "hipMalloc ke")))
+      break;
+    c.red_part = c.ke_part + 4 * (size_t)c.nb;
     if ((rc = check_hip(c, hipMemsetAsync(c.ke_part, 0, 4 * (size_t)c.nb * sizeof(double), c.stream), "memset ke")))
       break;
     if ((rc = fft_setup(c))) break;
@@ -846,11 +847,16 @@ int cup_run_steps(cup_ctx* ctx, const cup_step_params* p, int nsteps)
       if (int rc = plain_step(ctx, p)) return rc;
     return check_hip(c, hipStreamSynchronize(c.stream), "run_steps");
   }
-  // FUSED: measure the current velocity and set dt for the coming step on the device.
-  if (int rc = launch_reset_umax(c)) return rc;
+  // FUSED: measure the current velocity and set dt for the coming step on the device. With a
+  // given dt the measurement is only for a call of no steps, whose state it is.
   c.umax_bank = 0;
-  if (int rc = launch_max_u(c, p->uinf, true)) return rc;
-  if (int rc = launch_finalize_step(c, p->CFL, p->nu, p->rampup, p->fixed_dt, 0)) return rc;
+  if (p->fixed_dt > 0 && nsteps > 0) {
+    if (int rc = launch_start_fixed(c, p->fixed_dt)) return rc;
+  } else {
+    if (int rc = launch_reset_umax(c)) return rc;
+    if (int rc = launch_max_u(c, p->uinf, true)) return rc;
+    if (int rc = launch_finalize_step(c, p->CFL, p->nu, p->rampup, p->fixed_dt, 0)) return rc;
+  }
   // With the central scheme each step's bookkeeping (k_finalize_step) runs inside the next
   // step's advection; the ramp needs the device step counter, read once here.
   const bool fold_ok = p->scheme == CUP_CENTRAL_EULER;

@@ -182,7 +182,7 @@ struct Ctx {
   void* ghat = nullptr;   // (padded grid) the Green's function's spectrum, FP64 complex
   double* partials = nullptr;
   size_t partials_cap = 0;  // doubles
-  double* red_part = nullptr;  // launch_reduce's first stage: [REDUCE_CHUNKS][up to 32 components]
+  double* red_part = nullptr;  // launch_reduce's first stage, behind ke_part: [REDUCE_CHUNKS][up to 32 components]
   double* ke_part = nullptr;  // [nb][4] partial sums |u|^2 of the fused step's velocity (per wave)
   DevScalars* sc = nullptr;
   DevScalars* sc_host = nullptr;  // pinned
@@ -354,6 +354,7 @@ int launch_count_nan(Ctx& c, long long out[4]);  // NaN cells of u, v, w, p (syn
 // Records the message of a failed call that has no context (read by cup_last_error(NULL)).
 int free_error(int code, const std::string& msg);
 int launch_reset_umax(Ctx& c);  // clears both banks
+int launch_start_fixed(Ctx& c, double dt);  // clears both banks and sets the dt
 int launch_inflow_correction(Ctx& c);  // UpdateAndCorrectInflow on the open faces of u
 int launch_poisson_mixed(Ctx& c);      // PoissonSolverMixed: rbuf (RHS) -> p
 int launch_poisson_unbounded(Ctx& c);  // PoissonSolverUnbounded: rbuf (RHS) -> p
