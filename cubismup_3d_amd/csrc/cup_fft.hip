@@ -302,6 +302,13 @@ constexpr int XFFT = XROWS / 2;  // complex FFTs per workgroup (two real rows ea
 
 enum XSrc { XSRC_FIELD = 0, XSRC_DIV = 1 };
 
+// Up to three fields that one launch transforms (one per grid z): a pass over a single field of a
+// small grid leaves CUs idle (128^3 FP32: three forward transforms 59 us one by one, 37 together).
+template <typename T>
+struct Three {
+  T* p[3];
+};
+
 // Real rows -> packed half spectrum. grid = (Ny/8, Nz).
 // FORCE (fused linear forcing): the same pass also forms, per grid row, the x-DFT at
 // kx = 0, 1, 2 of each advected velocity component and sum |u*|^2: 16 values per row
@@ -313,7 +320,7 @@ enum XSrc { XSRC_FIELD = 0, XSRC_DIV = 1 };
 // shuffles over ix plus an LDS sum over the 4 waves.
 template <typename T, int N, int SRC, bool FORCE>
 __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, const T* __restrict__ src1,
-                                                  const T* __restrict__ src2, C2<T>* __restrict__ S,
+                                                  const T* __restrict__ src2, Three<C2<T>> spec,
                                                   const C2<T>* __restrict__ tw, GridArgs g,
                                                   const DevScalars* __restrict__ sc, const int* __restrict__ ob_slot,
                                                   const T* __restrict__ ob_rhs, double* __restrict__ rowbuf,
@@ -327,6 +334,8 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
   __shared__ double rowacc[FORCE ? NT / 64 : 1][FORCE ? XROWS : 1][FORCE ? 3 * NA + 1 : 1];
   const int by = blockIdx.x, z = blockIdx.y;
   const int bz = z >> 3, iz = z & 7;
+  C2<T>* __restrict__ S = spec.p[blockIdx.z];
+  const T* __restrict__ field = blockIdx.z == 0 ? src0 : (blockIdx.z == 1 ? src1 : src2);
   T fac = 0;
   if (SRC == XSRC_DIV) fac = (T)(0.5 * g.h * g.h / sc->dt);
   T* rb = (T*)buf;
@@ -345,7 +354,7 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
     const size_t o = (size_t)b * BS3 + (iz * BS + iy) * BS + ix0;
     T val[4];
     if (SRC == XSRC_FIELD) {
-      const V4 a = *reinterpret_cast<const V4*>(src0 + o);
+      const V4 a = *reinterpret_cast<const V4*>(field + o);
       val[0] = a.x; val[1] = a.y; val[2] = a.z; val[3] = a.w;
     } else {
       const int slot = ob_slot ? ob_slot[b] : -1;
@@ -449,7 +458,7 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
 // XF: also write each block's x faces (ix = 0 and 7) to xf[(b*2 + side)*64 + iz*8 + iy], so that
 // the gradient reads them as 64 contiguous values instead of one value per 32-byte sector.
 template <typename T, int N, bool XF = false>
-__global__ __launch_bounds__(NT) void k_fft_x_inv(const C2<T>* __restrict__ S, T* __restrict__ dst,
+__global__ __launch_bounds__(NT) void k_fft_x_inv(Three<C2<T>> spec, Three<T> fields,
                                                   const C2<T>* __restrict__ tw, GridArgs g, FftPlan pl,
                                                   T* __restrict__ xf = nullptr)
 {
@@ -457,6 +466,8 @@ __global__ __launch_bounds__(NT) void k_fft_x_inv(const C2<T>* __restrict__ S, T
   C2<T>* buf = lds_tile<T, N * XFFT>();
   const int by = blockIdx.x, z = blockIdx.y;
   const int bz = z >> 3, iz = z & 7;
+  const C2<T>* __restrict__ S = spec.p[blockIdx.z];
+  T* __restrict__ dst = fields.p[blockIdx.z];
   for (int t = threadIdx.x; t < XFFT * (n / 2); t += NT) {
     const int q = t / (n / 2), k = t % (n / 2);
     const int ya = by * BS + 2 * q;
@@ -688,7 +699,7 @@ struct ColStages {
 // Column FFT along y (axis 1) or z (axis 2). grid = (ceil(ncols/TK), other axis). POISSON (z only):
 // forward transform, grid-consistent division and inverse transform.
 template <typename T, int N, int M, bool POISSON>
-__global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw,
+__global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(Three<C2<T>> S, const C2<T>* __restrict__ tw,
                                                                int ncols, int axis, int inv, int Ny, double norm,
                                                                const double* __restrict__ cx,
                                                                const double* __restrict__ cy,
@@ -701,7 +712,7 @@ __global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(C2<T>* __restri
   const int kx0 = blockIdx.x * CS::TK, o = blockIdx.y;
   const size_t base = (axis == 1 ? (size_t)o * Ny : (size_t)o) * ncols + kx0;
   const size_t stride = axis == 1 ? (size_t)ncols : (size_t)Ny * ncols;
-  CS cs{S,   buf, tw, base, stride, inv != 0, N > 0 ? N : pl.n, min(CS::TK, ncols - kx0), kx0, o, Ny, norm,
+  CS cs{S.p[blockIdx.z], buf, tw, base, stride, inv != 0, N > 0 ? N : pl.n, min(CS::TK, ncols - kx0), kx0, o, Ny, norm,
         cx,  cy,  cz, lmp,  coef};
   if constexpr (N > 0) cs.template run_ct<POISSON>();
   else cs.template run_rt<POISSON>(pl);
@@ -784,7 +795,7 @@ __device__ __forceinline__ void fft_b_to_a(C2<T> (&v)[16], C2<T>* buf, const C2<
 // pass) or row stage (2, beside the z pass; coef is the forcing's coefficient table), in the
 // column tile's LDS.
 template <typename T, int N, int AXIS, int MODE, bool FORCE = false, int EXTRA = 0>
-__global__ __launch_bounds__(NT) void k_fft_colr(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw, int ncols,
+__global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>* __restrict__ tw, int ncols,
                                                  int Ny, int Nz, double norm, const double* __restrict__ cx,
                                                  const double* __restrict__ cy, const double* __restrict__ cz,
                                                  const LowModes* __restrict__ lmp, const double* __restrict__ coef,
@@ -805,6 +816,7 @@ __global__ __launch_bounds__(NT) void k_fft_colr(C2<T>* __restrict__ S, const C2
       return;
     }
   }
+  C2<T>* __restrict__ S = spec.p[blockIdx.z];
   const int kx0 = blockIdx.x * TK, other = blockIdx.y - (EXTRA != 0 ? ex.ey : 0);
   const int f = threadIdx.x % TK, j = threadIdx.x / TK;
   const bool live = kx0 + f < ncols;
@@ -915,26 +927,27 @@ struct XPass {
     const int* slot = c.body.present && !c.plain_rhs ? c.ob_slot_all : nullptr;
     if (src == XSRC_FIELD)
       hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_FIELD, false>), grid, dim3(NT), lds(c), c.stream, s0, s1, s2,
-                         (C2<T>*)c.spec, (const C2<T>*)c.tw[0], c.grid(), c.sc, (const int*)nullptr,
+                         Three<C2<T>>{(C2<T>*)c.spec}, (const C2<T>*)c.tw[0], c.grid(), c.sc, (const int*)nullptr,
                          (const T*)nullptr, (double*)nullptr, c.plan[0]);
     else if (force)
-      hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_DIV, true>), grid, dim3(NT), lds(c), c.stream, s0, s1, s2, (C2<T>*)c.spec,
+      hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_DIV, true>), grid, dim3(NT), lds(c), c.stream, s0, s1, s2, Three<C2<T>>{(C2<T>*)c.spec},
                          (const C2<T>*)c.tw[0], c.grid(), c.sc, slot, (const T*)c.ob_rhs_all, c.low_part, c.plan[0]);
     else
       hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_DIV, false>), grid, dim3(NT), lds(c), c.stream, s0, s1, s2,
-                         (C2<T>*)c.spec, (const C2<T>*)c.tw[0], c.grid(), c.sc, slot, (const T*)c.ob_rhs_all,
+                         Three<C2<T>>{(C2<T>*)c.spec}, (const C2<T>*)c.tw[0], c.grid(), c.sc, slot, (const T*)c.ob_rhs_all,
                          (double*)nullptr, c.plan[0]);
   }
-  static void fwd_to(Ctx& c, const T* s0, C2<T>* spec)
+  // nf fields to their spectra, and back
+  static void fwd_to(Ctx& c, const Three<const T>& s, const Three<C2<T>>& spec, int nf)
   {
-    dim3 grid(c.N[1] / BS, c.N[2]);
-    hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_FIELD, false>), grid, dim3(NT), lds(c), c.stream, s0, s0, s0, spec,
-                       (const C2<T>*)c.tw[0], c.grid(), c.sc, (const int*)nullptr, (const T*)nullptr,
+    dim3 grid(c.N[1] / BS, c.N[2], nf);
+    hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_FIELD, false>), grid, dim3(NT), lds(c), c.stream, s.p[0], s.p[1], s.p[2],
+                       spec, (const C2<T>*)c.tw[0], c.grid(), c.sc, (const int*)nullptr, (const T*)nullptr,
                        (double*)nullptr, c.plan[0]);
   }
-  static void inv(Ctx& c, const C2<T>* spec, T* dst, T* xf = nullptr)
+  static void inv(Ctx& c, const Three<C2<T>>& spec, const Three<T>& dst, int nf, T* xf)
   {
-    dim3 grid(c.N[1] / BS, c.N[2]);
+    dim3 grid(c.N[1] / BS, c.N[2], nf);
     if (xf)
       hipLaunchKernelGGL((k_fft_x_inv<T, N, true>), grid, dim3(NT), lds(c), c.stream, spec, dst, (const C2<T>*)c.tw[0],
                          c.grid(), c.plan[0], xf);
@@ -948,7 +961,7 @@ template <typename T, int N, int AXIS>
 struct ColPass {
   // extra: 1 (y forward) or 2 (z pass with the forcing) runs the forcing's plane or row stage
   // beside the transforms; only the register form takes it (col_extra_ok)
-  static void run(Ctx& c, C2<T>* spec, int mode, double norm, bool force = false, int extra = 0)
+  static void run(Ctx& c, const Three<C2<T>>& spec, int nf, int mode, double norm, bool force = false, int extra = 0)
   {
     if constexpr (ColReg<T, N>::ok) {
       constexpr int TK = ColReg<T, N>::TK;
@@ -961,7 +974,7 @@ struct ColPass {
         const int work = extra == 1 ? ex.nz * ex.parts : ex.nz;
         ex.ey = (work + gx - 1) / gx;
       }
-      dim3 grid(gx, other + ex.ey);
+      dim3 grid(gx, other + ex.ey, nf);
       const C2<T>* tw = (const C2<T>*)c.tw[AXIS];
       if (mode == ZM_FWD && extra == 1)
         hipLaunchKernelGGL((k_fft_colr<T, N, AXIS, ZM_FWD, false, 1>), grid, dim3(NT), 0, c.stream, spec, tw, ncols,
@@ -986,20 +999,20 @@ struct ColPass {
                            c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr,
                            ex);
     } else if constexpr (N >= 512) {
-      launch<N, N>(c, spec, mode, norm, force);
+      launch<N, N>(c, spec, nf, mode, norm, force);
     } else {
       const int n = c.N[AXIS];
-      if (n <= 256) launch<0, 256>(c, spec, mode, norm, force);
-      else if (n <= 512) launch<0, 512>(c, spec, mode, norm, force);
-      else launch<0, FFT_MAX_N>(c, spec, mode, norm, force);
+      if (n <= 256) launch<0, 256>(c, spec, nf, mode, norm, force);
+      else if (n <= 512) launch<0, 512>(c, spec, nf, mode, norm, force);
+      else launch<0, FFT_MAX_N>(c, spec, nf, mode, norm, force);
     }
   }
   template <int NN, int M>
-  static void launch(Ctx& c, C2<T>* spec, int mode, double norm, bool force)
+  static void launch(Ctx& c, const Three<C2<T>>& spec, int nf, int mode, double norm, bool force)
   {
     using CT = ColTile<T, M>;
     const int ncols = c.N[0] / 2;
-    const dim3 grid((ncols + CT::TK - 1) / CT::TK, AXIS == 1 ? c.N[2] : c.N[1]), bt(CT::BT);
+    const dim3 grid((ncols + CT::TK - 1) / CT::TK, AXIS == 1 ? c.N[2] : c.N[1], nf), bt(CT::BT);
     const size_t lds = NN > 0 ? 0 : (size_t)c.N[AXIS] * CT::TK * sizeof(C2<T>);
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, grid, bt, lds, c.stream, spec, (const C2<T>*)c.tw[AXIS], ncols, AXIS,
@@ -1038,32 +1051,50 @@ struct GoXFwd {
 };
 template <typename T, int N>
 struct GoXFwdTo {
-  static void go(Ctx& c, const T* s0, C2<T>* spec) { XPass<T, N>::fwd_to(c, s0, spec); }
+  static void go(Ctx& c, const Three<const T>& s, const Three<C2<T>>& spec, int nf) { XPass<T, N>::fwd_to(c, s, spec, nf); }
 };
 template <typename T, int N>
 struct GoXInv {
-  static void go(Ctx& c, const C2<T>* spec, T* dst, T* xf = nullptr) { XPass<T, N>::inv(c, spec, dst, xf); }
+  static void go(Ctx& c, const Three<C2<T>>& spec, const Three<T>& dst, int nf, T* xf = nullptr)
+  {
+    XPass<T, N>::inv(c, spec, dst, nf, xf);
+  }
 };
 template <typename T, int N>
 struct GoY {
-  static void go(Ctx& c, C2<T>* spec, int mode, double norm) { ColPass<T, N, 1>::run(c, spec, mode, norm); }
+  static void go(Ctx& c, const Three<C2<T>>& spec, int nf, int mode, double norm)
+  {
+    ColPass<T, N, 1>::run(c, spec, nf, mode, norm);
+  }
 };
 template <typename T, int N>
 struct GoZ {
-  static void go(Ctx& c, C2<T>* spec, int mode, double norm) { ColPass<T, N, 2>::run(c, spec, mode, norm); }
+  static void go(Ctx& c, const Three<C2<T>>& spec, int nf, int mode, double norm)
+  {
+    ColPass<T, N, 2>::run(c, spec, nf, mode, norm);
+  }
 };
 template <typename T, int N>
 struct GoZF {
-  static void go(Ctx& c, C2<T>* spec, int mode, double norm) { ColPass<T, N, 2>::run(c, spec, mode, norm, true); }
+  static void go(Ctx& c, const Three<C2<T>>& spec, int mode, double norm)
+  {
+    ColPass<T, N, 2>::run(c, spec, 1, mode, norm, true);
+  }
 };
 // the same passes with the forcing's plane stage (y forward) or row stage (z) beside them
 template <typename T, int N>
 struct GoYPlanes {
-  static void go(Ctx& c, C2<T>* spec, int mode, double norm) { ColPass<T, N, 1>::run(c, spec, mode, norm, false, 1); }
+  static void go(Ctx& c, const Three<C2<T>>& spec, int mode, double norm)
+  {
+    ColPass<T, N, 1>::run(c, spec, 1, mode, norm, false, 1);
+  }
 };
 template <typename T, int N>
 struct GoZFRows {
-  static void go(Ctx& c, C2<T>* spec, int mode, double norm) { ColPass<T, N, 2>::run(c, spec, mode, norm, true, 2); }
+  static void go(Ctx& c, const Three<C2<T>>& spec, int mode, double norm)
+  {
+    ColPass<T, N, 2>::run(c, spec, 1, mode, norm, true, 2);
+  }
 };
 
 // The column lengths whose passes take the register form (ColReg::ok over dispatch_n's cases).
@@ -1077,7 +1108,7 @@ static double poisson_norm(const Ctx& c)
 template <typename T>
 static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rate, bool xface)
 {
-  C2<T>* S = (C2<T>*)c.spec;
+  const Three<C2<T>> S{(C2<T>*)c.spec};
   const double norm = poisson_norm(c);
   stage_mark(c, ST_XFWD, false);
   dispatch_n<GoXFwd, T>(c.N[0], c, (const T*)c.f[c.ustar], (const T*)c.f[c.ustar + 1],
@@ -1096,7 +1127,7 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
   }
   stage_mark(c, ST_YFWD, false);
   if (extra) dispatch_n<GoYPlanes, T>(c.N[1], c, S, (int)ZM_FWD, norm);
-  else dispatch_n<GoY, T>(c.N[1], c, S, (int)ZM_FWD, norm);
+  else dispatch_n<GoY, T>(c.N[1], c, S, 1, (int)ZM_FWD, norm);
   stage_mark(c, ST_YFWD, true);
   if (extra) {
     stage_mark(c, ST_FREDUCE, false);
@@ -1106,13 +1137,13 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
   stage_mark(c, ST_ZPASS, false);
   if (extra) dispatch_n<GoZFRows, T>(c.N[2], c, S, (int)ZM_POISSON, norm);
   else if (force) dispatch_n<GoZF, T>(c.N[2], c, S, (int)ZM_POISSON, norm);
-  else dispatch_n<GoZ, T>(c.N[2], c, S, (int)ZM_POISSON, norm);
+  else dispatch_n<GoZ, T>(c.N[2], c, S, 1, (int)ZM_POISSON, norm);
   stage_mark(c, ST_ZPASS, true);
   stage_mark(c, ST_YINV, false);
-  dispatch_n<GoY, T>(c.N[1], c, S, (int)ZM_INV, norm);
+  dispatch_n<GoY, T>(c.N[1], c, S, 1, (int)ZM_INV, norm);
   stage_mark(c, ST_YINV, true);
   stage_mark(c, ST_XINV, false);
-  dispatch_n<GoXInv, T>(c.N[0], c, (const C2<T>*)S, (T*)c.f[CUP_P], xface ? (T*)c.xface : (T*)nullptr);
+  dispatch_n<GoXInv, T>(c.N[0], c, S, Three<T>{(T*)c.f[CUP_P]}, 1, xface ? (T*)c.xface : (T*)nullptr);
   stage_mark(c, ST_XINV, true);
   c.xface_ok = xface;
   return check_hip(c, hipGetLastError(), "poisson_fused");
@@ -1121,19 +1152,19 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
 template <typename T>
 static int poisson_plain_t(Ctx& c)
 {
-  C2<T>* S = (C2<T>*)c.spec;
+  const Three<C2<T>> S{(C2<T>*)c.spec};
   const double norm = poisson_norm(c);
-  dispatch_n<GoXFwdTo, T>(c.N[0], c, (const T*)c.rbuf, S);
-  dispatch_n<GoY, T>(c.N[1], c, S, (int)ZM_FWD, norm);
-  dispatch_n<GoZ, T>(c.N[2], c, S, (int)ZM_FWD, norm);
+  dispatch_n<GoXFwdTo, T>(c.N[0], c, Three<const T>{(const T*)c.rbuf}, S, 1);
+  dispatch_n<GoY, T>(c.N[1], c, S, 1, (int)ZM_FWD, norm);
+  dispatch_n<GoZ, T>(c.N[2], c, S, 1, (int)ZM_FWD, norm);
   const size_t n = (size_t)(c.N[0] / 2) * c.N[1] * c.N[2];
   size_t gsz = (n + NT - 1) / NT;
   if (gsz > 65536) gsz = 65536;
-  hipLaunchKernelGGL((k_divide<T>), dim3((unsigned)gsz), dim3(NT), 0, c.stream, S, c.N[0] / 2, c.N[1], c.N[2], norm,
+  hipLaunchKernelGGL((k_divide<T>), dim3((unsigned)gsz), dim3(NT), 0, c.stream, S.p[0], c.N[0] / 2, c.N[1], c.N[2], norm,
                      (const double*)c.cos4[0], (const double*)c.cos4[1], (const double*)c.cos4[2]);
-  dispatch_n<GoZ, T>(c.N[2], c, S, (int)ZM_INV, norm);
-  dispatch_n<GoY, T>(c.N[1], c, S, (int)ZM_INV, norm);
-  dispatch_n<GoXInv, T>(c.N[0], c, (const C2<T>*)S, (T*)c.rbuf);
+  dispatch_n<GoZ, T>(c.N[2], c, S, 1, (int)ZM_INV, norm);
+  dispatch_n<GoY, T>(c.N[1], c, S, 1, (int)ZM_INV, norm);
+  dispatch_n<GoXInv, T>(c.N[0], c, S, Three<T>{(T*)c.rbuf}, 1);
   return check_hip(c, hipGetLastError(), "poisson_plain");
 }
 
@@ -1151,33 +1182,45 @@ int launch_poisson_plain(Ctx& c)
 }
 
 template <typename T>
-static int fwd_field_t(Ctx& c, const void* real_blocks, void* spec)
+static int fwd_fields_t(Ctx& c, const void* const* real_blocks, void* const* spec, int nf)
 {
-  C2<T>* S = (C2<T>*)spec;
-  dispatch_n<GoXFwdTo, T>(c.N[0], c, (const T*)real_blocks, S);
-  dispatch_n<GoY, T>(c.N[1], c, S, (int)ZM_FWD, 0.0);
-  dispatch_n<GoZ, T>(c.N[2], c, S, (int)ZM_FWD, 0.0);
-  return check_hip(c, hipGetLastError(), "fft_forward_field");
+  Three<const T> s{};
+  Three<C2<T>> S{};
+  for (int q = 0; q < nf; ++q) {
+    s.p[q] = (const T*)real_blocks[q];
+    S.p[q] = (C2<T>*)spec[q];
+  }
+  dispatch_n<GoXFwdTo, T>(c.N[0], c, s, S, nf);
+  dispatch_n<GoY, T>(c.N[1], c, S, nf, (int)ZM_FWD, 0.0);
+  dispatch_n<GoZ, T>(c.N[2], c, S, nf, (int)ZM_FWD, 0.0);
+  return check_hip(c, hipGetLastError(), "fft_forward_fields");
 }
 
 template <typename T>
-static int inv_field_t(Ctx& c, void* spec, void* real_blocks)
+static int inv_fields_t(Ctx& c, void* const* spec, void* const* real_blocks, int nf)
 {
-  C2<T>* S = (C2<T>*)spec;
-  dispatch_n<GoZ, T>(c.N[2], c, S, (int)ZM_INV, 0.0);
-  dispatch_n<GoY, T>(c.N[1], c, S, (int)ZM_INV, 0.0);
-  dispatch_n<GoXInv, T>(c.N[0], c, (const C2<T>*)S, (T*)real_blocks);
-  return check_hip(c, hipGetLastError(), "fft_inverse_field");
+  Three<T> d{};
+  Three<C2<T>> S{};
+  for (int q = 0; q < nf; ++q) {
+    d.p[q] = (T*)real_blocks[q];
+    S.p[q] = (C2<T>*)spec[q];
+  }
+  dispatch_n<GoZ, T>(c.N[2], c, S, nf, (int)ZM_INV, 0.0);
+  dispatch_n<GoY, T>(c.N[1], c, S, nf, (int)ZM_INV, 0.0);
+  dispatch_n<GoXInv, T>(c.N[0], c, S, d, nf);
+  return check_hip(c, hipGetLastError(), "fft_inverse_fields");
 }
 
-int launch_fft_forward_field(Ctx& c, const void* real_blocks, void* spec)
+int launch_fft_forward_fields(Ctx& c, const void* const* real_blocks, void* const* spec, int nf)
 {
-  return c.precision == 4 ? fwd_field_t<float>(c, real_blocks, spec) : fwd_field_t<double>(c, real_blocks, spec);
+  return c.precision == 4 ? fwd_fields_t<float>(c, real_blocks, spec, nf)
+                          : fwd_fields_t<double>(c, real_blocks, spec, nf);
 }
 
-int launch_fft_inverse_field(Ctx& c, void* spec, void* real_blocks)
+int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_blocks, int nf)
 {
-  return c.precision == 4 ? inv_field_t<float>(c, spec, real_blocks) : inv_field_t<double>(c, spec, real_blocks);
+  return c.precision == 4 ? inv_fields_t<float>(c, spec, real_blocks, nf)
+                          : inv_fields_t<double>(c, spec, real_blocks, nf);
 }
 
 // ------------------------------------------------------- PoissonSolverMixed
@@ -1541,7 +1584,7 @@ static int unbounded_setup_t(Ctx& c)
     return CUP_E_NOMEM;
   // the Green's function's spectrum, normalized by the padded size, kept in FP64
   hipLaunchKernelGGL((k_green<T>), dim3(p->nb), dim3(NT), 0, c.stream, (T*)p->rbuf, p->grid(), c.h);
-  if (int rc = launch_fft_forward_field(*p, p->rbuf, p->spec)) return set_error(c, rc, "poisson_unbounded: " + p->err);
+  if (int rc = launch_fft_forward_fields(*p, &p->rbuf, &p->spec, 1)) return set_error(c, rc, "poisson_unbounded: " + p->err);
   const double norm = 1.0 / ((double)p->N[0] * p->N[1] * p->N[2]);
   std::vector<C2<T>> hs(nspec);
   std::vector<C2<double>> gd(nspec);
@@ -1567,12 +1610,12 @@ static int poisson_unbounded_t(Ctx& c)
   Ctx& p = *c.unb;
   p.stream = c.stream;
   hipLaunchKernelGGL((k_pad_blocks<T>), dim3(c.nb), dim3(NT), 0, c.stream, (const T*)c.rbuf, (T*)p.rbuf, c.grid(), 0);
-  if (int rc = launch_fft_forward_field(p, p.rbuf, p.spec)) return set_error(c, rc, "poisson_unbounded: " + p.err);
+  if (int rc = launch_fft_forward_fields(p, &p.rbuf, &p.spec, 1)) return set_error(c, rc, "poisson_unbounded: " + p.err);
   const size_t n = (size_t)(p.N[0] / 2) * p.N[1] * p.N[2];
   const unsigned gsz = (unsigned)std::min<size_t>(65536, (n + NT - 1) / NT);
   hipLaunchKernelGGL((k_green_mul<T>), dim3(gsz), dim3(NT), 0, c.stream, (C2<T>*)p.spec, (const C2<double>*)p.ghat,
                      p.N[0] / 2, p.N[1], p.N[2]);
-  if (int rc = launch_fft_inverse_field(p, p.spec, p.f[CUP_P])) return set_error(c, rc, "poisson_unbounded: " + p.err);
+  if (int rc = launch_fft_inverse_fields(p, &p.spec, &p.f[CUP_P], 1)) return set_error(c, rc, "poisson_unbounded: " + p.err);
   hipLaunchKernelGGL((k_pad_blocks<T>), dim3(c.nb), dim3(NT), 0, c.stream, (const T*)p.f[CUP_P], (T*)c.f[CUP_P],
                      c.grid(), 1);
   return check_hip(c, hipGetLastError(), "poisson_unbounded");

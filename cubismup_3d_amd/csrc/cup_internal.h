@@ -368,12 +368,13 @@ int fft_setup(Ctx& c);
 int launch_poisson_fused(Ctx& c, bool force = false, double tke_target = 0, double inj_rate = 0,
                          bool xface = false);  // div(tmp) -> p
 int launch_poisson_plain(Ctx& c);   // rhs in rbuf -> solution in rbuf (separate divide pass)
-int launch_fft_forward_field(Ctx& c, const void* real_blocks, void* spec);  // 3 passes
+// nf <= 3 fields to their spectra and back, one launch per pass (3 passes)
+int launch_fft_forward_fields(Ctx& c, const void* const* real_blocks, void* const* spec, int nf);
+int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_blocks, int nf);
 // HIT analysis: out[0..2] = raw sums tke, eps, l_integral numerator; E[nbin] raw shell sums;
 // grad[2] = sum sqrt(grad2), sum grad2 (see cup_hit_analysis)
 int launch_hit_analysis(Ctx& c, double* tke_eps_lint, double* E, int nbin, double grad[2]);
 int launch_grad_stats(Ctx& c, double out[2]);  // sums of sqrt(grad2) and grad2 (synchronous)
-int launch_fft_inverse_field(Ctx& c, void* spec, void* real_blocks);        // 3 passes
 // cup_spectral.hip
 int spectral_setup(Ctx& c);
 int launch_ic_hit(Ctx& c, double k0, const double* K, const double* E, int tn, double u_rms, uint64_t seed);

@@ -177,9 +177,8 @@ int launch_ic_hit(Ctx& c, double k0, const double* K, const double* E, int tn, d
     hipFree(table);
   }
   if (krc) return krc;
-  if (int rc = launch_fft_inverse_field(c, c.spec, c.f[CUP_U])) return rc;
-  if (int rc = launch_fft_inverse_field(c, c.spec2, c.f[CUP_V])) return rc;
-  if (int rc = launch_fft_inverse_field(c, c.spec3, c.f[CUP_W])) return rc;
+  void* specs[3] = {c.spec, c.spec2, c.spec3};
+  if (int rc = launch_fft_inverse_fields(c, specs, c.f + CUP_U, 3)) return rc;
   const double zero[3] = {0, 0, 0};
   if (int rc = launch_max_u(c, zero)) return rc;
   if (int rc = launch_reduce(c, c.nb, 2, 1u, c.sc->red)) return rc;
@@ -312,9 +311,8 @@ static int forcing_plain_t(Ctx& c, double dt, double sim_dt, double nu, double t
   if (int rc = alloc_extra_spectra(c)) return rc;
   const int v0 = field >= 0 ? field : (c.decomposition == CUP_FUSED ? c.ustar : CUP_U);
   // SpectralForcing::_cub2fftw + runFwd: three forward transforms.
-  if (int rc = launch_fft_forward_field(c, c.f[v0], c.spec)) return rc;
-  if (int rc = launch_fft_forward_field(c, c.f[v0 + 1], c.spec2)) return rc;
-  if (int rc = launch_fft_forward_field(c, c.f[v0 + 2], c.spec3)) return rc;
+  void* specs[3] = {c.spec, c.spec2, c.spec3};
+  if (int rc = launch_fft_forward_fields(c, c.f + v0, specs, 3)) return rc;
   const size_t n = (size_t)(c.N[0] / 2) * c.N[1] * c.N[2];
   dim3 g = grid_for(n);
   if (g.x > 4096) g.x = 4096;
@@ -341,9 +339,8 @@ static int forcing_plain_t(Ctx& c, double dt, double sim_dt, double nu, double t
   else if (inj_rate > 0) inj = inj_rate;
   const double fac = sim_dt * inj / (2 * tkeF);
   if (fac > 0) {
-    void* specs[3] = {c.spec, c.spec2, c.spec3};
     for (int q = 0; q < 3; ++q) {
-      if (int rc = launch_fft_inverse_field(c, specs[q], c.rbuf)) return rc;
+      if (int rc = launch_fft_inverse_fields(c, specs + q, &c.rbuf, 1)) return rc;
       hipLaunchKernelGGL((k_axpy_blocks<T>), grid_for(c.ncell), dim3(NT), 0, c.stream, (T*)c.f[v0 + q],
                          (const T*)c.rbuf, c.ncell, fac / normFFT);
       if (int rc = check_hip(c, hipGetLastError(), "k_axpy_blocks")) return rc;
@@ -405,16 +402,14 @@ static int adjoint_forcing_t(Ctx& c, int us0, double dt, double tke_target, doub
   const double wf[3] = {2 * M_PI / c.extent[0], 2 * M_PI / c.extent[1], 2 * M_PI / c.extent[2]};
   void* specs[3] = {c.spec, c.spec2, c.spec3};
   auto filtered = [&](int f0) {  // spectra of fields f0.. filtered, band sums in c.partials
-    for (int q = 0; q < 3; ++q)
-      if (int rc = launch_fft_forward_field(c, c.f[f0 + q], specs[q])) return rc;
+    if (int rc = launch_fft_forward_fields(c, c.f + f0, specs, 3)) return rc;
     hipLaunchKernelGGL((k_forcing_filter<T>), g, dim3(NT), 0, c.stream, (C2<T>*)c.spec, (C2<T>*)c.spec2,
                        (C2<T>*)c.spec3, c.N[0], c.N[1], c.N[2], wf[0], wf[1], wf[2], c.partials);
     return check_hip(c, hipGetLastError(), "k_forcing_filter");
   };
   auto inverse = [&](T* dst) {
-    for (int q = 0; q < 3; ++q)
-      if (int rc = launch_fft_inverse_field(c, specs[q], dst + q * c.ncell)) return rc;
-    return CUP_OK;
+    void* d[3] = {dst, dst + c.ncell, dst + 2 * c.ncell};
+    return launch_fft_inverse_fields(c, specs, d, 3);
   };
   auto scalars = [&]() {
     if (int rc = check_hip(c, hipMemcpyAsync(c.sc_host, c.sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c.stream),
@@ -837,9 +832,8 @@ static int hit_analysis_t(Ctx& c, double* sums, double* E, int nbin)
   const size_t nrows = 3 + (size_t)nbin;
   if (!c.ana && check_hip(c, hipMalloc(&c.ana, (nrows * nlines + nrows) * sizeof(double)), "hipMalloc analysis"))
     return CUP_E_NOMEM;
-  if (int rc = launch_fft_forward_field(c, c.f[CUP_U], c.spec)) return rc;
-  if (int rc = launch_fft_forward_field(c, c.f[CUP_V], c.spec2)) return rc;
-  if (int rc = launch_fft_forward_field(c, c.f[CUP_W], c.spec3)) return rc;
+  void* specs[3] = {c.spec, c.spec2, c.spec3};
+  if (int rc = launch_fft_forward_fields(c, c.f + CUP_U, specs, 3)) return rc;
   if (int rc = check_hip(c, hipMemsetAsync(c.ana, 0, nrows * nlines * sizeof(double), c.stream), "memset analysis"))
     return rc;
   int maxN = std::max(c.N[0], std::max(c.N[1], c.N[2]));
