@@ -53,6 +53,8 @@ static void release(Ctx& c)
     if (p) { hipFree(p); p = nullptr; }
   if (c.ana) hipFree(c.ana);
   c.ana = nullptr;
+  if (c.ana_host) hipHostFree(c.ana_host);
+  c.ana_host = nullptr;
   void** bufs[] = {&c.spec, &c.spec2, &c.spec3, &c.rbuf, &c.xface, &c.tw[0], &c.tw[1], &c.tw[2]};
   for (void** b : bufs)
     if (*b) { hipFree(*b); *b = nullptr; }

@@ -163,7 +163,8 @@ struct Ctx {
   bool periodic() const { return bc[0] == CUP_BC_PERIODIC && bc[1] == CUP_BC_PERIODIC && bc[2] == CUP_BC_PERIODIC; }
   bool plain_rhs = false; // the fused x pass ignores the obstacle RHS (the adjoint's projection)
   void* spec = nullptr;   // packed half spectrum, complex, [z][y][kx], kx < Nx/2
-  double* ana = nullptr;  // HIT analysis: per-line sums [3 + nbin][Ny*Nz], then the row totals (lazy)
+  double* ana = nullptr;  // HIT analysis: per-wave sums [3 + nbin][waves], then the row totals (lazy)
+  double* ana_host = nullptr;  // pinned: the totals
   void* spec2 = nullptr;  // extra spectra for the plain forcing path
   void* spec3 = nullptr;
   void* rbuf = nullptr;   // block-layout real scratch (plain RHS / solution)
@@ -374,7 +375,7 @@ int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_block
 // HIT analysis: out[0..2] = raw sums tke, eps, l_integral numerator; E[nbin] raw shell sums;
 // grad[2] = sum sqrt(grad2), sum grad2 (see cup_hit_analysis)
 int launch_hit_analysis(Ctx& c, double* tke_eps_lint, double* E, int nbin, double grad[2]);
-int launch_grad_stats(Ctx& c, double out[2]);  // sums of sqrt(grad2) and grad2 (synchronous)
+int launch_grad_stats(Ctx& c, double* out_dev);  // sums of sqrt(grad2) and grad2
 // cup_spectral.hip
 int spectral_setup(Ctx& c);
 int launch_ic_hit(Ctx& c, double k0, const double* K, const double* E, int tn, double u_rms, uint64_t seed);

@@ -1676,58 +1676,89 @@ int launch_finalize_step(Ctx& c, double CFL, double nu, int rampup, double fixed
 
 // ------------------------------------------------------------------ diagnostics
 
-// KernelDissipation (ComputeDissipation.cpp:46-115): 20 FP64 integrals. A workgroup sums
-// nbw consecutive blocks (one block reduction per workgroup) into part[20*wg].
+// The seven values of a 7-point stencil at cell k (0 or 1) of a thread's pair in a pipelined lab.
 template <typename T>
+struct Star {
+  T c, E, W, N, S, B, F;
+};
+template <int PXV, typename T>
+__device__ __forceinline__ void star_pair(const T* F, int l, Star<T> (&o)[2])
+{
+  using V2 = typename Vec2<T>::type;
+  using LG = LabGeom<PXV>;
+  const V2 C = *reinterpret_cast<const V2*>(F + l);
+  const V2 Nn = *reinterpret_cast<const V2*>(F + l + LG::PY), Sn = *reinterpret_cast<const V2*>(F + l - LG::PY);
+  const V2 Bn = *reinterpret_cast<const V2*>(F + l + LG::PZ), Fn = *reinterpret_cast<const V2*>(F + l - LG::PZ);
+  o[0] = Star<T>{C.x, C.y, F[l - 1], Nn.x, Sn.x, Bn.x, Fn.x};
+  o[1] = Star<T>{C.y, F[l + 2], C.x, Nn.y, Sn.y, Bn.y, Fn.y};
+}
+
+// KernelDissipation (ComputeDissipation.cpp:46-115): 20 FP64 integrals. A workgroup sums
+// nbw consecutive blocks (one block reduction per workgroup) into part[20*wg], fetching the next
+// block's lab while the current one is summed: about 200 FP64 operations a cell bound it (37 us
+// at 128^3 FP32 with each block fetched, waited for and summed in turn, 34 so).
+template <typename T, bool BC>
 __global__ __launch_bounds__(NT) void k_diagnostics(const T* __restrict__ u, const T* __restrict__ v,
                                                     const T* __restrict__ w, const T* __restrict__ p,
                                                     const T* __restrict__ chi, GridArgs g, double nu, double cx,
                                                     double cy, double cz, double* __restrict__ part, int nbw)
 {
-  __shared__ T lab[4][L1C];
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  using V2 = typename Vec2<T>::type;
+  __shared__ __align__(16) T lab[4][LabGeom<PX_GRAD>::PLC];
+  const LabSlots s = lab_slots<PX_GRAD>();
+  const int b0 = xcd_remap(blockIdx.x, gridDim.x) * nbw, c0 = 2 * threadIdx.x;
   const T* src[4] = {u, v, w, p};
+  LabRegs<T, 4> r;
+  V2 xc;
+  auto fetch = [&](int b) {
+    lab_fetch<BC>(r, src, s, g, b, {HK_VEL, HK_VEL, HK_VEL, HK_COPY});
+    xc = *reinterpret_cast<const V2*>(chi + (size_t)b * BS3 + c0);
+  };
+  fetch(b0);
   const double h = g.h, hCube = h * h * h, inv2h = .5 / h, invHh = 1 / (h * h);
   double R[20];
 #pragma unroll
   for (int i = 0; i < 20; ++i) R[i] = 0;
   for (int j = 0; j < nbw; ++j) {
-    const int b = wg * nbw + j;
+    const int b = b0 + j;
     int bx, by, bz;
     block_coords(g, b, bx, by, bz);
     if (j) __syncthreads();  // the previous block is done with the lab
-    gather_g1<T, 4>(src, lab, g, b, bx, by, bz, {HK_VEL, HK_VEL, HK_VEL, HK_COPY});
+    lab_put<PX_GRAD>(r, lab, s);
+    const T xv[2] = {xc.x, xc.y};
     __syncthreads();
-    for (int c = threadIdx.x; c < BS3; c += NT) {
-      const int ix = c & 7, iy = (c >> 3) & 7, iz = c >> 6;
-      const int l = ((iz + 1) * L1 + iy + 1) * L1 + ix + 1;
-      const int E = l + 1, W = l - 1, N = l + L1, S = l - L1, B = l + L1 * L1, F = l - L1 * L1;
-      const T* U = lab[0];
-      const T* V = lab[1];
-      const T* Wv = lab[2];
-      const T* P = lab[3];
-      const double X = (double)chi[(size_t)b * BS3 + c];
+    if (j + 1 < nbw) fetch(b + 1);
+    Star<T> su[2], sv[2], sw[2], sp[2];
+    star_pair<PX_GRAD>(lab[0], s.li, su);
+    star_pair<PX_GRAD>(lab[1], s.li, sv);
+    star_pair<PX_GRAD>(lab[2], s.li, sw);
+    star_pair<PX_GRAD>(lab[3], s.li, sp);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const Star<T>&U = su[k], &V = sv[k], &Q = sw[k], &P = sp[k];
+      const int c = c0 + k, ix = c & 7, iy = (c >> 3) & 7, iz = c >> 6;
+      const double X = (double)xv[k];
       const double PX = (bx * BS + ix + 0.5) * h - cx, PY = (by * BS + iy + 0.5) * h - cy, PZ = (bz * BS + iz + 0.5) * h - cz;
-      const double Lu = U[l], Lv = V[l], Lw = Wv[l];
-      const double WX = inv2h * (((double)Wv[N] - Wv[S]) - ((double)V[B] - V[F]));
-      const double WY = inv2h * (((double)U[B] - U[F]) - ((double)Wv[E] - Wv[W]));
-      const double WZ = inv2h * (((double)V[E] - V[W]) - ((double)U[N] - U[S]));
-      const double dPdx = inv2h * ((double)P[E] - P[W]);
-      const double dPdy = inv2h * ((double)P[N] - P[S]);
-      const double dPdz = inv2h * ((double)P[B] - P[F]);
+      const double Lu = U.c, Lv = V.c, Lw = Q.c;
+      const double WX = inv2h * (((double)Q.N - Q.S) - ((double)V.B - V.F));
+      const double WY = inv2h * (((double)U.B - U.F) - ((double)Q.E - Q.W));
+      const double WZ = inv2h * (((double)V.E - V.W) - ((double)U.N - U.S));
+      const double dPdx = inv2h * ((double)P.E - P.W);
+      const double dPdy = inv2h * ((double)P.N - P.S);
+      const double dPdz = inv2h * ((double)P.B - P.F);
       R[15] -= (1 - X) * hCube * (dPdx * Lu + dPdy * Lv + dPdz * Lw);
-      const double lapU = invHh * ((double)U[E] + U[W] + U[N] + U[S] + U[B] + U[F] - 6 * Lu);
-      const double lapV = invHh * ((double)V[E] + V[W] + V[N] + V[S] + V[B] + V[F] - 6 * Lv);
-      const double lapW = invHh * ((double)Wv[E] + Wv[W] + Wv[N] + Wv[S] + Wv[B] + Wv[F] - 6 * Lw);
+      const double lapU = invHh * ((double)U.E + U.W + U.N + U.S + U.B + U.F - 6 * Lu);
+      const double lapV = invHh * ((double)V.E + V.W + V.N + V.S + V.B + V.F - 6 * Lv);
+      const double lapW = invHh * ((double)Q.E + Q.W + Q.N + Q.S + Q.B + Q.F - 6 * Lw);
       const double V1 = lapU * Lu + lapV * Lv + lapW * Lw;
-      const double D11 = inv2h * ((double)U[E] - U[W]);
-      const double D22 = inv2h * ((double)V[N] - V[S]);
-      const double D33 = inv2h * ((double)Wv[B] - Wv[F]);
-      const double D12 = inv2h * ((double)U[N] - U[S] + V[E] - V[W]) / 2;
-      const double D13 = inv2h * ((double)U[B] - U[F] + Wv[E] - Wv[W]) / 2;
-      const double D23 = inv2h * ((double)Wv[N] - Wv[S] + V[B] - V[F]) / 2;
-      const double V2 = D11 * D11 + D22 * D22 + D33 * D33 + 2 * (D12 * D12 + D13 * D13 + D23 * D23);
-      R[16] += (1 - X) * hCube * nu * (V1 + 2 * V2);
+      const double D11 = inv2h * ((double)U.E - U.W);
+      const double D22 = inv2h * ((double)V.N - V.S);
+      const double D33 = inv2h * ((double)Q.B - Q.F);
+      const double D12 = inv2h * ((double)U.N - U.S + V.E - V.W) / 2;
+      const double D13 = inv2h * ((double)U.B - U.F + Q.E - Q.W) / 2;
+      const double D23 = inv2h * ((double)Q.N - Q.S + V.B - V.F) / 2;
+      const double V2s = D11 * D11 + D22 * D22 + D33 * D33 + 2 * (D12 * D12 + D13 * D13 + D23 * D23);
+      R[16] += (1 - X) * hCube * nu * (V1 + 2 * V2s);
       R[0] += hCube * WX;
       R[1] += hCube * WY;
       R[2] += hCube * WZ;
@@ -1748,20 +1779,21 @@ __global__ __launch_bounds__(NT) void k_diagnostics(const T* __restrict__ u, con
       R[19] += sqrt(WX * WX + WY * WY + WZ * WZ);
     }
   }
-  block_reduce<20>(R, 0u, part + 20 * (size_t)wg);
+  block_reduce<20>(R, 0u, part + 20 * (size_t)(b0 / nbw));
 }
 
-// Blocks per diagnostics workgroup: 8 when the x rows allow it.
-inline int diag_nbw_x(int bpdx) { return bpdx % 8 == 0 ? 8 : (bpdx % 4 == 0 ? 4 : (bpdx % 2 == 0 ? 2 : 1)); }
-inline int diag_nbw(const Ctx& c) { return diag_nbw_x(c.bpd[0]); }
+// Blocks per diagnostics workgroup: 8 where the x rows allow it and 1024 workgroups remain.
+inline int diag_nbw(int bpdx, long long nb) { return walk_blocks(bpdx, (int)std::min(nb, 1ll << 30), 8, 1024); }
+inline int diag_nbw(const Ctx& c) { return diag_nbw(c.bpd[0], c.nb); }
 
 template <typename T>
 static int diagnostics_t(Ctx& c, double nu)
 {
   const int nbw = diag_nbw(c);
-  hipLaunchKernelGGL((k_diagnostics<T>), dim3(c.nb / nbw), dim3(NT), 0, c.stream, (const T*)c.f[CUP_U],
-                     (const T*)c.f[CUP_V], (const T*)c.f[CUP_W], (const T*)c.f[CUP_P], (const T*)c.f[CUP_CHI],
-                     c.grid(), nu, c.extent[0] / 2, c.extent[1] / 2, c.extent[2] / 2, c.partials, nbw);
+  auto kern = c.periodic() ? k_diagnostics<T, false> : k_diagnostics<T, true>;
+  hipLaunchKernelGGL(kern, dim3(c.nb / nbw), dim3(NT), 0, c.stream, (const T*)c.f[CUP_U], (const T*)c.f[CUP_V],
+                     (const T*)c.f[CUP_W], (const T*)c.f[CUP_P], (const T*)c.f[CUP_CHI], c.grid(), nu,
+                     c.extent[0] / 2, c.extent[1] / 2, c.extent[2] / 2, c.partials, nbw);
   return check_hip(c, hipGetLastError(), "k_diagnostics");
 }
 
@@ -1773,37 +1805,41 @@ __global__ __launch_bounds__(NT) void k_grad_stats(const T* __restrict__ u, cons
                                                    const T* __restrict__ w, GridArgs g, double* __restrict__ part,
                                                    int nbw)
 {
-  __shared__ T lab[3][L1C];
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  __shared__ __align__(16) T lab[3][LabGeom<PX_GRAD>::PLC];
+  const LabSlots s = lab_slots<PX_GRAD>();
+  const int b0 = xcd_remap(blockIdx.x, gridDim.x) * nbw;
   const T* src[3] = {u, v, w};
   const double fac = 1 / (4 * g.h * g.h);
   double R[2] = {0, 0};
+  LabRegs<T, 3> r;
+  lab_fetch<false>(r, src, s, g, b0, {HK_VEL, HK_VEL, HK_VEL});  // the HIT analysis is of periodic boxes
   for (int j = 0; j < nbw; ++j) {
-    const int b = wg * nbw + j;
-    int bx, by, bz;
-    block_coords(g, b, bx, by, bz);
     if (j) __syncthreads();  // the previous block is done with the lab
-    gather_g1<T, 3>(src, lab, g, b, bx, by, bz, {HK_VEL, HK_VEL, HK_VEL});
+    lab_put<PX_GRAD>(r, lab, s);
     __syncthreads();
-    for (int c = threadIdx.x; c < BS3; c += NT) {
-      const int l = (((c >> 6) + 1) * L1 + ((c >> 3) & 7) + 1) * L1 + (c & 7) + 1;
-      double g2 = 0;
+    if (j + 1 < nbw) lab_fetch<false>(r, src, s, g, b0 + j + 1, {HK_VEL, HK_VEL, HK_VEL});
+    double g2[2] = {0, 0};
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const T* F = lab[q];
-        const double dx = (double)F[l + 1] - F[l - 1], dy = (double)F[l + L1] - F[l - L1],
-                     dz = (double)F[l + L1 * L1] - F[l - L1 * L1];
-        g2 += dx * dx + dy * dy + dz * dz;
+    for (int q = 0; q < 3; ++q) {
+      Star<T> f[2];
+      star_pair<PX_GRAD>(lab[q], s.li, f);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const double dx = (double)f[k].E - f[k].W, dy = (double)f[k].N - f[k].S, dz = (double)f[k].B - f[k].F;
+        g2[k] += dx * dx + dy * dy + dz * dz;
       }
-      g2 *= fac;
-      R[0] += sqrt(g2);
-      R[1] += g2;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      g2[k] *= fac;
+      R[0] += sqrt(g2[k]);
+      R[1] += g2[k];
     }
   }
-  block_reduce<2>(R, 0u, part + 2 * (size_t)wg);
+  block_reduce<2>(R, 0u, part + 2 * (size_t)(b0 / nbw));
 }
 
-int launch_grad_stats(Ctx& c, double out[2])
+int launch_grad_stats(Ctx& c, double* out_dev)
 {
   if (int e = ensure_partials(c, 2 * (size_t)c.nb)) return e;
   const int nbw = diag_nbw(c);
@@ -1813,11 +1849,7 @@ int launch_grad_stats(Ctx& c, double out[2])
   else
     hipLaunchKernelGGL((k_grad_stats<double>), dim3(c.nb / nbw), dim3(NT), 0, c.stream, (const double*)c.f[CUP_U],
                        (const double*)c.f[CUP_V], (const double*)c.f[CUP_W], c.grid(), c.partials, nbw);
-  if (int rc = launch_reduce(c, c.nb / nbw, 2, 0u, c.sc->red)) return rc;
-  if (int rc = check_hip(c, hipMemcpyAsync(out, c.sc->red, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream),
-                         "hipMemcpy grad stats"))
-    return rc;
-  return check_hip(c, hipStreamSynchronize(c.stream), "synchronize");
+  return launch_reduce(c, c.nb / nbw, 2, 0u, out_dev);
 }
 
 int launch_diagnostics(Ctx& c, double nu, int* nparts)
@@ -1857,7 +1889,8 @@ template <typename T>
 static int diagnostics_noalloc_t(const void* const fields[5], const GridArgs& g, const double half_extent[3],
                                  double nu, int nbw, double* part, hipStream_t s, double* out_dev)
 {
-  hipLaunchKernelGGL((k_diagnostics<T>), dim3(g.nb / nbw), dim3(NT), 0, s, (const T*)fields[CUP_U],
+  auto kern = g.bcany ? k_diagnostics<T, true> : k_diagnostics<T, false>;
+  hipLaunchKernelGGL(kern, dim3(g.nb / nbw), dim3(NT), 0, s, (const T*)fields[CUP_U],
                      (const T*)fields[CUP_V], (const T*)fields[CUP_W], (const T*)fields[CUP_P],
                      (const T*)fields[CUP_CHI], g, nu, half_extent[0], half_extent[1], half_extent[2], part, nbw);
   hipError_t e = hipGetLastError();
@@ -1928,7 +1961,7 @@ extern "C" int cup_diagnostics_noalloc(const cup_grid_desc* d, const void* const
   if (d->device < 0 || d->device >= SCRATCH_MAX_DEVICES)
     return free_error(CUP_E_INVALID, "diagnostics_noalloc: device ordinal out of range");
   const long long nb = (long long)d->bpd[0] * d->bpd[1] * d->bpd[2];
-  const int nbw = diag_nbw_x(d->bpd[0]);
+  const int nbw = diag_nbw(d->bpd[0], nb);
   if (nb / nbw > CUP_NOALLOC_MAX_PARTS)
     return free_error(CUP_E_INVALID, "diagnostics_noalloc: the grid needs " + std::to_string(nb / nbw) +
                                          " partial sums, more than the static scratch holds (" +
