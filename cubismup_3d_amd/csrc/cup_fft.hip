@@ -309,6 +309,48 @@ struct Three {
   T* p[3];
 };
 
+// Reduce-scatter steps over lanes that differ in bit 5, 4 or 0: of the pair (a, b), the lanes
+// with the bit clear get a's sum over both, the others b's. The first two are one register swap
+// between halves or rows of 16 (no LDS traffic, unlike a general shuffle).
+__device__ __forceinline__ float scatter_step32(float a, float b)
+{
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float scatter_step16(float a, float b)
+{
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap_lane1(float v)  // the value of lane ^ 1
+{
+  return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0xB1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double join64(unsigned lo, unsigned hi) { return __hiloint2double((int)hi, (int)lo); }
+__device__ __forceinline__ double scatter_step32(double a, double b)
+{
+  const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return join64(l[0], h[0]) + join64(l[1], h[1]);
+}
+__device__ __forceinline__ double scatter_step16(double a, double b)
+{
+  const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return join64(l[0], h[0]) + join64(l[1], h[1]);
+}
+__device__ __forceinline__ double swap_lane1(double v)
+{
+  return join64(__builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xf, 0xf, true),
+                __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xf, 0xf, true));
+}
+template <typename T>
+__device__ __forceinline__ T scatter_step1(T a, T b, bool odd)
+{
+  const T keep = odd ? b : a, send = odd ? a : b;
+  return keep + swap_lane1(send);
+}
+
 // Real rows -> packed half spectrum. grid = (Ny/8, Nz).
 // FORCE (fused linear forcing): the same pass also forms, per grid row, the x-DFT at
 // kx = 0, 1, 2 of each advected velocity component and sum |u*|^2: 16 values per row
@@ -316,8 +358,11 @@ struct Three {
 // rowbuf[(z*Ny + y)*16 + slot]. The divergence already loads v on row y+1 and w on plane
 // z+1, so the workgroup of row (y, z) takes u of (y, z), v of (y+1, z) and w of (y, z+1);
 // every row of every component is summed by exactly one workgroup.
-// Each thread's cells lie in one row (t -> bx = t/64, iy, ix), so row sums are lane
-// shuffles over ix plus an LDS sum over the 4 waves.
+// Each thread's cells lie in one row; the 8 lanes of a row in a wave (bits 0, 4 and 5) reduce
+// their 16 sums by halving, each ending with two of them (14 exchanges in registers, where summing
+// every value over every lane took 48 shuffles through the LDS pipe: the pass
+// took 66 us at 256^3 FP32 and 24 at 128^3 FP64, now 61 and 19), and the 4
+// waves' sums meet in LDS.
 template <typename T, int N, int SRC, bool FORCE>
 __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, const T* __restrict__ src1,
                                                   const T* __restrict__ src2, Three<C2<T>> spec,
@@ -413,14 +458,15 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
   if (FORCE) {
     // rows: lanes with the same iy = (lane >> 1) & 7 differ in bits 0 (half) and 4-5 (bx)
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, iy = (lane >> 1) & 7;
+    const bool odd = lane & 1;
+    T a8[8], a4[4];
 #pragma unroll
-    for (int q = 0; q < 3 * NA + 1; ++q) {
-      T v = acc[q];
-      v += __shfl_xor(v, 1, 64);
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      if ((lane & 0x31) == 0) rowacc[wv][iy][q] = (double)v;
-    }
+    for (int q = 0; q < 8; ++q) a8[q] = scatter_step32(acc[q], acc[q + 8]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a4[q] = scatter_step16(a8[q], a8[q + 4]);
+    const int q0 = 8 * (lane >> 5) + 4 * ((lane >> 4) & 1) + 2 * (lane & 1);
+    rowacc[wv][iy][q0] = (double)scatter_step1(a4[0], a4[2], odd);
+    rowacc[wv][iy][q0 + 1] = (double)scatter_step1(a4[1], a4[3], odd);
   }
   __syncthreads();
   if (FORCE && threadIdx.x < XROWS * (3 * NA + 1)) {
