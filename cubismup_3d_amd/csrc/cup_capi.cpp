@@ -420,8 +420,7 @@ int cup_pressure_rhs(cup_ctx* ctx, double dt)
   if (!(dt > 0)) return set_error(c, CUP_E_INVALID, "pressure_rhs: dt must be > 0");
   if (int rc = launch_set_dt(c, dt)) return rc;
   if (c.decomposition == CUP_PLAIN) {
-    if (int rc = launch_fill(c, c.rbuf, c.ncell, 0.0)) return rc;  // PoissonSolver::reset
-    if (int rc = launch_rhs_plain(c)) return rc;
+    if (int rc = launch_rhs_plain(c)) return rc;  // every cell of rbuf, so no PoissonSolver::reset
     if (c.body.present)
       if (int rc = launch_rhs_obstacle(c, c.rbuf)) return rc;
   } else if (c.body.present) {
@@ -434,11 +433,7 @@ int cup_poisson_periodic(cup_ctx* ctx)
 {
   CUP_GUARD(ctx);
   if (!c.periodic()) return set_error(c, CUP_E_INVALID, "poisson_periodic: non-periodic boundaries take cup_poisson_mixed");
-  if (c.decomposition == CUP_PLAIN) {
-    if (int rc = launch_poisson_plain(c)) return rc;
-    return launch_copy(c, c.f[CUP_P], c.rbuf, c.ncell);  // PoissonSolver::_fftw2cub
-  }
-  return launch_poisson_fused(c);
+  return c.decomposition == CUP_PLAIN ? launch_poisson_plain(c) : launch_poisson_fused(c);
 }
 
 int cup_poisson_mixed(cup_ctx* ctx)

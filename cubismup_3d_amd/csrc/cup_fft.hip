@@ -940,27 +940,6 @@ __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>*
     for (int m = 0; m < 16; ++m) S[gi(j + NTH * m)] = v[m];
 }
 
-// Separate spectral division (the PLAIN decomposition's "FFTW solve" pass).
-template <typename T>
-__global__ void k_divide(C2<T>* __restrict__ S, int ncols, int Ny, int Nz, double norm, const double* __restrict__ cx,
-                         const double* __restrict__ cy, const double* __restrict__ cz)
-{
-  const size_t n = (size_t)ncols * Ny * Nz;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const int kx = (int)(i % ncols);
-    const int ky = (int)((i / ncols) % Ny);
-    const int kz = (int)(i / ((size_t)ncols * Ny));
-    const double D = cx[kx] + cy[ky] + cz[kz];
-    const double fac = norm / (2 * D - 6);
-    const bool zero = kx == 0 && (ky == 0 || 2 * ky == Ny) && (kz == 0 || 2 * kz == Nz);
-    C2<T> v = S[i];
-    v.x = (T)((double)v.x * fac);
-    v.y = (T)((double)v.y * fac);
-    if (zero) v = C2<T>{0, 0};
-    S[i] = v;
-  }
-}
-
 // ------------------------------------------------------------------ dispatch
 
 template <typename T, int N>
@@ -1195,6 +1174,7 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
   return check_hip(c, hipGetLastError(), "poisson_fused");
 }
 
+// The RHS stays in rbuf; the solution goes to p.
 template <typename T>
 static int poisson_plain_t(Ctx& c)
 {
@@ -1202,15 +1182,9 @@ static int poisson_plain_t(Ctx& c)
   const double norm = poisson_norm(c);
   dispatch_n<GoXFwdTo, T>(c.N[0], c, Three<const T>{(const T*)c.rbuf}, S, 1);
   dispatch_n<GoY, T>(c.N[1], c, S, 1, (int)ZM_FWD, norm);
-  dispatch_n<GoZ, T>(c.N[2], c, S, 1, (int)ZM_FWD, norm);
-  const size_t n = (size_t)(c.N[0] / 2) * c.N[1] * c.N[2];
-  size_t gsz = (n + NT - 1) / NT;
-  if (gsz > 65536) gsz = 65536;
-  hipLaunchKernelGGL((k_divide<T>), dim3((unsigned)gsz), dim3(NT), 0, c.stream, S.p[0], c.N[0] / 2, c.N[1], c.N[2], norm,
-                     (const double*)c.cos4[0], (const double*)c.cos4[1], (const double*)c.cos4[2]);
-  dispatch_n<GoZ, T>(c.N[2], c, S, 1, (int)ZM_INV, norm);
+  dispatch_n<GoZ, T>(c.N[2], c, S, 1, (int)ZM_POISSON, norm);
   dispatch_n<GoY, T>(c.N[1], c, S, 1, (int)ZM_INV, norm);
-  dispatch_n<GoXInv, T>(c.N[0], c, S, Three<T>{(T*)c.rbuf}, 1);
+  dispatch_n<GoXInv, T>(c.N[0], c, S, Three<T>{(T*)c.f[CUP_P]}, 1);
   return check_hip(c, hipGetLastError(), "poisson_plain");
 }
 

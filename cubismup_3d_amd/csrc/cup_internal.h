@@ -348,7 +348,6 @@ int launch_gradp_fused(Ctx& c, const double uinf[3], const int* skip_slot, bool 
 int launch_diagnostics(Ctx& c, double nu, int* nparts);  // partials[nparts][20]
 int launch_ic_taylor_green(Ctx& c, double uMax);
 int launch_fill(Ctx& c, void* ptr, size_t n, double value);
-int launch_copy(Ctx& c, void* dst, const void* src, size_t n);
 int launch_set_dt(Ctx& c, double dt);
 int launch_reduce(Ctx& c, int n, int width, unsigned maxmask, double* out_dev, const double* part = nullptr);
 int launch_count_nan(Ctx& c, long long out[4]);  // NaN cells of u, v, w, p (synchronizes)
@@ -368,7 +367,7 @@ int fft_setup(Ctx& c);
 // xface: the x inverse pass also writes p's x faces to c.xface (for launch_gradp_fused)
 int launch_poisson_fused(Ctx& c, bool force = false, double tke_target = 0, double inj_rate = 0,
                          bool xface = false);  // div(tmp) -> p
-int launch_poisson_plain(Ctx& c);   // rhs in rbuf -> solution in rbuf (separate divide pass)
+int launch_poisson_plain(Ctx& c);   // rhs in rbuf -> p
 // nf <= 3 fields to their spectra and back, one launch per pass (3 passes)
 int launch_fft_forward_fields(Ctx& c, const void* const* real_blocks, void* const* spec, int nf);
 int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_blocks, int nf);

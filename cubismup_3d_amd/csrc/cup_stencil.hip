@@ -983,13 +983,6 @@ __global__ void k_copy3(T* __restrict__ a, T* __restrict__ b, T* __restrict__ cc
 }
 
 template <typename T>
-__global__ void k_copy1(T* __restrict__ a, const T* __restrict__ sa, size_t n)
-{
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    a[i] = sa[i];
-}
-
-template <typename T>
 __global__ void k_fill(T* __restrict__ a, size_t n, T value)
 {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -1054,15 +1047,6 @@ int launch_copy_tmp_to_u(Ctx& c)
                        (double*)c.f[CUP_V], (double*)c.f[CUP_W], (const double*)c.f[CUP_TMPU],
                        (const double*)c.f[CUP_TMPV], (const double*)c.f[CUP_TMPW], c.ncell);
   return check_hip(c, hipGetLastError(), "k_copy3");
-}
-
-int launch_copy(Ctx& c, void* dst, const void* src, size_t n)
-{
-  if (c.precision == 4)
-    hipLaunchKernelGGL((k_copy1<float>), ew_grid(n), dim3(NT), 0, c.stream, (float*)dst, (const float*)src, n);
-  else
-    hipLaunchKernelGGL((k_copy1<double>), ew_grid(n), dim3(NT), 0, c.stream, (double*)dst, (const double*)src, n);
-  return check_hip(c, hipGetLastError(), "k_copy1");
 }
 
 int launch_fill(Ctx& c, void* ptr, size_t n, double value)

@@ -38,11 +38,11 @@ enum cup_field {
 };
 
 /* Decomposition of one step. PLAIN follows the reference's operator decomposition
- * kernel by kernel (AdvectionDiffusion.cpp:402-428 kernel + copy, PressureRHS.cpp:273-346
- * memset + kernel, PoissonSolverPeriodic.cpp:129-146 r2c / solve / c2r as separate passes,
- * PoissonSolver.cpp:116-130 copy, PressureProjection.cpp:107-129 gradient). FUSED keeps
- * the arithmetic but fuses passes (RHS into the first FFT pass, the spectral division
- * into the z pass, reductions into the gradient epilogue, dt kept on the device). */
+ * operator by operator, each leaving its fields complete (AdvectionDiffusion.cpp:402-428
+ * kernel + copy, PressureRHS.cpp:273-346 into the RHS buffer, PoissonSolverPeriodic.cpp:129-146
+ * from it to p, PressureProjection.cpp:107-129 gradient). FUSED keeps the arithmetic but
+ * fuses across operators (RHS into the first FFT pass, reductions into the gradient
+ * epilogue, no copy back, dt kept on the device). */
 enum cup_decomposition { CUP_PLAIN = 0, CUP_FUSED = 1 };
 
 /* Advection scheme. CENTRAL_EULER is the reference's (AdvectionDiffusion.cpp:106-145).
