@@ -72,8 +72,6 @@ static void release(Ctx& c)
   c.red_part = nullptr;
   if (c.low_part) hipFree(c.low_part);
   if (c.low_red) hipFree(c.low_red);
-  if (c.low_coef) hipFree(c.low_coef);
-  if (c.low_counter) hipFree(c.low_counter);
   if (c.low_dev) hipFree(c.low_dev);
   if (c.low_rows) hipFree(c.low_rows);
   if (c.adjf) hipFree(c.adjf);
@@ -83,11 +81,11 @@ static void release(Ctx& c)
   c.body_ft_n = 0;
   c.low_dev = nullptr;
   c.low_rows = nullptr;
-  c.low_part = nullptr; c.low_red = nullptr; c.low_counter = nullptr;
+  c.low_part = nullptr; c.low_red = nullptr;
   if (c.sc) hipFree(c.sc);
   if (c.sc_host) hipHostFree(c.sc_host);
   if (c.host_red) hipHostFree(c.host_red);
-  c.partials = nullptr; c.low_coef = nullptr; c.sc = nullptr; c.sc_host = nullptr;
+  c.partials = nullptr; c.sc = nullptr; c.sc_host = nullptr;
   c.host_red = nullptr;
   if (c.stream) hipStreamDestroy(c.stream);
   c.stream = nullptr;

@@ -568,6 +568,14 @@ struct ColTile {
 // next integer by at least 1/(2 Ns), more than the product's rounding.
 __device__ __forceinline__ int mod_ns(int j, int Ns, float rNs) { return j - Ns * (int)(((float)j + 0.5f) * rNs); }
 
+// The forcing's factor times h^2/dt, 0 where it does not force (called by whole waves).
+__device__ __forceinline__ double forcing_gg(const ForcingArgs& fa, const LowModes& lm)
+{
+  double tke, tke_low;
+  const double fac = forcing_factor(fa, lm.n, tke, tke_low);
+  return fac > 0 ? fac * fa.h * fa.h / fa.sc->dt : 0.0;
+}
+
 template <typename T, int N, int M>
 struct ColStages {
   using CT = ColTile<T, M>;
@@ -582,7 +590,8 @@ struct ColStages {
   double norm;
   const double *cx, *cy, *cz;
   const LowModes* lmp;  // null: no forcing
-  const double* coef;
+  ForcingArgs fa;
+  double gg;            // the forcing's factor times h^2/dt (0: none)
 
   __device__ __forceinline__ C2<T> load(int f, int e) const
   {
@@ -600,12 +609,12 @@ struct ColStages {
       for (int e = 0; e < lm.npos; ++e) {
         const int slot = lm.pos[e][0], kye = lm.pos[e][1], kz = lm.pos[e][2], mc = lm.pos[e][3];
         if (kye != ky || slot != f) continue;
-        const double* cm = coef + 8 * (mc >> 1);
-        const double ci = (mc & 1) ? -cm[1] : cm[1];
+        const C2<double> cm = forcing_rhs_mode(fa, lm, mc >> 1, gg);
+        const double ci = (mc & 1) ? -cm.y : cm.y;
 #pragma unroll
         for (int r = 0; r < R; ++r)
           if (kz == j + r * m) {
-            v[r].x = (T)((double)v[r].x + cm[0]);
+            v[r].x = (T)((double)v[r].x + cm.x);
             v[r].y = (T)((double)v[r].y + ci);
           }
       }
@@ -750,8 +759,8 @@ __global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(Three<C2<T>> S,
                                                                const double* __restrict__ cx,
                                                                const double* __restrict__ cy,
                                                                const double* __restrict__ cz,
-                                                               const LowModes* __restrict__ lmp,
-                                                               const double* __restrict__ coef, FftPlan pl)
+                                                               const LowModes* __restrict__ lmp, ForcingArgs fa,
+                                                               FftPlan pl)
 {
   using CS = ColStages<T, N, M>;
   C2<T>* buf = lds_tile<T, N * CS::TK>();
@@ -759,7 +768,7 @@ __global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(Three<C2<T>> S,
   const size_t base = (axis == 1 ? (size_t)o * Ny : (size_t)o) * ncols + kx0;
   const size_t stride = axis == 1 ? (size_t)ncols : (size_t)Ny * ncols;
   CS cs{S.p[blockIdx.z], buf, tw, base, stride, inv != 0, N > 0 ? N : pl.n, min(CS::TK, ncols - kx0), kx0, o, Ny, norm,
-        cx,  cy,  cz, lmp,  coef};
+        cx,  cy,  cz, lmp,  fa, POISSON && lmp && kx0 == 0 ? forcing_gg(fa, *lmp) : 0.0};
   if constexpr (N > 0) cs.template run_ct<POISSON>();
   else cs.template run_rt<POISSON>(pl);
 }
@@ -844,8 +853,7 @@ template <typename T, int N, int AXIS, int MODE, bool FORCE = false, int EXTRA =
 __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>* __restrict__ tw, int ncols,
                                                  int Ny, int Nz, double norm, const double* __restrict__ cx,
                                                  const double* __restrict__ cy, const double* __restrict__ cz,
-                                                 const LowModes* __restrict__ lmp, const double* __restrict__ coef,
-                                                 ColExtra ex)
+                                                 const LowModes* __restrict__ lmp, ForcingArgs fa, ColExtra ex)
 {
   using CR = ColReg<T, N>;
   constexpr int TK = CR::TK, NTH = CR::NTH, RPT = CR::RPT;
@@ -858,7 +866,7 @@ __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>*
       if (EXTRA == 1 && w < ex.nz * ex.parts)
         forcing_planes_wg<T>(ex.rowbuf, ex.plane, Ny, (const C2<T>*)ex.twy, w / ex.parts, w % ex.parts, ex.parts, buf);
       else if (EXTRA == 2 && w < ex.nz)
-        forcing_rows_wg<T>(lmp, coef, (const C2<T>*)ex.twy, (const C2<T>*)ex.twz, (T*)ex.rows, Ny, Nz, w, buf);
+        forcing_rows_step<T>(lmp, fa, (const C2<T>*)ex.twy, (const C2<T>*)ex.twz, (T*)ex.rows, Ny, Nz, w, buf);
       return;
     }
   }
@@ -884,21 +892,22 @@ __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>*
   }
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = live ? S[gi(j + NTH * m)] : C2<T>{0, 0};
+  const double gg = FORCE && kx0 == 0 ? forcing_gg(fa, *lmp) : 0.0;  // while the columns arrive
   fft_a_to_b<T, N, -1>(v, buf, tw, f, j);
   if (FORCE && kx0 == 0) {
-    // fused forcing: add the forcing's RHS modes (coefficients from k_forcing_reduce) to the
+    // fused forcing: add the forcing's RHS modes (from the mode sums of k_forcing_reduce) to the
     // entries this thread holds (column f, k = k1 + 16 k2 with k1 / RPT = j)
     const LowModes& lm = *lmp;
     for (int e = 0; e < lm.npos; ++e) {
       const int slot = lm.pos[e][0], ky = lm.pos[e][1], kz = lm.pos[e][2], mc = lm.pos[e][3];
       if (ky != other || slot != f || (kz & 15) / RPT != j) continue;
       const int r = ((kz & 15) % RPT) * NTH + (kz >> 4);
-      const double* cm = coef + 8 * (mc >> 1);
-      const double ci = (mc & 1) ? -cm[1] : cm[1];
+      const C2<double> cm = forcing_rhs_mode(fa, lm, mc >> 1, gg);
+      const double ci = (mc & 1) ? -cm.y : cm.y;
 #pragma unroll
       for (int q = 0; q < 16; ++q)
         if (q == r) {
-          v[q].x = (T)((double)v[q].x + cm[0]);
+          v[q].x = (T)((double)v[q].x + cm.x);
           v[q].y = (T)((double)v[q].y + ci);
         }
     }
@@ -994,6 +1003,7 @@ struct ColPass {
       const int other = AXIS == 1 ? c.N[2] : c.N[1];
       const int gx = (ncols + TK - 1) / TK;
       ColExtra ex{};
+      const ForcingArgs fa = c.forcing;
       if (extra) {
         ex = forcing_planes_extra(c);
         const int work = extra == 1 ? ex.nz * ex.parts : ex.nz;
@@ -1003,26 +1013,22 @@ struct ColPass {
       const C2<T>* tw = (const C2<T>*)c.tw[AXIS];
       if (mode == ZM_FWD && extra == 1)
         hipLaunchKernelGGL((k_fft_colr<T, N, AXIS, ZM_FWD, false, 1>), grid, dim3(NT), 0, c.stream, spec, tw, ncols,
-                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr,
-                           ex);
+                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, fa, ex);
       else if (mode == ZM_FWD)
         hipLaunchKernelGGL((k_fft_colr<T, N, AXIS, ZM_FWD>), grid, dim3(NT), 0, c.stream, spec, tw, ncols, c.N[1],
-                           c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr, ex);
+                           c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, fa, ex);
       else if (mode == ZM_INV)
         hipLaunchKernelGGL((k_fft_colr<T, N, AXIS, ZM_INV>), grid, dim3(NT), 0, c.stream, spec, tw, ncols, c.N[1],
-                           c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr, ex);
+                           c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, fa, ex);
       else if (AXIS == 2 && force && extra == 2)
         hipLaunchKernelGGL((k_fft_colr<T, N, 2, ZM_POISSON, true, 2>), grid, dim3(NT), 0, c.stream, spec, tw, ncols,
-                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev,
-                           (const double*)c.low_coef, ex);
+                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, fa, ex);
       else if (AXIS == 2 && force)
         hipLaunchKernelGGL((k_fft_colr<T, N, 2, ZM_POISSON, true>), grid, dim3(NT), 0, c.stream, spec, tw, ncols,
-                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev,
-                           (const double*)c.low_coef, ex);
+                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, fa, ex);
       else if (AXIS == 2)
         hipLaunchKernelGGL((k_fft_colr<T, N, 2, ZM_POISSON, false>), grid, dim3(NT), 0, c.stream, spec, tw, ncols,
-                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, (const double*)nullptr,
-                           ex);
+                           c.N[1], c.N[2], norm, c.cos4[0], c.cos4[1], c.cos4[2], c.low_dev, fa, ex);
     } else if constexpr (N >= 512) {
       launch<N, N>(c, spec, nf, mode, norm, force);
     } else {
@@ -1043,7 +1049,7 @@ struct ColPass {
       hipLaunchKernelGGL(kern, grid, bt, lds, c.stream, spec, (const C2<T>*)c.tw[AXIS], ncols, AXIS,
                          mode == ZM_INV ? 1 : 0, c.N[1], norm, (const double*)c.cos4[0], (const double*)c.cos4[1],
                          (const double*)c.cos4[2], (const LowModes*)(force ? c.low_dev : nullptr),
-                         (const double*)c.low_coef, c.plan[AXIS]);
+                         c.forcing, c.plan[AXIS]);
     };
     if (mode == ZM_POISSON) go(k_fft_col<T, NN, M, true>);
     else go(k_fft_col<T, NN, M, false>);
@@ -1135,6 +1141,7 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
 {
   const Three<C2<T>> S{(C2<T>*)c.spec};
   const double norm = poisson_norm(c);
+  if (force) c.forcing = forcing_args(c, tke_target, inj_rate);
   stage_mark(c, ST_XFWD, false);
   dispatch_n<GoXFwd, T>(c.N[0], c, (const T*)c.f[c.ustar], (const T*)c.f[c.ustar + 1],
                         (const T*)c.f[c.ustar + 2], (int)XSRC_DIV, force);
@@ -1146,7 +1153,7 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
   const bool extra = force && col_extra_ok(c.N[1]) && col_extra_ok(c.N[2]);
   if (force && !extra) {
     stage_mark(c, ST_FREDUCE, false);
-    if (int rc = launch_forcing_reduce(c, tke_target, inj_rate)) return rc;
+    if (int rc = launch_forcing_reduce(c)) return rc;
     if (int rc = launch_forcing_rows(c)) return rc;
     stage_mark(c, ST_FREDUCE, true);
   }
@@ -1156,7 +1163,7 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
   stage_mark(c, ST_YFWD, true);
   if (extra) {
     stage_mark(c, ST_FREDUCE, false);
-    if (int rc = launch_forcing_reduce(c, tke_target, inj_rate, false)) return rc;
+    if (int rc = launch_forcing_reduce(c, false)) return rc;
     stage_mark(c, ST_FREDUCE, true);
   }
   stage_mark(c, ST_ZPASS, false);

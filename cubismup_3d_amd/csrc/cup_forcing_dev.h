@@ -11,6 +11,33 @@
 
 namespace cup {
 
+// SpectralForcing's injection and factor (SpectralForcing.cpp:37-77) from tke = <|u*|^2>/2 (Parseval)
+// and tke_low = sum over the n low modes, in every lane of a wave (all 64 lanes call it).
+__device__ __forceinline__ double forcing_factor(const ForcingArgs& f, int n, double& tke, double& tke_low)
+{
+  const int lane = threadIdx.x & 63;
+  double e = 0;
+  for (int o = lane; o < 3 * n; o += 64) e += f.red[2 * o] * f.red[2 * o] + f.red[2 * o + 1] * f.red[2 * o + 1];
+  e = wave_sum(e);
+  const double dt = f.sc->dt;
+  tke = 0.5 * f.red[6 * n] / f.norm;
+  tke_low = e / (f.norm * f.norm);
+  double inj = 0;
+  if (f.tke_target > 0) inj = (f.tke_target - tke) / dt;
+  else if (f.inj_rate > 0) inj = f.inj_rate;
+  return dt * inj / (2 * tke_low);
+}
+
+// The forcing's pressure-RHS mode (fac h^2/dt) i sum_d sin(2 pi k_d/N_d) u_d(k) of mode m, for
+// gg = fac h^2/dt.
+__device__ __forceinline__ C2<double> forcing_rhs_mode(const ForcingArgs& f, const LowModes& lm, int m, double gg)
+{
+  const double* r = f.red + 6 * m;
+  const double s0 = lm.sk[m][0], s1 = lm.sk[m][1], s2 = lm.sk[m][2];
+  const double dr = s0 * r[0] + s1 * r[2] + s2 * r[4], di = s0 * r[1] + s1 * r[3] + s2 * r[5];
+  return C2<double>{-gg * di, gg * dr};  // i (dr + i di)
+}
+
 // The extra workgroups of a column pass: the first ey rows of its grid (every x index) are
 // workgroups of the plane stage (kind 1, nz * parts of them, the rest idle) or of the row stage
 // (kind 2, nz of them); the column transforms take the rows after them.
@@ -22,6 +49,9 @@ struct ColExtra {
   void* rows;            // row stage: output (context precision)
   int parts, nz, ey;
 };
+
+// Plane partials per z plane at most (forcing_plane_parts).
+constexpr int FR_PARTS_MAX = 4;
 
 // LDS bytes the two stages need (carved from the column pass's tile).
 constexpr int FORCING_PLANES_LDS = 16 * 16 * 5 * 8;
@@ -67,7 +97,7 @@ __device__ __forceinline__ void forcing_planes_wg(const double* __restrict__ row
 // Fused forcing, stage 4: for every grid row (y, z) the coefficients of the velocity modes'
 // synthesis along x, fac*u_low(x) = R0 + 2 Re(R1 e^{2 pi i x/Nx}) + 2 Re(R2 e^{4 pi i x/Nx})
 // per component (5 values x 3 = 15, padded to 16), so the gradient pass evaluates the forcing
-// with a handful of FMAs per cell. Mode m (velocity coefficient c, component by component)
+// with a handful of FMAs per cell. Mode m (velocity coefficient c = scale times its mode sums red)
 // contributes c e^{2 pi i (ky y/Ny + kz z/Nz)} to the entries of |kx|: 2 Re at kx = 0, Re and
 // (sign kx) Im at |kx| = 1, 2. Taking a mode with kx < 0 as its conjugate (conj c, -ky, -kz; the
 // real parts are unchanged), the row value is a sum over ky of A_ky(z) e^{2 pi i ky y/Ny} with
@@ -76,7 +106,7 @@ __device__ __forceinline__ void forcing_planes_wg(const double* __restrict__ row
 // entries of one row from two y twiddles. All in FP64; the phases are conjugates of the twiddles
 // e^{-2 pi i t/N}. lds: FORCING_ROWS_LDS bytes.
 template <typename T>
-__device__ __forceinline__ void forcing_rows_wg(const LowModes* __restrict__ lmp, const double* __restrict__ coef,
+__device__ __forceinline__ void forcing_rows_wg(const LowModes* __restrict__ lmp, const double* __restrict__ red, double scale,
                                                 const C2<T>* __restrict__ twy, const C2<T>* __restrict__ twz,
                                                 T* __restrict__ rows, int Ny, int Nz, int z, void* lds)
 {
@@ -95,7 +125,7 @@ __device__ __forceinline__ void forcing_rows_wg(const LowModes* __restrict__ lmp
     const double ec = (double)e.x, es = -(double)e.y;  // e^{+2 pi i kz z/Nz}
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      const double cr = coef[8 * t + 2 + 2 * q], ci = sg * coef[8 * t + 3 + 2 * q];
+      const double cr = scale * red[6 * t + 2 * q], ci = sg * scale * red[6 * t + 2 * q + 1];
       B[t][q][0] = cr * ec - ci * es;
       B[t][q][1] = cr * es + ci * ec;
     }
@@ -139,6 +169,22 @@ __device__ __forceinline__ void forcing_rows_wg(const LowModes* __restrict__ lmp
     }
     o[15] = (T)0;
   }
+}
+
+// The row stage in the fused step: the scale from the factor; plane 0 records the statistics.
+template <typename T>
+__device__ __forceinline__ void forcing_rows_step(const LowModes* __restrict__ lmp, const ForcingArgs& f,
+                                                  const C2<T>* __restrict__ twy, const C2<T>* __restrict__ twz,
+                                                  T* __restrict__ rows, int Ny, int Nz, int z, void* lds)
+{
+  double tke, tke_low;
+  const double fac = forcing_factor(f, lmp->n, tke, tke_low);
+  if (z == 0 && threadIdx.x == 0) {
+    f.sc->tke = tke;
+    f.sc->tke_low = tke_low;
+    f.sc->forcing_fac = fac;
+  }
+  forcing_rows_wg<T>(lmp, f.red, fac > 0 ? fac / f.norm : 0.0, twy, twz, rows, Ny, Nz, z, lds);
 }
 
 }  // namespace cup

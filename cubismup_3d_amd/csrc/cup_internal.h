@@ -106,6 +106,18 @@ struct LowModes {
   double sk[LOW_MAX][3];    // sin(2 pi k_d / N_d): the central-difference symbol of each mode
 };
 
+// What the consumers of the forcing's mode sums need to form the forcing for themselves. The
+// factor is a sum over at most 97 values: each wave that needs it forms it (forcing_factor), which
+// takes the place of a last-workgroup tail in the mode stage, whose device-scope fence wrote the
+// L2s back: the stage went from 6.8 to 4.4 us at 128^3 FP64 with 1 us more in the z pass (from 10
+// to 6 with 2.6 more at 256^3 FP32).
+struct ForcingArgs {
+  const double* red;  // the mode sums: re, im of u, v, w per mode, then sum |u*|^2
+  DevScalars* sc;     // dt; the row stage records tke, tke_low and the factor
+  double tke_target, inj_rate, h;
+  double norm;        // cells
+};
+
 // Geometry passed by value to kernels.
 struct GridArgs {
   int nbx, nby, nbz;  // blocks per dimension
@@ -195,8 +207,7 @@ struct Ctx {
   LowModes* low_dev = nullptr;  // device copy (kernels index it per lane)
   double* low_part = nullptr;  // x-pass row values [Nz][Ny][16]: per component the row's x-DFT at kx 0..2, |u|^2
   double* low_red = nullptr;   // plane DFTs in y [Nz][16][5], then the W mode sums (6 per mode: re/im of u,v,w; |u|^2)
-  double* low_coef = nullptr;  // per mode: RHS addition (re,im), synthesis of u,v,w (re,im) x3
-  unsigned* low_counter = nullptr;
+  ForcingArgs forcing{};       // of the fused step being launched
   void* low_rows = nullptr;    // per grid row (y, z): 16 synthesis coefficients (context precision)
   double* body_ft = nullptr;   // device: 6 per body, each body's last penalization force/torque in the loop
   int body_ft_n = 0;
@@ -382,7 +393,8 @@ int launch_ic_hit(Ctx& c, double k0, const double* K, const double* E, int tn, d
 int forcing_plain(Ctx& c, double dt, double sim_dt, double nu, double tke_target, double inj,
                   double stats[5], int field = -1);
 // planes = false: the plane stage ran beside the y pass (forcing_planes_extra)
-int launch_forcing_reduce(Ctx& c, double tke_target, double inj_rate, bool planes = true);
+int launch_forcing_reduce(Ctx& c, bool planes = true);
+ForcingArgs forcing_args(const Ctx& c, double tke_target, double inj_rate);
 struct ColExtra;
 ColExtra forcing_planes_extra(Ctx& c);  // the plane and row stages' buffers, for the column passes
 int launch_forcing_rows(Ctx& c);

@@ -11,7 +11,6 @@ namespace cup {
 
 // The forcing's plane stage splits each z plane into up to FR_PARTS_MAX equal row ranges of
 // at least 64 rows, one workgroup each.
-constexpr int FR_PARTS_MAX = 4;
 inline int forcing_plane_parts(int ny)
 {
   int p = ny / 64;
@@ -508,14 +507,10 @@ int spectral_setup(Ctx& c)
   if (check_hip(c, hipMalloc(&c.low_part, nrow * 16 * sizeof(double)), "hipMalloc low row values") ||
       check_hip(c, hipMalloc(&c.low_red, ((size_t)c.N[2] * FR_PARTS_MAX * 16 * 5 + W) * sizeof(double)),
                 "hipMalloc low red") ||
-      check_hip(c, hipMalloc(&c.low_coef, (size_t)c.nlow * 8 * sizeof(double)), "hipMalloc low coef") ||
-      check_hip(c, hipMalloc(&c.low_counter, sizeof(unsigned)), "hipMalloc counter") ||
       check_hip(c, hipMalloc(&c.low_dev, sizeof(LowModes)), "hipMalloc low modes") ||
       check_hip(c, hipMalloc(&c.low_rows, (size_t)c.N[1] * c.N[2] * 16 * c.esz), "hipMalloc low rows"))
     return CUP_E_NOMEM;
   hipMemcpy(c.low_dev, &c.low, sizeof(LowModes), hipMemcpyHostToDevice);
-  hipMemsetAsync(c.low_counter, 0, sizeof(unsigned), c.stream);
-  hipMemsetAsync(c.low_coef, 0, (size_t)c.nlow * 8 * sizeof(double), c.stream);
   return CUP_OK;
 }
 
@@ -534,51 +529,54 @@ __global__ __launch_bounds__(NT) void k_forcing_planes(const double* __restrict_
 // plane value is U(z) = Pr + i sg Pi, with Pr, Pi the plane DFTs (at ky, conjugated for
 // ky < 0) of the slots holding re and im of the x-DFT at |kx| (sg = -1 for kx < 0, the
 // conjugate; Pi = 0 at kx = 0); the owner sums U(z) e^{-i kz z} over z, threads over planes
-// and a fixed shuffle tree (deterministic), into red[6m + 2q + {re, im}] (red[W-1] for
-// |u*|^2). The last workgroup to finish computes, on the device, SpectralForcing's injection
-// and factor (SpectralForcing.cpp:37-77) from tke = <|u*|^2>/2 (Parseval) and tke_low = sum
-// over the low modes, and the coefficient tables: the forcing's pressure-RHS modes
-// fac*(h^2/dt)*i*sum_d sin(2 pi k_d/N_d) u_d(k) (added in the z pass) and the velocity modes
-// fac/N^3 u(k) (added in the gradient pass).
+// and a fixed shuffle tree (deterministic), into red[6m + 2q + {re, im}] (red[6n] for |u*|^2). The z
+// pass and the row stage form the factor and their coefficients from these sums (ForcingArgs).
 template <typename T>
-__global__ __launch_bounds__(NT) void k_forcing_reduce(const double* __restrict__ plane, int W,
-                                                       double* __restrict__ red, unsigned* __restrict__ counter,
-                                                       const LowModes* __restrict__ lmp, DevScalars* __restrict__ sc,
-                                                       double* __restrict__ coef, double tke_target, double inj_rate,
-                                                       double h, double ncell, int N0, int N1, int N2,
+__global__ __launch_bounds__(NT) void k_forcing_reduce(const double* __restrict__ plane, double* __restrict__ red,
+                                                       const LowModes* __restrict__ lmp, int N2,
                                                        const C2<T>* __restrict__ twz, int parts)
 {
   __shared__ double wsum[NT / 64][2];
-  __shared__ double fin[6 * LOW_MAX + 1];
-  __shared__ double facs[1];
-  __shared__ bool last;
   const LowModes& lm = *lmp;
   const int t = threadIdx.x, o = blockIdx.x, nq = 3 * lm.n;
   double ar = 0, ai = 0;
-  // plane partials zp = z*parts + part
-  const int nzp = N2 * parts;
+  // the plane partials of z: plane[((z*parts + part)*16 + slot)*5 + k], all loads of a z in flight
   if (o == nq) {
-    for (int zp = t; zp < nzp; zp += NT) ar += plane[((size_t)zp * 16 + 15) * 5];
+    for (int z = t; z < N2; z += NT) {
+      double v[FR_PARTS_MAX];
+#pragma unroll
+      for (int p = 0; p < FR_PARTS_MAX; ++p) v[p] = p < parts ? plane[(((size_t)z * parts + p) * 16 + 15) * 5] : 0.0;
+#pragma unroll
+      for (int p = 0; p < FR_PARTS_MAX; ++p) ar += v[p];
+    }
   } else {
     const int m = o / 3, q = o % 3;
     const int kx = lm.k[m][0], ky = lm.k[m][1], kz = lm.k[m][2];
     const int ak = kx < 0 ? -kx : kx, aky = ky < 0 ? -ky : ky;
     const int sre = ak == 0 ? 5 * q : 5 * q + 2 * ak - 1;
     const double sg = kx < 0 ? -1.0 : 1.0, cy = ky < 0 ? -1.0 : 1.0;
-    for (int zp = t; zp < nzp; zp += NT) {
-      const int z = zp / parts;
-      const double* P = plane + (size_t)zp * 16 * 5;
-      // plane DFT of slot s at ky: (P[s][0], 0) for ky = 0, else (P[s][2|ky|-1], cy P[s][2|ky|])
-      const double rr = aky == 0 ? P[sre * 5] : P[sre * 5 + 2 * aky - 1];
-      const double ri = aky == 0 ? 0.0 : cy * P[sre * 5 + 2 * aky];
-      double ir = 0, ii = 0;
-      if (ak != 0) {
-        ir = aky == 0 ? P[(sre + 1) * 5] : P[(sre + 1) * 5 + 2 * aky - 1];
-        ii = aky == 0 ? 0.0 : cy * P[(sre + 1) * 5 + 2 * aky];
+    const int kzm = (kz % N2 + N2) % N2;
+    // plane DFT of slot s at ky: (P[s][0], 0) for ky = 0, else (P[s][2|ky|-1], cy P[s][2|ky|])
+    const int kre = aky == 0 ? 0 : 2 * aky - 1, kim = 2 * aky;
+    for (int z = t; z < N2; z += NT) {
+      double v[FR_PARTS_MAX][4];
+#pragma unroll
+      for (int p = 0; p < FR_PARTS_MAX; ++p) {
+        const double* P = plane + (((size_t)z * parts + p) * 16 + sre) * 5;
+        const bool on = p < parts;
+        v[p][0] = on ? P[kre] : 0.0;
+        v[p][1] = on && aky ? P[kim] : 0.0;
+        v[p][2] = on && ak ? P[5 + kre] : 0.0;
+        v[p][3] = on && ak && aky ? P[5 + kim] : 0.0;
       }
-      // U = (rr + i ri) + i sg (ir + i ii)
-      const double Ur = rr - sg * ii, Ui = ri + sg * ir;
-      const C2<T> e = twz[((kz * z) % N2 + N2) % N2];
+      double f[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int p = 0; p < FR_PARTS_MAX; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f[k] += v[p][k];
+      // U = (re + i im) of the real slot + i sg (the imaginary slot)
+      const double Ur = f[0] - sg * cy * f[3], Ui = cy * f[1] + sg * f[2];
+      const C2<T> e = twz[(kzm * z) % N2];
       const double er = (double)e.x, ei = (double)e.y;
       ar += Ur * er - Ui * ei;
       ai += Ur * ei + Ui * er;
@@ -598,59 +596,11 @@ __global__ __launch_bounds__(NT) void k_forcing_reduce(const double* __restrict_
       si += wsum[w][1];
     }
     if (o == nq) {
-      red[W - 1] = sr;
+      red[2 * nq] = sr;
     } else {
       red[2 * o] = sr;  // column 6m + 2q = 2o
       red[2 * o + 1] = si;
     }
-    __threadfence();
-    last = atomicAdd(counter, 1u) == (unsigned)(gridDim.x - 1);
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();  // acquire: the other workgroups' sums are visible to plain loads
-  if (t < W) fin[t] = red[t];
-  __syncthreads();
-  const double* r = fin;
-  const double dt = sc->dt;
-  const double norm = (double)N0 * N1 * N2;
-  if (t < 64) {
-    // sum over the low modes' 3n columns of |c|^2, lanes over columns and a fixed shuffle tree
-    double e = 0;
-    for (int o2 = t; o2 < nq; o2 += 64) e += r[2 * o2] * r[2 * o2] + r[2 * o2 + 1] * r[2 * o2 + 1];
-    e = wave_sum(e);
-    if (t == 0) {
-      *counter = 0u;
-      const double tke = 0.5 * r[W - 1] / ncell;
-      const double tke_low = e / (norm * norm);
-      double inj = 0;
-      if (tke_target > 0) inj = (tke_target - tke) / dt;
-      else if (inj_rate > 0) inj = inj_rate;
-      const double fac = dt * inj / (2 * tke_low);
-      sc->tke = tke;
-      sc->tke_low = tke_low;
-      sc->forcing_fac = fac;
-      facs[0] = fac;
-    }
-  }
-  __syncthreads();
-  const double fac = facs[0];
-  if (t >= lm.n) return;
-  const int m = t;  // one thread per mode
-  double* cm = coef + 8 * m;
-  if (!(fac > 0)) {
-    for (int q = 0; q < 8; ++q) cm[q] = 0;
-    return;
-  }
-  const double s0 = lm.sk[m][0], s1 = lm.sk[m][1], s2 = lm.sk[m][2];
-  const double dr = s0 * r[6 * m] + s1 * r[6 * m + 2] + s2 * r[6 * m + 4];
-  const double di = s0 * r[6 * m + 1] + s1 * r[6 * m + 3] + s2 * r[6 * m + 5];
-  const double gg = fac * h * h / dt;
-  cm[0] = -gg * di;  // i * (dr + i di) = -di + i dr
-  cm[1] = gg * dr;
-  for (int q = 0; q < 3; ++q) {
-    cm[2 + 2 * q] = fac / norm * r[6 * m + 2 * q];
-    cm[3 + 2 * q] = fac / norm * r[6 * m + 2 * q + 1];
   }
 }
 
@@ -667,54 +617,51 @@ ColExtra forcing_planes_extra(Ctx& c)
   return e;
 }
 
-int launch_forcing_reduce(Ctx& c, double tke_target, double inj_rate, bool planes)
+// The mode sums, behind the plane partials [Nz][parts][16][5].
+static double* forcing_red(const Ctx& c) { return c.low_red + (size_t)c.N[2] * FR_PARTS_MAX * 16 * 5; }
+
+ForcingArgs forcing_args(const Ctx& c, double tke_target, double inj_rate)
 {
-  const int W = 6 * c.nlow + 1;
-  const int nz = c.N[2];
-  const int parts = forcing_plane_parts(c.N[1]);
-  double* plane = c.low_red;  // [Nz][parts][16][5] plane DFTs, then the W column sums
-  double* red = plane + (size_t)nz * FR_PARTS_MAX * 16 * 5;
-  if (c.precision == 4) {
-    if (planes)
-      hipLaunchKernelGGL((k_forcing_planes<float>), dim3(nz, parts), dim3(NT), 0, c.stream,
-                         (const double*)c.low_part, plane, c.N[1], (const C2<float>*)c.tw[1]);
-    hipLaunchKernelGGL((k_forcing_reduce<float>), dim3(3 * c.nlow + 1), dim3(NT), 0, c.stream, (const double*)plane, W,
-                       red, c.low_counter, c.low_dev, c.sc, c.low_coef, tke_target, inj_rate, c.h, (double)c.ncell,
-                       c.N[0], c.N[1], c.N[2], (const C2<float>*)c.tw[2], parts);
-  } else {
-    if (planes)
-      hipLaunchKernelGGL((k_forcing_planes<double>), dim3(nz, parts), dim3(NT), 0, c.stream,
-                         (const double*)c.low_part, plane, c.N[1], (const C2<double>*)c.tw[1]);
-    hipLaunchKernelGGL((k_forcing_reduce<double>), dim3(3 * c.nlow + 1), dim3(NT), 0, c.stream, (const double*)plane,
-                       W, red, c.low_counter, c.low_dev, c.sc, c.low_coef, tke_target, inj_rate, c.h,
-                       (double)c.ncell, c.N[0], c.N[1], c.N[2], (const C2<double>*)c.tw[2], parts);
-  }
+  return ForcingArgs{forcing_red(c), c.sc, tke_target, inj_rate, c.h, (double)c.ncell};
+}
+
+template <typename T>
+static int forcing_reduce_t(Ctx& c, bool planes)
+{
+  const int nz = c.N[2], parts = forcing_plane_parts(c.N[1]);
+  if (planes)
+    hipLaunchKernelGGL((k_forcing_planes<T>), dim3(nz, parts), dim3(NT), 0, c.stream, (const double*)c.low_part,
+                       c.low_red, c.N[1], (const C2<T>*)c.tw[1]);
+  hipLaunchKernelGGL((k_forcing_reduce<T>), dim3(3 * c.nlow + 1), dim3(NT), 0, c.stream, (const double*)c.low_red,
+                     forcing_red(c), c.low_dev, nz, (const C2<T>*)c.tw[2], parts);
   return check_hip(c, hipGetLastError(), "k_forcing_reduce");
+}
+
+int launch_forcing_reduce(Ctx& c, bool planes)
+{
+  return c.precision == 4 ? forcing_reduce_t<float>(c, planes) : forcing_reduce_t<double>(c, planes);
 }
 
 // Fused forcing, stage 4 (the per-row synthesis coefficients, forcing_rows_wg) as a kernel of
 // its own: one workgroup per z plane.
 template <typename T>
-__global__ __launch_bounds__(NT) void k_forcing_rows(const LowModes* __restrict__ lmp,
-                                                     const double* __restrict__ coef, const C2<T>* __restrict__ twy,
-                                                     const C2<T>* __restrict__ twz, T* __restrict__ rows, int Ny,
-                                                     int Nz)
+__global__ __launch_bounds__(NT) void k_forcing_rows(const LowModes* __restrict__ lmp, ForcingArgs fa,
+                                                     const C2<T>* __restrict__ twy, const C2<T>* __restrict__ twz,
+                                                     T* __restrict__ rows, int Ny, int Nz)
 {
   __shared__ double lds[(FORCING_ROWS_LDS + 7) / 8];
-  forcing_rows_wg<T>(lmp, coef, twy, twz, rows, Ny, Nz, blockIdx.x, lds);
+  forcing_rows_step<T>(lmp, fa, twy, twz, rows, Ny, Nz, blockIdx.x, lds);
 }
 
 int launch_forcing_rows(Ctx& c)
 {
   const dim3 grid(c.N[2]);
   if (c.precision == 4)
-    hipLaunchKernelGGL((k_forcing_rows<float>), grid, dim3(NT), 0, c.stream, (const LowModes*)c.low_dev,
-                       (const double*)c.low_coef, (const C2<float>*)c.tw[1], (const C2<float>*)c.tw[2],
-                       (float*)c.low_rows, c.N[1], c.N[2]);
+    hipLaunchKernelGGL((k_forcing_rows<float>), grid, dim3(NT), 0, c.stream, (const LowModes*)c.low_dev, c.forcing,
+                       (const C2<float>*)c.tw[1], (const C2<float>*)c.tw[2], (float*)c.low_rows, c.N[1], c.N[2]);
   else
-    hipLaunchKernelGGL((k_forcing_rows<double>), grid, dim3(NT), 0, c.stream, (const LowModes*)c.low_dev,
-                       (const double*)c.low_coef, (const C2<double>*)c.tw[1], (const C2<double>*)c.tw[2],
-                       (double*)c.low_rows, c.N[1], c.N[2]);
+    hipLaunchKernelGGL((k_forcing_rows<double>), grid, dim3(NT), 0, c.stream, (const LowModes*)c.low_dev, c.forcing,
+                       (const C2<double>*)c.tw[1], (const C2<double>*)c.tw[2], (double*)c.low_rows, c.N[1], c.N[2]);
   return check_hip(c, hipGetLastError(), "k_forcing_rows");
 }
 
