@@ -398,6 +398,7 @@ ForcingArgs forcing_args(const Ctx& c, double tke_target, double inj_rate);
 struct ColExtra;
 ColExtra forcing_planes_extra(Ctx& c);  // the plane and row stages' buffers, for the column passes
 int launch_forcing_rows(Ctx& c);
+int launch_add_rows(Ctx& c, int field0);  // fields += the row coefficients' synthesis along x
 // adjoint fields += the forcing's transpose at u* (fields us0..us0+2); synchronous
 int launch_adjoint_forcing(Ctx& c, int us0, double dt, double tke_target, double inj_rate);
 // cup_obstacle.hip

@@ -19,6 +19,9 @@ inline int forcing_plane_parts(int ny)
   return p;
 }
 
+// The mode sums, behind the plane partials [Nz][parts][16][5].
+static double* forcing_red(const Ctx& c) { return c.low_red + (size_t)c.N[2] * FR_PARTS_MAX * 16 * 5; }
+
 __device__ __forceinline__ int signed_k(int i, int n) { return i <= n / 2 ? i : i - n; }
 
 // Philox-4x32-10 (Salmon, Moraes, Dror, Shaw: "Parallel random numbers: as easy as
@@ -303,6 +306,104 @@ __global__ void k_axpy_blocks(T* __restrict__ y, const T* __restrict__ x, size_t
     y[i] = (T)((double)y[i] + a * (double)x[i]);
 }
 
+// k_forcing_filter's four sums without its filtering, for the boxes whose band the row synthesis
+// takes (low_fused_ok): waves over (ky, kz) lines with lanes along kx, so the spectra are read in
+// whole cache lines and a line's sines are formed once (the filter forms three per mode and writes
+// all three spectra back: 35 us at 128^3 FP64, this takes 13). part[4*wave + {0..3}] as k_forcing_filter.
+constexpr int STAT_LPW_MAX = 64;  // lines per wave: one per lane
+
+template <typename T>
+__global__ __launch_bounds__(NT) void k_forcing_stats(const C2<T>* __restrict__ su, const C2<T>* __restrict__ sv,
+                                                      const C2<T>* __restrict__ sw, int N0, int N1, int N2, double wfx,
+                                                      double wfy, double wfz, int lpw, int nwaves,
+                                                      double* __restrict__ part)
+{
+  const int lane = threadIdx.x & 63, W = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  const int nlines = N1 * N2, ncols = N0 / 2, l0 = W * lpw, nl = min(lpw, nlines - l0);
+  const C2<T>* S[3] = {su, sv, sw};
+  // lane i: line l0 + i
+  const int ml = min(l0 + lane, nlines - 1), mly = ml % N1, mlz = ml / N1;
+  const int mjj = signed_k(mly, N1), mkk = signed_k(mlz, N2);
+  const double mdY = 2 * sin(2 * M_PI / N1 * mjj), mdZ = 2 * sin(2 * M_PI / N2 * mkk);
+  double acc[4] = {0, 0, 0, 0};
+  auto add = [&](const C2<double> (&U)[3], double wgt, int ii, int jj, int kk, double dX, double dY, double dZ) {
+    const double kx = ii * wfx, ky = jj * wfy, kz = kk * wfz;
+    const double k2 = kx * kx + ky * ky + kz * kz;
+    const double OXr = -U[2].y * dY + U[1].y * dZ, OXi = U[2].x * dY - U[1].x * dZ;
+    const double OYr = -U[0].y * dZ + U[2].y * dX, OYi = U[0].x * dZ - U[2].x * dX;
+    const double OZr = -U[1].y * dX + U[0].y * dY, OZi = U[1].x * dX - U[0].x * dY;
+    const double E = 0.5 * (U[0].x * U[0].x + U[0].y * U[0].y + U[1].x * U[1].x + U[1].y * U[1].y +
+                            U[2].x * U[2].x + U[2].y * U[2].y);
+    acc[0] += wgt * E;
+    acc[1] += wgt * 0.5 * (OXr * OXr + OXi * OXi + OYr * OYr + OYi * OYi + OZr * OZr + OZi * OZi);
+    if (k2 > 0 && k2 <= 4) acc[2] += wgt * E;
+    acc[3] += k2 > 0 ? wgt * E / sqrt(k2) : 0.0;
+  };
+  for (int m0 = 0; m0 < ncols; m0 += 64) {
+    const int m = m0 + lane;
+    const double dX = 2 * sin(2 * M_PI / N0 * m);
+    for (int i = 0; i < nl; ++i) {
+      const int jj = __shfl(mjj, i, 64), kk = __shfl(mkk, i, 64);
+      const double dY = __shfl(mdY, i, 64), dZ = __shfl(mdZ, i, 64);
+      if (m == 0 || m >= ncols) continue;
+      C2<double> U[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) U[q] = ld(S[q], (size_t)(l0 + i) * ncols + m);
+      add(U, 2.0, m, jj, kk, dX, dY, dZ);
+    }
+  }
+  // slot 0 of line l0 + lane: the kx = 0 and kx = Nx/2 modes
+  if (lane < nl) {
+    const size_t id = (size_t)ml * ncols, mid = ((size_t)((N2 - mlz) % N2) * N1 + (N1 - mly) % N1) * ncols;
+    C2<double> A[3], B[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const C2<double> Z = ld(S[q], id), Zm = ld(S[q], mid);
+      A[q] = C2<double>{0.5 * (Z.x + Zm.x), 0.5 * (Z.y - Zm.y)};
+      B[q] = C2<double>{0.5 * (Z.y + Zm.y), 0.5 * (Zm.x - Z.x)};
+    }
+    add(A, 1.0, 0, mjj, mkk, 0.0, mdY, mdZ);
+    add(B, 1.0, N0 / 2, mjj, mkk, 2 * sin(2 * M_PI / N0 * (N0 / 2)), mdY, mdZ);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = wave_sum(acc[i]);
+  if (lane == 0 && W < nwaves)
+    for (int i = 0; i < 4; ++i) part[4 * (size_t)W + i] = acc[i];
+}
+
+// The band's modes out of the spectra, as k_forcing_reduce leaves its sums: red[6m + 2q + {re, im}].
+template <typename T>
+__global__ void k_low_modes(const C2<T>* __restrict__ su, const C2<T>* __restrict__ sv, const C2<T>* __restrict__ sw,
+                            const LowModes* __restrict__ lmp, double* __restrict__ red, int N0, int N1, int N2)
+{
+  const LowModes& lm = *lmp;
+  const int m = threadIdx.x / 3, q = threadIdx.x % 3;
+  if (m >= lm.n) return;
+  const C2<T>* S = q == 0 ? su : (q == 1 ? sv : sw);
+  const int kx = lm.k[m][0], sg = kx < 0 ? -1 : 1, ncols = N0 / 2;
+  const int ky = sg * lm.k[m][1], kz = sg * lm.k[m][2];  // kx < 0: the conjugate partner
+  auto at = [&](int y, int z) { return ld(S, ((size_t)((z % N2 + N2) % N2) * N1 + (y % N1 + N1) % N1) * ncols + sg * kx); };
+  C2<double> v = at(ky, kz);
+  if (kx == 0) {  // slot 0 holds A + iB: A = (Z + conj Zm)/2
+    const C2<double> Zm = at(-ky, -kz);
+    v = C2<double>{0.5 * (v.x + Zm.x), 0.5 * (v.y - Zm.y)};
+  }
+  red[6 * m + 2 * q] = v.x;
+  red[6 * m + 2 * q + 1] = sg * v.y;
+}
+
+// The row stage for a given scale of the mode sums.
+template <typename T>
+__global__ __launch_bounds__(NT) void k_forcing_rows_scaled(const LowModes* __restrict__ lmp,
+                                                            const double* __restrict__ red, double scale,
+                                                            const C2<T>* __restrict__ twy,
+                                                            const C2<T>* __restrict__ twz, T* __restrict__ rows,
+                                                            int Ny, int Nz)
+{
+  __shared__ double lds[(FORCING_ROWS_LDS + 7) / 8];
+  forcing_rows_wg<T>(lmp, red, scale, twy, twz, rows, Ny, Nz, blockIdx.x, lds);
+}
+
 template <typename T>
 static int forcing_plain_t(Ctx& c, double dt, double sim_dt, double nu, double tke_target, double inj_rate,
                            double stats[5], int field)
@@ -312,15 +413,29 @@ static int forcing_plain_t(Ctx& c, double dt, double sim_dt, double nu, double t
   // SpectralForcing::_cub2fftw + runFwd: three forward transforms.
   void* specs[3] = {c.spec, c.spec2, c.spec3};
   if (int rc = launch_fft_forward_fields(c, c.f + v0, specs, 3)) return rc;
-  const size_t n = (size_t)(c.N[0] / 2) * c.N[1] * c.N[2];
-  dim3 g = grid_for(n);
-  if (g.x > 4096) g.x = 4096;
-  if (int rc = ensure_partials(c, 4 * (size_t)g.x)) return rc;
   const double wf[3] = {2 * M_PI / c.extent[0], 2 * M_PI / c.extent[1], 2 * M_PI / c.extent[2]};
-  hipLaunchKernelGGL((k_forcing_filter<T>), g, dim3(NT), 0, c.stream, (C2<T>*)c.spec, (C2<T>*)c.spec2,
-                     (C2<T>*)c.spec3, c.N[0], c.N[1], c.N[2], wf[0], wf[1], wf[2], c.partials);
-  if (int rc = check_hip(c, hipGetLastError(), "k_forcing_filter")) return rc;
-  if (int rc = launch_reduce(c, (int)g.x, 4, 0u, c.sc->red)) return rc;
+  // a band of few low modes is added from its modes, row by row; any other by filtering the spectra
+  // and transforming them back (128^3 FP64: 38 us with the statistics, against 148 for the filter, 3 inverse transforms
+  // and the additions)
+  const bool rows = c.low_fused_ok;
+  int nparts;
+  if (rows) {
+    const int nlines = c.N[1] * c.N[2], lpw = std::min(STAT_LPW_MAX, (nlines + 4095) / 4096);
+    nparts = (nlines + lpw - 1) / lpw;
+    if (int rc = ensure_partials(c, 4 * (size_t)nparts)) return rc;
+    hipLaunchKernelGGL((k_forcing_stats<T>), dim3((nparts + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, c.stream,
+                       (const C2<T>*)c.spec, (const C2<T>*)c.spec2, (const C2<T>*)c.spec3, c.N[0], c.N[1], c.N[2],
+                       wf[0], wf[1], wf[2], lpw, nparts, c.partials);
+  } else {
+    dim3 g = grid_for((size_t)(c.N[0] / 2) * c.N[1] * c.N[2]);
+    if (g.x > 4096) g.x = 4096;
+    nparts = (int)g.x;
+    if (int rc = ensure_partials(c, 4 * (size_t)nparts)) return rc;
+    hipLaunchKernelGGL((k_forcing_filter<T>), g, dim3(NT), 0, c.stream, (C2<T>*)c.spec, (C2<T>*)c.spec2,
+                       (C2<T>*)c.spec3, c.N[0], c.N[1], c.N[2], wf[0], wf[1], wf[2], c.partials);
+  }
+  if (int rc = check_hip(c, hipGetLastError(), "forcing statistics")) return rc;
+  if (int rc = launch_reduce(c, nparts, 4, 0u, c.sc->red)) return rc;
   if (int rc = check_hip(c, hipMemcpyAsync(c.sc_host, c.sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c.stream),
                          "forcing"))
     return rc;
@@ -337,7 +452,15 @@ static int forcing_plain_t(Ctx& c, double dt, double sim_dt, double nu, double t
   if (tke_target > 0) inj = (tke_target - tke) / dt;
   else if (inj_rate > 0) inj = inj_rate;
   const double fac = sim_dt * inj / (2 * tkeF);
-  if (fac > 0) {
+  if (fac > 0 && rows) {
+    double* red = forcing_red(c);
+    hipLaunchKernelGGL((k_low_modes<T>), dim3(1), dim3(128), 0, c.stream, (const C2<T>*)c.spec, (const C2<T>*)c.spec2,
+                       (const C2<T>*)c.spec3, c.low_dev, red, c.N[0], c.N[1], c.N[2]);
+    hipLaunchKernelGGL((k_forcing_rows_scaled<T>), dim3(c.N[2]), dim3(NT), 0, c.stream, c.low_dev, (const double*)red,
+                       fac / normFFT, (const C2<T>*)c.tw[1], (const C2<T>*)c.tw[2], (T*)c.low_rows, c.N[1], c.N[2]);
+    if (int rc = check_hip(c, hipGetLastError(), "forcing rows")) return rc;
+    if (int rc = launch_add_rows(c, v0)) return rc;
+  } else if (fac > 0) {
     for (int q = 0; q < 3; ++q) {
       if (int rc = launch_fft_inverse_fields(c, specs + q, &c.rbuf, 1)) return rc;
       hipLaunchKernelGGL((k_axpy_blocks<T>), grid_for(c.ncell), dim3(NT), 0, c.stream, (T*)c.f[v0 + q],
@@ -616,9 +739,6 @@ ColExtra forcing_planes_extra(Ctx& c)
   e.nz = c.N[2];
   return e;
 }
-
-// The mode sums, behind the plane partials [Nz][parts][16][5].
-static double* forcing_red(const Ctx& c) { return c.low_red + (size_t)c.N[2] * FR_PARTS_MAX * 16 * 5; }
 
 ForcingArgs forcing_args(const Ctx& c, double tke_target, double inj_rate)
 {

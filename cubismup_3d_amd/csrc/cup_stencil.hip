@@ -1306,6 +1306,51 @@ static int gradp_t(Ctx& c, bool fused, const double uinf[3], const int* skip, bo
   return check_hip(c, hipGetLastError(), "k_gradp");
 }
 
+// The forcing's velocity modes added to three fields, as k_gradp adds them.
+template <typename T>
+__global__ __launch_bounds__(NT) void k_add_rows(T* __restrict__ u, T* __restrict__ v, T* __restrict__ w, GridArgs g,
+                                                 const T* __restrict__ rows, const C2<T>* __restrict__ twx)
+{
+  using V2 = typename Vec2<T>::type;
+  using V4 = typename Vec4<T>::type;
+  __shared__ __align__(16) T rl[64 * 16];
+  const int t = threadIdx.x, b = xcd_remap(blockIdx.x, gridDim.x);
+  int bx, by, bz;
+  block_coords(g, b, bx, by, bz);
+  const size_t o = (size_t)b * BS3 + 2 * t;
+  T* f[3] = {u, v, w};
+  V2 a[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) a[q] = *reinterpret_cast<const V2*>(f[q] + o);
+  *reinterpret_cast<V4*>(rl + 4 * t) =
+      *reinterpret_cast<const V4*>(rows + ((size_t)(bz * BS + (t >> 5)) * g.Ny + by * BS) * 16 + (t & 31) * 4);
+  __syncthreads();
+  const T* R = rl + (t >> 2) * 16;  // the row (iz, iy) of the thread's pair
+  T add[3][2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const C2<T> e1 = twx[bx * BS + ((2 * t) & 7) + k];
+    const C2<T> e2 = {e1.x * e1.x - e1.y * e1.y, 2 * e1.x * e1.y};
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      add[q][k] = R[5 * q] + 2 * (R[5 * q + 1] * e1.x + R[5 * q + 2] * e1.y) +
+                  2 * (R[5 * q + 3] * e2.x + R[5 * q + 4] * e2.y);
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<V2*>(f[q] + o) = V2{a[q].x + add[q][0], a[q].y + add[q][1]};
+}
+
+int launch_add_rows(Ctx& c, int f0)
+{
+  if (c.precision == 4)
+    hipLaunchKernelGGL((k_add_rows<float>), dim3(c.nb), dim3(NT), 0, c.stream, (float*)c.f[f0], (float*)c.f[f0 + 1],
+                       (float*)c.f[f0 + 2], c.grid(), (const float*)c.low_rows, (const C2<float>*)c.tw[0]);
+  else
+    hipLaunchKernelGGL((k_add_rows<double>), dim3(c.nb), dim3(NT), 0, c.stream, (double*)c.f[f0], (double*)c.f[f0 + 1],
+                       (double*)c.f[f0 + 2], c.grid(), (const double*)c.low_rows, (const C2<double>*)c.tw[0]);
+  return check_hip(c, hipGetLastError(), "k_add_rows");
+}
+
 // Gradient step in place on the three fields from field0 (no reductions): the adjoint
 // projection's last pass.
 int launch_gradp_inplace(Ctx& c, int field0)
