@@ -388,15 +388,22 @@ int cup_calc_max_timestep(cup_ctx* ctx, double CFL, double nu, const double uinf
   }
   if (dt_out) *dt_out = dt;
   if (umax_out) *umax_out = umax;
-  return launch_set_dt(c, dt);
+  c.host_dt = dt;
+  return c.decomposition == CUP_FUSED ? launch_set_dt(c, dt) : CUP_OK;
 }
 
 int cup_advect_diffuse(cup_ctx* ctx, double dt, double nu, const double uinf[3], int scheme)
 {
   CUP_GUARD(ctx);
   if (!uinf || !(dt > 0)) return set_error(c, CUP_E_INVALID, "advect_diffuse: dt must be > 0");
-  if (int rc = launch_set_dt(c, dt)) return rc;
-  if (int rc = launch_advdiff(c, nu, uinf, scheme)) return rc;
+  // the PLAIN central advection takes dt as an argument; the others' kernels, and what follows them
+  // in the FUSED decomposition, read it from the device
+  c.host_dt = dt;
+  const StepFold arg{nullptr, 0, 0.0, 0, dt};
+  const bool by_arg = c.decomposition == CUP_PLAIN && scheme == CUP_CENTRAL_EULER;
+  if (!by_arg)
+    if (int rc = launch_set_dt(c, dt)) return rc;
+  if (int rc = launch_advdiff(c, nu, uinf, scheme, by_arg ? &arg : nullptr)) return rc;
   if (c.decomposition == CUP_PLAIN) {  // u = tmp = u*, as after the reference's copy
     if (int rc = c.ustar == CUP_U ? launch_copy_u_to_tmp(c) : launch_copy_tmp_to_u(c)) return rc;
     if (!c.periodic())
@@ -416,9 +423,11 @@ int cup_pressure_rhs(cup_ctx* ctx, double dt)
 {
   CUP_GUARD(ctx);
   if (!(dt > 0)) return set_error(c, CUP_E_INVALID, "pressure_rhs: dt must be > 0");
-  if (int rc = launch_set_dt(c, dt)) return rc;
+  c.host_dt = dt;
+  if (c.decomposition == CUP_FUSED)  // the fused solve reads it
+    if (int rc = launch_set_dt(c, dt)) return rc;
   if (c.decomposition == CUP_PLAIN) {
-    if (int rc = launch_rhs_plain(c)) return rc;  // every cell of rbuf, so no PoissonSolver::reset
+    if (int rc = launch_rhs_plain(c, dt)) return rc;  // every cell of rbuf, so no PoissonSolver::reset
     if (c.body.present)
       if (int rc = launch_rhs_obstacle(c, c.rbuf)) return rc;
   } else if (c.body.present) {
@@ -454,8 +463,9 @@ int cup_pressure_project(cup_ctx* ctx, double dt)
 {
   CUP_GUARD(ctx);
   if (!(dt > 0)) return set_error(c, CUP_E_INVALID, "pressure_project: dt must be > 0");
+  c.host_dt = dt;
+  if (c.decomposition == CUP_PLAIN) return launch_gradp_plain(c, dt);
   if (int rc = launch_set_dt(c, dt)) return rc;
-  if (c.decomposition == CUP_PLAIN) return launch_gradp_plain(c);
   const double zero[3] = {0, 0, 0};
   return launch_gradp_fused(c, zero, nullptr);
 }

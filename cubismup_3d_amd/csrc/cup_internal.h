@@ -192,7 +192,7 @@ struct Ctx {
   double* mden[3] = {};   // PoissonSolverMixed's per-axis symbol terms (lazy)
   bool unbounded = false; // freespace faces on every axis: PoissonSolverUnbounded (bc[] holds them as open)
   Ctx* unb = nullptr;     // PoissonSolverUnbounded's padded periodic grid (lazy)
-  void* ghat = nullptr;   // (padded grid) the Green's function's spectrum, FP64 complex
+  void* ghat = nullptr;   // (padded grid) the Green's function's spectrum, FP64: [Nz][Ny][Nx/2], then kx = Nx/2's [Nz][Ny]
   double* partials = nullptr;
   size_t partials_cap = 0;  // doubles
   double* red_part = nullptr;  // launch_reduce's first stage, behind ke_part: [REDUCE_CHUNKS][up to 32 components]
@@ -326,7 +326,7 @@ struct StepFold {
   long long step;
   double CFL;
   int rampup;
-  double fixed_dt;
+  double fixed_dt;  // with slots null: > 0, the dt (a host-driven operator's), else DevScalars' dt
 };
 int launch_advdiff(Ctx& c, double nu, const double uinf[3], int scheme, const StepFold* fold = nullptr);  // -> tmp
 int launch_copy_tmp_to_u(Ctx& c);
@@ -351,8 +351,10 @@ struct AdjBodyArgs {
   bool centre = false;
 };
 int launch_adjoint_body(Ctx& c, AdjBodyPhase phase, const AdjBodyArgs& a);
-int launch_rhs_plain(Ctx& c);                                   // -> rbuf
-int launch_gradp_plain(Ctx& c);                                 // u += -dt/2h grad p
+// A host-driven operator's dt goes to its kernel as an argument: a launch that puts it on the device
+// first costs as much as a third of such a kernel on small grids.
+int launch_rhs_plain(Ctx& c, double dt);    // -> rbuf
+int launch_gradp_plain(Ctx& c, double dt);  // u += -dt/2h grad p
 // xface: take p's x faces from c.xface when the fused Poisson solve just wrote them
 int launch_gradp_fused(Ctx& c, const double uinf[3], const int* skip_slot, bool force = false,
                        bool xface = false);  // u = tmp - dt/2h grad p; max, ke_part

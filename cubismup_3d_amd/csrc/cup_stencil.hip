@@ -493,7 +493,7 @@ __global__ __launch_bounds__(NT) void k_advdiff_xwalk(const T* __restrict__ u, c
       sc->dt = dt;
     }
   } else {
-    dt = sc->dt;
+    dt = fold.fixed_dt > 0 ? fold.fixed_dt : sc->dt;
   }
   const T facA = (T)(-dt / (2 * g.h));
   const T facD = (T)((nu / g.h) * (dt / g.h));
@@ -879,7 +879,7 @@ int launch_advdiff(Ctx& c, double nu, const double uinf[3], int scheme, const St
   if (scheme != CUP_UPWIND3_EULER && scheme != CUP_UPWIND3_RK2)
     return set_error(c, CUP_E_INVALID, "advect_diffuse: unknown scheme");
   if (!c.periodic()) return set_error(c, CUP_E_INVALID, "advect_diffuse: the upwind schemes need a periodic box");
-  if (fold) return set_error(c, CUP_E_STATE, "advect_diffuse: the folded step bookkeeping takes the central scheme");
+  if (fold) return set_error(c, CUP_E_STATE, "advect_diffuse: the step fold takes the central scheme");
   auto stage = [&](int src0, int base0, int out0, double mult) {
     return c.precision == 4 ? up3_stage<float>(c, src0, base0, out0, nu, uinf, mult)
                             : up3_stage<double>(c, src0, base0, out0, nu, uinf, mult);
@@ -1074,7 +1074,7 @@ int launch_set_dt(Ctx& c, double dt)
 template <typename T>
 __global__ __launch_bounds__(NT) void k_rhs(const T* __restrict__ u, const T* __restrict__ v,
                                             const T* __restrict__ w, T* __restrict__ rhs, GridArgs g,
-                                            const DevScalars* __restrict__ sc)
+                                            double dt)
 {
   __shared__ T lab[3][L1C];
   const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(NT) void k_rhs(const T* __restrict__ u, const T* __
   const T* src[3] = {u, v, w};
   gather_g1<T, 3>(src, lab, g, b, bx, by, bz, {HK_VEL, HK_VEL, HK_VEL});
   __syncthreads();
-  const T fac = (T)(0.5 * g.h * g.h / sc->dt);
+  const T fac = (T)(0.5 * g.h * g.h / dt);
   for (int c = threadIdx.x; c < BS3; c += NT) {
     const int ix = c & 7, iy = (c >> 3) & 7, iz = c >> 6;
     const int l = ((iz + 1) * L1 + iy + 1) * L1 + ix + 1;
@@ -1092,15 +1092,15 @@ __global__ __launch_bounds__(NT) void k_rhs(const T* __restrict__ u, const T* __
   }
 }
 
-int launch_rhs_plain(Ctx& c)
+int launch_rhs_plain(Ctx& c, double dt)
 {
   const int src0 = c.decomposition == CUP_FUSED ? c.ustar : CUP_U;
   if (c.precision == 4)
     hipLaunchKernelGGL((k_rhs<float>), dim3(c.nb), dim3(NT), 0, c.stream, (const float*)c.f[src0],
-                       (const float*)c.f[src0 + 1], (const float*)c.f[src0 + 2], (float*)c.rbuf, c.grid(), c.sc);
+                       (const float*)c.f[src0 + 1], (const float*)c.f[src0 + 2], (float*)c.rbuf, c.grid(), dt);
   else
     hipLaunchKernelGGL((k_rhs<double>), dim3(c.nb), dim3(NT), 0, c.stream, (const double*)c.f[src0],
-                       (const double*)c.f[src0 + 1], (const double*)c.f[src0 + 2], (double*)c.rbuf, c.grid(), c.sc);
+                       (const double*)c.f[src0 + 1], (const double*)c.f[src0 + 2], (double*)c.rbuf, c.grid(), dt);
   return check_hip(c, hipGetLastError(), "k_rhs");
 }
 
@@ -1153,7 +1153,8 @@ __global__ __launch_bounds__(NT) void k_gradp(const T* __restrict__ p, const T* 
                                               double* __restrict__ ke_part, const int* __restrict__ skip_slot,
                                               const T* __restrict__ rows, const C2<T>* __restrict__ twx, int nbw,
                                               unsigned long long* __restrict__ slots,
-                                              unsigned long long* __restrict__ clear_slots, const T* __restrict__ xf)
+                                              unsigned long long* __restrict__ clear_slots, const T* __restrict__ xf,
+                                              double dt_arg)
 {
   using V2 = typename Vec2<T>::type;
   using V4 = typename Vec4<T>::type;
@@ -1195,7 +1196,7 @@ __global__ __launch_bounds__(NT) void k_gradp(const T* __restrict__ p, const T* 
       e2[k] = C2<T>{e1[k].x * e1[k].x - e1[k].y * e1[k].y, 2 * e1[k].x * e1[k].y};  // e^{-2 i a x}
     }
   }
-  const T fac = (T)(-0.5 * sc->dt / g.h);
+  const T fac = (T)(-0.5 * (FUSED ? sc->dt : (dt_arg > 0 ? dt_arg : sc->dt)) / g.h);
   double mx = 0.0;
   for (int j = 0; j < nbw; ++j) {
     const int b = b0 + j * nxy;
@@ -1265,7 +1266,8 @@ __global__ __launch_bounds__(NT) void k_gradp(const T* __restrict__ p, const T* 
 }
 
 template <typename T>
-static int gradp_t(Ctx& c, bool fused, const double uinf[3], const int* skip, bool force, bool xface = false)
+static int gradp_t(Ctx& c, bool fused, const double uinf[3], const int* skip, bool force, bool xface = false,
+                   double dt = 0)
 {
   const T* p = (const T*)c.f[CUP_P];
   const int s = fused ? c.ustar : CUP_U;
@@ -1277,32 +1279,32 @@ static int gradp_t(Ctx& c, bool fused, const double uinf[3], const int* skip, bo
     hipLaunchKernelGGL((k_gradp<T, true, true, false, true>), grid, dim3(NT), 0, c.stream, p, (const T*)c.f[s],
                        (const T*)c.f[s + 1], (const T*)c.f[s + 2], (T*)c.f[CUP_U], (T*)c.f[CUP_V], (T*)c.f[CUP_W],
                        c.grid(), c.sc, uinf[0], uinf[1], uinf[2], c.ke_part, skip, (const T*)c.low_rows, tx, nbw,
-                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), xf);
+                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), xf, 0.0);
   else if (fused && xface)
     hipLaunchKernelGGL((k_gradp<T, true, false, false, true>), grid, dim3(NT), 0, c.stream, p, (const T*)c.f[s],
                        (const T*)c.f[s + 1], (const T*)c.f[s + 2], (T*)c.f[CUP_U], (T*)c.f[CUP_V], (T*)c.f[CUP_W],
                        c.grid(), c.sc, uinf[0], uinf[1], uinf[2], c.ke_part, skip, (const T*)nullptr, tx, nbw,
-                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), xf);
+                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), xf, 0.0);
   else if (fused && force)
     hipLaunchKernelGGL((k_gradp<T, true, true, false>), grid, dim3(NT), 0, c.stream, p, (const T*)c.f[s],
                        (const T*)c.f[s + 1], (const T*)c.f[s + 2], (T*)c.f[CUP_U], (T*)c.f[CUP_V], (T*)c.f[CUP_W],
                        c.grid(), c.sc, uinf[0], uinf[1], uinf[2], c.ke_part, skip, (const T*)c.low_rows, tx, nbw,
-                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), nullptr);
+                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), nullptr, 0.0);
   else if (fused)
     hipLaunchKernelGGL((k_gradp<T, true, false, false>), grid, dim3(NT), 0, c.stream, p, (const T*)c.f[s],
                        (const T*)c.f[s + 1], (const T*)c.f[s + 2], (T*)c.f[CUP_U], (T*)c.f[CUP_V], (T*)c.f[CUP_W],
                        c.grid(), c.sc, uinf[0], uinf[1], uinf[2], c.ke_part, skip, (const T*)nullptr, tx, nbw,
-                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), nullptr);
+                       umax_slots_dev(c, c.umax_bank), umax_slots_dev(c, c.umax_bank ^ 1), nullptr, 0.0);
   else if (c.periodic())
     hipLaunchKernelGGL((k_gradp<T, false, false, false>), grid, dim3(NT), 0, c.stream, p, (const T*)c.f[s],
                        (const T*)c.f[s + 1], (const T*)c.f[s + 2], (T*)c.f[CUP_U], (T*)c.f[CUP_V], (T*)c.f[CUP_W],
                        c.grid(), c.sc, 0.0, 0.0, 0.0, (double*)nullptr, (const int*)nullptr, (const T*)nullptr, tx,
-                       nbw, (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr);
+                       nbw, (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr, dt);
   else
     hipLaunchKernelGGL((k_gradp<T, false, false, true>), grid, dim3(NT), 0, c.stream, p, (const T*)c.f[s],
                        (const T*)c.f[s + 1], (const T*)c.f[s + 2], (T*)c.f[CUP_U], (T*)c.f[CUP_V], (T*)c.f[CUP_W],
                        c.grid(), c.sc, 0.0, 0.0, 0.0, (double*)nullptr, (const int*)nullptr, (const T*)nullptr, tx,
-                       nbw, (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr);
+                       nbw, (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr, dt);
   return check_hip(c, hipGetLastError(), "k_gradp");
 }
 
@@ -1362,13 +1364,13 @@ int launch_gradp_inplace(Ctx& c, int field0)
     hipLaunchKernelGGL((k_gradp<float, false, false, false>), grid, dim3(NT), 0, c.stream, (const float*)c.f[CUP_P], f[0],
                        f[1], f[2], f[0], f[1], f[2], c.grid(), c.sc, 0.0, 0.0, 0.0, (double*)nullptr,
                        (const int*)nullptr, (const float*)nullptr, (const C2<float>*)c.tw[0], nbw,
-                       (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr);
+                       (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr, 0.0);
   } else {
     double* f[3] = {(double*)c.f[field0], (double*)c.f[field0 + 1], (double*)c.f[field0 + 2]};
     hipLaunchKernelGGL((k_gradp<double, false, false, false>), grid, dim3(NT), 0, c.stream, (const double*)c.f[CUP_P],
                        f[0], f[1], f[2], f[0], f[1], f[2], c.grid(), c.sc, 0.0, 0.0, 0.0, (double*)nullptr,
                        (const int*)nullptr, (const double*)nullptr, (const C2<double>*)c.tw[0], nbw,
-                       (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr);
+                       (unsigned long long*)nullptr, (unsigned long long*)nullptr, nullptr, 0.0);
   }
   return check_hip(c, hipGetLastError(), "k_gradp");
 }
@@ -1552,10 +1554,10 @@ int launch_up3_stage(Ctx& c, int src0, int base0, int out0, double nu, const dou
                           : up3_stage<double>(c, src0, base0, out0, nu, uinf, mult);
 }
 
-int launch_gradp_plain(Ctx& c)
+int launch_gradp_plain(Ctx& c, double dt)
 {
-  return c.precision == 4 ? gradp_t<float>(c, false, nullptr, nullptr, false)
-                          : gradp_t<double>(c, false, nullptr, nullptr, false);
+  return c.precision == 4 ? gradp_t<float>(c, false, nullptr, nullptr, false, false, dt)
+                          : gradp_t<double>(c, false, nullptr, nullptr, false, false, dt);
 }
 
 int launch_gradp_fused(Ctx& c, const double uinf[3], const int* skip_slot, bool force, bool xface)
