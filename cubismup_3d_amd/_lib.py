@@ -58,6 +58,8 @@ SIGNATURES = {
     "cup_field_device_ptr": (_i, [_p, _i, C.POINTER(C.c_void_p)]),
     "cup_set_field_device": (_i, [_p, _i, _p]),
     "cup_get_field_device": (_i, [_p, _i, _p]),
+    "cup_set_velocity_device": (_i, [_p, _p]),
+    "cup_get_velocity_device": (_i, [_p, _p]),
     "cup_lab_shift": (_i, [_p, _i, _i, _i, _i]),
     "cup_max_velocity": (_i, [_p, _dp, _dp]),
     "cup_calc_max_timestep": (_i, [_p, _d, _d, _dp, _i, _i, _dp, _dp]),

@@ -349,6 +349,24 @@ int cup_get_field_device(cup_ctx* ctx, int field, void* dst)
                    "get_field_device");
 }
 
+int cup_set_velocity_device(cup_ctx* ctx, const void* src)
+{
+  CUP_GUARD(ctx);
+  if (!src) return set_error(c, CUP_E_INVALID, "set_velocity_device: null pointer");
+  const size_t fb = c.ncell * c.esz;
+  const void* s[3] = {src, (const char*)src + fb, (const char*)src + 2 * fb};
+  return launch_copy3(c, c.f + CUP_U, s);
+}
+
+int cup_get_velocity_device(cup_ctx* ctx, void* dst)
+{
+  CUP_GUARD(ctx);
+  if (!dst) return set_error(c, CUP_E_INVALID, "get_velocity_device: null pointer");
+  const size_t fb = c.ncell * c.esz;
+  void* d[3] = {dst, (char*)dst + fb, (char*)dst + 2 * fb};
+  return launch_copy3(c, d, c.f + CUP_U);
+}
+
 int cup_lab_shift(cup_ctx* ctx, int g, int dx, int dy, int dz)
 {
   CUP_GUARD(ctx);
@@ -982,13 +1000,8 @@ static int keep_velocity(Ctx& c, bool back)
 {
   const size_t fb = c.ncell * c.esz;
   char* keep = (char*)c.adjf + 6 * fb;
-  for (int q = 0; q < 3; ++q) {
-    void* dst = back ? c.f[CUP_U + q] : (void*)(keep + q * fb);
-    const void* src = back ? (const void*)(keep + q * fb) : c.f[CUP_U + q];
-    if (int e = check_hip(c, hipMemcpyAsync(dst, src, fb, hipMemcpyDeviceToDevice, c.stream), "keep velocity"))
-      return e;
-  }
-  return CUP_OK;
+  void* k[3] = {keep, keep + fb, keep + 2 * fb};
+  return back ? launch_copy3(c, c.f + CUP_U, k) : launch_copy3(c, k, c.f + CUP_U);
 }
 
 static int alloc_adjf(Ctx& c)

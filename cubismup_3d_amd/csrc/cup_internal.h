@@ -330,6 +330,7 @@ struct StepFold {
 };
 int launch_advdiff(Ctx& c, double nu, const double uinf[3], int scheme, const StepFold* fold = nullptr);  // -> tmp
 int launch_copy_tmp_to_u(Ctx& c);
+int launch_copy3(Ctx& c, void* const* dst, const void* const* src);  // three fields
 int launch_copy_u_to_tmp(Ctx& c);
 int launch_adjoint_advdiff(Ctx& c, double nu, const double uinf[3]);
 constexpr int F_ADJ2 = 11;

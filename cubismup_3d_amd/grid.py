@@ -152,12 +152,10 @@ class Grid:
         return out
 
     def keep_velocity(self, buf):
-        for q, n in enumerate("uvw"):
-            self._c(L.lib().cup_get_field_device(self._h, L.FIELD_IDS[n], C.c_void_p(buf[q].data_ptr())))
+        self._c(L.lib().cup_get_velocity_device(self._h, C.c_void_p(buf.data_ptr())))
 
     def restore_velocity(self, buf):
-        for q, n in enumerate("uvw"):
-            self._c(L.lib().cup_set_field_device(self._h, L.FIELD_IDS[n], C.c_void_p(buf[q].data_ptr())))
+        self._c(L.lib().cup_set_velocity_device(self._h, C.c_void_p(buf.data_ptr())))
 
     def set_torch_adjoint(self, lam):
         for q, n in enumerate(("adjU", "adjV", "adjW")):

@@ -98,6 +98,9 @@ int cup_field_device_ptr(cup_ctx* ctx, int field, void** dptr);
  * calls cup_synchronize before reading dst elsewhere). */
 int cup_set_field_device(cup_ctx* ctx, int field, const void* src);
 int cup_get_field_device(cup_ctx* ctx, int field, void* dst);
+/* The same for u, v and w together, one behind the other in src or dst: one pass over the three. */
+int cup_set_velocity_device(cup_ctx* ctx, const void* src);
+int cup_get_velocity_device(cup_ctx* ctx, void* dst);
 
 /* TestBoundaries.cpp:19-75 restated on the device: tmpU = lab(-dx,-dy,-dz).u through the
  * LDS-staged periodic halo gather with halo width g (1 or 2). */
