@@ -577,7 +577,10 @@ static int advdiff_t(Ctx& c, double nu, const double uinf[3], const StepFold* fo
   // on 160 x 96 x 120, 18.5 / 15.8 / 15.6 / 16.5 on 128^3, 130 / 106 / 100 / 106 on 256^3. FP64,
   // whose x faces cost more sectors: 12.1 / 12.4 / 13.1 / 16.6 on 64^3, 19.1 / 17.7 / 14.8 on
   // 96^3, 33.8 / 26.4 / 24.9 / 23.4 on 128^3.
-  const int nbw = sizeof(T) == 4 ? walk_blocks(c.bpd[0], c.nb, 4, 1024) : walk_blocks(c.bpd[0], c.nb, 8, 256);
+  // Non-periodic grids take 8 or 2: the compiler keeps some of the 4 and 1 forms' state in scratch
+  // or LDS there (26 against 16 us for 4 against 8 on 128 x 96 x 64 FP64).
+  int nbw = sizeof(T) == 4 ? walk_blocks(c.bpd[0], c.nb, 4, 1024) : walk_blocks(c.bpd[0], c.nb, 8, 256);
+  if (!c.periodic()) nbw = c.bpd[0] % 8 == 0 && c.nb / 8 >= 128 ? 8 : (c.bpd[0] % 2 == 0 ? 2 : 1);
   if (nbw == 8) launch_advdiff_xwalk<T, 8>(c, nu, uinf, fold, fd);
   else if (nbw == 4) launch_advdiff_xwalk<T, 4>(c, nu, uinf, fold, fd);
   else if (nbw == 2) launch_advdiff_xwalk<T, 2>(c, nu, uinf, fold, fd);
