@@ -1348,10 +1348,10 @@ int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_block
 //
 // One workgroup transforms LN lines of N cells: it stages them in LDS as X[j][line] and forms
 // Y = M X in 16 x 16 tiles of the 16x16x4 matrix instruction (M's fragments from the cache, 16
-// columns of j in flight; X's from LDS, two line groups per fragment of M), then stores each tile
+// columns of j ahead; X's from LDS, two line groups per fragment of M), then stores each tile
 // back over its lines. What bounds it is the latency of M's fragments in the cache, not the
 // matrix units (2 us a pass at their rate) or the field's traffic: on 128 x 96 x 64 cells in FP64
-// a pass takes 9 to 14 us, against 50 us with one thread per output walking its line, where every
+// a pass takes 9 to 12 us, against 50 us with one thread per output walking its line, where every
 // line read the whole matrix.
 template <typename T>
 struct MatTile;
@@ -1378,23 +1378,27 @@ struct MatTile<float> {
 constexpr int R2R_STAGE = 17;  // row pitch of a wave's 16 x 16 staging tile
 // Row pitch of X: the four rows a fragment reads fall on distinct banks.
 constexpr int r2r_pitch(int ln) { return ln == 16 ? 16 : ln + 16; }
+// Threads: a wave for each 16 x 16 tile of 16 lines up to 128 cells (a launch of few workgroups lasts
+// as long as a wave's tiles), four waves otherwise.
+template <int LN>
+constexpr int r2r_threads() { return LN == 16 ? 512 : NT; }
 template <typename T, int LN, int AXIS>
 inline size_t r2r_lds(int n)
 {
-  return ((size_t)n * r2r_pitch(LN) + (AXIS == 0 ? NT / 64 * 16 * R2R_STAGE : 0)) * sizeof(T);
+  return ((size_t)n * r2r_pitch(LN) + (AXIS == 0 ? r2r_threads<LN>() / 64 * 16 * R2R_STAGE : 0)) * sizeof(T);
 }
 
 // src and dst may be the same field: a workgroup reads its lines before it writes them. dx, dy,
 // dz: the symbol's terms when this pass (along z) also divides, else null.
 template <typename T, int LN, int AXIS>
-__global__ __launch_bounds__(NT) void k_r2r_axis(const T* src, T* dst, const T* __restrict__ mt, GridArgs g,
+__global__ __launch_bounds__(r2r_threads<LN>()) void k_r2r_axis(const T* src, T* dst, const T* __restrict__ mt, GridArgs g,
                                                  double norm, const double* __restrict__ dx,
                                                  const double* __restrict__ dy, const double* __restrict__ dz)
 {
   using MT = MatTile<T>;
   using V2 = typename Vec2<T>::type;
   using V4 = typename Vec4<T>::type;
-  constexpr int PX = r2r_pitch(LN), SUB = 64 / LN, NG = LN / 16, GI = NG > 1 ? 2 : 1;
+  constexpr int BT = r2r_threads<LN>(), PX = r2r_pitch(LN), SUB = 64 / LN, NG = LN / 16, GI = NG > 1 ? 2 : 1;
   extern __shared__ __align__(32) unsigned char r2r_lds_buf[];
   T* X = reinterpret_cast<T*>(r2r_lds_buf);
   const int n = AXIS == 0 ? g.Nx : (AXIS == 1 ? g.Ny : g.Nz);
@@ -1407,7 +1411,8 @@ __global__ __launch_bounds__(NT) void k_r2r_axis(const T* src, T* dst, const T* 
   };
   // Pairs of x-adjacent cells; line = (iz, iy) for x, (iz, ix) for y, (iy, ix) for z, the first
   // index from sub * LN/8 on. Each wave reads whole 64-byte sectors and writes runs of lines.
-  for (int r = threadIdx.x; r < n * LN / 2; r += NT) {
+  #pragma unroll 4
+  for (int r = threadIdx.x; r < n * LN / 2; r += BT) {
     const int q = r / (LN * 4), p = r % (LN * 4);
     int cell, j, line;
     if (AXIS == 0) {
@@ -1437,31 +1442,37 @@ __global__ __launch_bounds__(NT) void k_r2r_axis(const T* src, T* dst, const T* 
   __syncthreads();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lc = lane & 15, lr = lane >> 4;
   const int items = (n + 15) / 16 * (NG / GI);
-  for (int item = wv; item < items; item += NT / 64) {
+  for (int item = wv; item < items; item += BT / 64) {
     const int i0 = item / (NG / GI) * 16, g0 = item % (NG / GI) * GI;
     const int ai = min(i0 + lc, n - 1);  // the last tile's rows past n are not stored
     typename MT::acc acc[GI];
 #pragma unroll
     for (int q = 0; q < GI; ++q) acc[q] = typename MT::acc{0, 0, 0, 0};
-    T a[4], an[4];
-    auto fetch = [&](T (&f)[4], int j0) {  // n is a multiple of 8: the last 16 columns may be half empty
+    // M's fragments, two groups of 16 columns ahead (n is a multiple of 8: the last group may be half
+    // empty)
+    T a[3][4];
+    auto fetch = [&](T (&f)[4], int j0) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int j = j0 + 4 * q + lr;
         f[q] = j < n ? mt[(size_t)j * n + ai] : (T)0;
       }
     };
-    fetch(a, 0);
+    fetch(a[0], 0);
+    fetch(a[1], 16);
     for (int j0 = 0; j0 < n; j0 += 16) {
-      if (j0 + 16 < n) fetch(an, j0 + 16);
+      fetch(a[2], j0 + 32);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int j = min(j0 + 4 * q + lr, n - 1);
 #pragma unroll
-        for (int k = 0; k < GI; ++k) acc[k] = MT::mma(a[q], X[j * PX + (g0 + k) * 16 + lc], acc[k]);
+        for (int k = 0; k < GI; ++k) acc[k] = MT::mma(a[0][q], X[j * PX + (g0 + k) * 16 + lc], acc[k]);
       }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) a[q] = an[q];
+      for (int q = 0; q < 4; ++q) {
+        a[0][q] = a[1][q];
+        a[1][q] = a[2][q];
+      }
     }
 #pragma unroll
     for (int k = 0; k < GI; ++k) {
@@ -1550,7 +1561,7 @@ static void r2r_pass(Ctx& c, const T* src, T* dst, int q, double norm, bool divi
 {
   const int n = c.N[AXIS], rows = (int)(c.ncell / (size_t)n / 64);
   auto go = [&](auto kern, int ln, size_t lds) {
-    hipLaunchKernelGGL(kern, dim3(rows * (64 / ln)), dim3(NT), lds, c.stream, src, dst, (const T*)c.r2r[AXIS][q],
+    hipLaunchKernelGGL(kern, dim3(rows * (64 / ln)), dim3(ln == 16 ? r2r_threads<16>() : NT), lds, c.stream, src, dst, (const T*)c.r2r[AXIS][q],
                        c.grid(), norm, (const double*)(divide ? c.mden[0] : nullptr), (const double*)c.mden[1],
                        (const double*)c.mden[2]);
   };
