@@ -53,8 +53,6 @@ static void release(Ctx& c)
     if (p) { hipFree(p); p = nullptr; }
   if (c.ana) hipFree(c.ana);
   c.ana = nullptr;
-  if (c.ana_host) hipHostFree(c.ana_host);
-  c.ana_host = nullptr;
   void** bufs[] = {&c.spec, &c.spec2, &c.spec3, &c.rbuf, &c.xface, &c.tw[0], &c.tw[1], &c.tw[2]};
   for (void** b : bufs)
     if (*b) { hipFree(*b); *b = nullptr; }
@@ -214,7 +212,7 @@ int cup_create(const cup_grid_desc* d, cup_ctx** out)
     if ((rc = check_hip(c, hipHostMalloc((void**)&c.sc_host, sizeof(DevScalars), hipHostMallocDefault),
                         "hipHostMalloc")))
       break;
-    if ((rc = check_hip(c, hipHostMalloc((void**)&c.host_red, 64 * sizeof(double), hipHostMallocDefault),
+    if ((rc = check_hip(c, hipHostMalloc((void**)&c.host_red, HOST_RED * sizeof(double), hipHostMallocDefault),
                         "hipHostMalloc")))
       break;
     if ((rc = ensure_partials(c, 20 * (size_t)c.nb + 1024))) break;

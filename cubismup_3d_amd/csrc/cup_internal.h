@@ -89,6 +89,7 @@ constexpr int REDUCE_CHUNKS = 256;  // workgroups per component of a large reduc
 // Radix plan of a transform length that is not a power of two (FFT passes with the length
 // known at run time): n = r[0] r[1] ... r[ns-1], radices 8, 4, 2, 3, 5.
 constexpr int FFT_MAX_N = 1024;
+constexpr int HOST_RED = 1024;  // values of Ctx::host_red: the HIT analysis reads FFT_MAX_N/2 shells and 5 totals
 struct FftPlan {
   int n = 0, ns = 0;
   int r[16] = {};
@@ -176,7 +177,6 @@ struct Ctx {
   bool plain_rhs = false; // the fused x pass ignores the obstacle RHS (the adjoint's projection)
   void* spec = nullptr;   // packed half spectrum, complex, [z][y][kx], kx < Nx/2
   double* ana = nullptr;  // HIT analysis: per-wave sums [3 + nbin][waves], then the row totals (lazy)
-  double* ana_host = nullptr;  // pinned: the totals
   void* spec2 = nullptr;  // extra spectra for the plain forcing path
   void* spec3 = nullptr;
   void* rbuf = nullptr;   // block-layout real scratch (plain RHS / solution)
@@ -199,7 +199,7 @@ struct Ctx {
   double* ke_part = nullptr;  // [nb][4] partial sums |u|^2 of the fused step's velocity (per wave)
   DevScalars* sc = nullptr;
   DevScalars* sc_host = nullptr;  // pinned
-  double* host_red = nullptr;     // pinned scratch for reductions
+  double* host_red = nullptr;     // pinned scratch for reductions, HOST_RED values
   // forcing: canonical low modes and the fused path's device tables
   int nlow = 0;
   bool low_fused_ok = false;   // modes fit LowModes (count, |kx|)

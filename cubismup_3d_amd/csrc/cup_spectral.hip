@@ -954,9 +954,7 @@ static int hit_analysis_t(Ctx& c, double* sums, double* E, int nbin, double grad
   const size_t nrows = 3 + (size_t)nbin, ntot = nrows + 2;
   if (!c.ana && check_hip(c, hipMalloc(&c.ana, (nrows * nwaves + ntot) * sizeof(double)), "hipMalloc analysis"))
     return CUP_E_NOMEM;
-  if (!c.ana_host && check_hip(c, hipHostMalloc((void**)&c.ana_host, ntot * sizeof(double), hipHostMallocDefault),
-                               "hipHostMalloc analysis"))
-    return CUP_E_NOMEM;
+  static_assert(FFT_MAX_N / 2 + 5 <= HOST_RED, "the totals are read back through host_red");
   void* specs[3] = {c.spec, c.spec2, c.spec3};
   if (int rc = launch_fft_forward_fields(c, c.f + CUP_U, specs, 3)) return rc;
   const int maxN = std::max(c.N[0], std::max(c.N[1], c.N[2]));
@@ -969,13 +967,13 @@ static int hit_analysis_t(Ctx& c, double* sums, double* E, int nbin, double grad
   hipLaunchKernelGGL(k_rows_sum, dim3((unsigned)nrows), dim3(NT), 0, c.stream, (const double*)c.ana, nwaves, tot);
   if (int rc = check_hip(c, hipGetLastError(), "k_hit_analysis")) return rc;
   if (int rc = launch_grad_stats(c, tot + nrows)) return rc;
-  if (int rc = check_hip(c, hipMemcpyAsync(c.ana_host, tot, ntot * sizeof(double), hipMemcpyDeviceToHost, c.stream),
+  if (int rc = check_hip(c, hipMemcpyAsync(c.host_red, tot, ntot * sizeof(double), hipMemcpyDeviceToHost, c.stream),
                          "hipMemcpy analysis"))
     return rc;
   if (int rc = check_hip(c, hipStreamSynchronize(c.stream), "synchronize")) return rc;
-  for (int q = 0; q < 3; ++q) sums[q] = c.ana_host[q];
-  for (int b = 0; b < nbin; ++b) E[b] = c.ana_host[3 + b];
-  for (int q = 0; q < 2; ++q) grad[q] = c.ana_host[nrows + q];
+  for (int q = 0; q < 3; ++q) sums[q] = c.host_red[q];
+  for (int b = 0; b < nbin; ++b) E[b] = c.host_red[3 + b];
+  for (int q = 0; q < 2; ++q) grad[q] = c.host_red[nrows + q];
   return CUP_OK;
 }
 
