@@ -315,8 +315,7 @@ constexpr int x_max(int N) { return N < 0 ? -N : FFT_MAX_N; }
 constexpr int XROWS = 8;         // rows per workgroup = one block row of a z plane
 constexpr int XFFT = XROWS / 2;  // complex FFTs per workgroup (two real rows each)
 
-// XSRC_PAD: a field of half the cells per axis, zero beyond it (the free-space solve); its kx = 0 and
-// kx = Nx/2 values are kept apart, the latter in a column of their own (edge).
+// XSRC_PAD: a field of half the cells per axis, zero beyond it (the free-space solve).
 enum XSrc { XSRC_FIELD = 0, XSRC_DIV = 1, XSRC_PAD = 2 };
 
 // Up to three fields that one launch transforms (one per grid z): a pass over a single field of a
@@ -386,7 +385,7 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
                                                   const C2<T>* __restrict__ tw, GridArgs g,
                                                   const DevScalars* __restrict__ sc, const int* __restrict__ ob_slot,
                                                   const T* __restrict__ ob_rhs, double* __restrict__ rowbuf,
-                                                  FftPlan pl, C2<T>* __restrict__ edge = nullptr)
+                                                  FftPlan pl)
 {
   const int n = N > 0 ? N : pl.n;
   C2<T>* buf = lds_tile<T, (N > 0 ? N : 0) * XFFT>();
@@ -513,10 +512,6 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
     if (k == 0) {
       const C2<T> Zn = buf[(n / 2) * XFFT + q];
       out = odd ? C2<T>{Z.y, Zn.y} : C2<T>{Z.x, Zn.x};
-      if (SRC == XSRC_PAD) {
-        edge[(size_t)z * g.Ny + by * BS + row] = C2<T>{out.y, 0};
-        out.y = 0;
-      }
     } else {
       const C2<T> Zm = buf[(n - k) * XFFT + q];
       // Xa = (Z + conj Zm)/2 ; Xb = -i (Z - conj Zm)/2
@@ -535,7 +530,7 @@ __global__ __launch_bounds__(NT) void k_fft_x_fwd(const T* __restrict__ src0, co
 template <typename T, int N, bool XF = false, bool PAD = false>
 __global__ __launch_bounds__(NT) void k_fft_x_inv(Three<C2<T>> spec, Three<T> fields,
                                                   const C2<T>* __restrict__ tw, GridArgs g, FftPlan pl,
-                                                  T* __restrict__ xf = nullptr, const C2<T>* __restrict__ edge = nullptr)
+                                                  T* __restrict__ xf = nullptr)
 {
   const int n = N > 0 ? N : pl.n;
   C2<T>* buf = lds_tile<T, (N > 0 ? N : 0) * XFFT>();
@@ -547,12 +542,8 @@ __global__ __launch_bounds__(NT) void k_fft_x_inv(Three<C2<T>> spec, Three<T> fi
   for (int t = threadIdx.x; t < XFFT * (n / 2); t += NT) {
     const int q = t / (n / 2), k = t % (n / 2);
     const int ya = by * BS + 2 * q;
-    C2<T> A = S[((size_t)z * g.Ny + ya) * (n / 2) + k];
-    C2<T> B = S[((size_t)z * g.Ny + ya + 1) * (n / 2) + k];
-    if (PAD && k == 0) {
-      A.y = edge[(size_t)z * g.Ny + ya].x;
-      B.y = edge[(size_t)z * g.Ny + ya + 1].x;
-    }
+    const C2<T> A = S[((size_t)z * g.Ny + ya) * (n / 2) + k];
+    const C2<T> B = S[((size_t)z * g.Ny + ya + 1) * (n / 2) + k];
     if (k == 0) {
       buf[0 * XFFT + q] = C2<T>{A.x, B.x};
       buf[(n / 2) * XFFT + q] = C2<T>{A.y, B.y};
@@ -610,7 +601,7 @@ __device__ __forceinline__ double forcing_gg(const ForcingArgs& fa, const LowMod
   return fac > 0 ? fac * fa.h * fa.h / fa.sc->dt : 0.0;
 }
 
-template <typename T, int N, int M, bool FREE>
+template <typename T, int N, int M>
 struct ColStages {
   using CT = ColTile<T, M>;
   static constexpr int TK = CT::TK, BT = CT::BT;
@@ -626,14 +617,10 @@ struct ColStages {
   const LowModes* lmp;  // null: no forcing
   ForcingArgs fa;
   double gg;            // the forcing's factor times h^2/dt (0: none)
-  // FREE, the free-space solve: elements that are not known to be zero, and that are wanted; the
-  // Green's function's spectrum at S's indices
-  int nin, nout;
-  const double* green;
 
   __device__ __forceinline__ C2<T> load(int f, int e) const
   {
-    const C2<T> a = f < nc && (!FREE || e < nin) ? S[base + f + e * stride] : C2<T>{0, 0};
+    const C2<T> a = f < nc ? S[base + f + e * stride] : C2<T>{0, 0};
     return inv ? C2<T>{a.y, a.x} : a;
   }
 
@@ -642,15 +629,6 @@ struct ColStages {
   __device__ __forceinline__ void divide(C2<T> (&v)[R], int f, int j) const
   {
     const int m = n / R;
-    if (FREE) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const double gg0 = f < nc ? green[base + f + (j + r * m) * stride] : 0.0;
-        v[r].x = (T)((double)v[r].x * gg0);
-        v[r].y = (T)((double)v[r].y * gg0);
-      }
-      return;
-    }
     if (lmp && kx0 == 0) {
       const LowModes& lm = *lmp;
       for (int e = 0; e < lm.npos; ++e) {
@@ -729,7 +707,7 @@ struct ColStages {
       if (LAST) {
 #pragma unroll
         for (int r = 0; r < R; ++r)
-          if (f < nc && (!FREE || j + r * m < nout)) S[base + f + (j + r * m) * stride] = swap ? C2<T>{v[it][r].y, v[it][r].x} : v[it][r];
+          if (f < nc) S[base + f + (j + r * m) * stride] = swap ? C2<T>{v[it][r].y, v[it][r].x} : v[it][r];
       } else {
         // MID's outputs are those of the inverse's first stage: k = 0, from j R on
         const int k = MID || FIRST ? 0 : (N > 0 ? j % Ns : mod_ns(j, Ns, rNs));
@@ -798,44 +776,25 @@ struct ColStages {
   }
 };
 
-// The free-space solve's form of a column pass: the padded grid's elements from nin on are zero and
-// those from nout on are not wanted, a last tile of workgroups takes the kx = Nx/2 column (edge),
-// and the z pass multiplies by the Green's function's spectrum (green, and edge_green for the edge).
-template <typename T>
-struct ColFree {
-  int nin, nout;
-  C2<T>* edge;
-  const double *green, *edge_green;
-};
-
 // Column FFT along y (axis 1) or z (axis 2). grid = (ceil(ncols/TK), other axis). POISSON (z only):
 // forward transform, grid-consistent division and inverse transform.
-template <typename T, int N, int M, bool POISSON, bool FREE = false>
+template <typename T, int N, int M, bool POISSON>
 __global__ __launch_bounds__((ColTile<T, M>::BT)) void k_fft_col(Three<C2<T>> S, const C2<T>* __restrict__ tw,
                                                                int ncols, int axis, int inv, int Ny, double norm,
                                                                const double* __restrict__ cx,
                                                                const double* __restrict__ cy,
                                                                const double* __restrict__ cz,
                                                                const LowModes* __restrict__ lmp, ForcingArgs fa,
-                                                               FftPlan pl, ColFree<T> fr)
+                                                               FftPlan pl)
 {
-  using CS = ColStages<T, N, M, FREE>;
+  using CS = ColStages<T, N, M>;
   C2<T>* buf = lds_tile<T, N * CS::TK>();
-  const int o = blockIdx.y;
-  int kx0 = blockIdx.x * CS::TK;
-  C2<T>* Sp = S.p[blockIdx.z];
-  const double* green = fr.green;
-  if (FREE && blockIdx.x == gridDim.x - 1) {
-    Sp = fr.edge;
-    green = fr.edge_green;
-    ncols = 1;
-    kx0 = 0;
-  }
+  const int kx0 = blockIdx.x * CS::TK, o = blockIdx.y;
   const size_t base = (axis == 1 ? (size_t)o * Ny : (size_t)o) * ncols + kx0;
   const size_t stride = axis == 1 ? (size_t)ncols : (size_t)Ny * ncols;
   const int n = N > 0 ? N : pl.n;
-  CS cs{Sp, buf, tw, base, stride, inv != 0, n, min(CS::TK, ncols - kx0), kx0, o, Ny, norm,
-        cx,  cy,  cz, lmp,  fa, POISSON && !FREE && lmp && kx0 == 0 ? forcing_gg(fa, *lmp) : 0.0, fr.nin, fr.nout, green};
+  CS cs{S.p[blockIdx.z], buf, tw, base, stride, inv != 0, n, min(CS::TK, ncols - kx0), kx0, o, Ny, norm,
+        cx, cy, cz, lmp, fa, POISSON && lmp && kx0 == 0 ? forcing_gg(fa, *lmp) : 0.0};
   if constexpr (N > 0) cs.template run_ct<POISSON>();
   else cs.template run_rt<POISSON>(pl);
 }
@@ -1016,6 +975,160 @@ __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>*
     for (int m = 0; m < 16; ++m) S[gi(j + NTH * m)] = v[m];
 }
 
+// ----------------------------------------------- y / z passes of the free-space solve
+
+enum FreeMode { FC_FWD = 0, FC_INV = 1, FC_CONV = 2 };
+
+// L: a length (64 .. 256 in the register form, 512 or 1024 by lds_fft), or minus the bound of a
+// run-time length (lds_fft_rt). 16 elements per thread, or as many columns as 64 KiB of LDS hold.
+template <typename T, int L>
+struct FreeTile {
+  static constexpr int M = L > 0 ? L : -L, TK = L >= 512 ? 65536 / (M * (int)sizeof(C2<T>)) : 16 * NT / M;
+};
+
+// A transform's results, formed where this stands and not in the branches behind it: which product of
+// a sum is rounded depends on the block that the compiler forms the sum in.
+template <typename T>
+__device__ __forceinline__ void hold(C2<T> (&v)[16])
+{
+#pragma unroll
+  for (int q = 0; q < 16; ++q) asm volatile("" : "+v"(v[q].x), "+v"(v[q].y));
+}
+
+// Column passes on the padded grid of which only a part is needed: elements from nin on are zero,
+// those from nout on are not wanted. FC_CONV (z) transforms forward, multiplies by the Green's
+// function's spectrum (real, green, at the spectrum's indices) and transforms back. Slot 0 packs the
+// kx = 0 and kx = Nx/2 planes as A + iB, for which the Green's function has two values, G0 = green and
+// GN = green_n[kz][ky]: the product is a Z(k) + b conj Z(-k), a = (G0 + GN)/2, b = (G0 - GN)/2, so the
+// slot's columns ky and -ky go together, TK/2 such pairs to each workgroup of the grid's last x index.
+//
+// The stages, their order and the packing are those of passes over whole columns and of a product of
+// its own, so the result is theirs bit for bit. After the inflow correction the RHS's sum is rounding
+// noise, and the solve returns it as most of the pressure's mean: another rounding of the solve changes
+// the next step's noise, in FP32 by several times the solve's own error (3e-7 to 1e-5 of |p|).
+template <typename T, int L, int MODE>
+__global__ __launch_bounds__(NT) void k_free_col(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw, int ncols,
+                                                 int axis, int Ny, int nin, int nout,
+                                                 const double* __restrict__ green,
+                                                 const double* __restrict__ green_n, FftPlan pl)
+{
+  constexpr bool REG = L > 0 && ColReg<T, (L > 0 ? L : 8)>::ok;
+  constexpr int M = FreeTile<T, L>::M, TK = FreeTile<T, L>::TK, H = TK / 2, NR = REG ? L : 64;
+  using CR = ColReg<T, NR>;
+  static_assert(!REG || CR::TK == TK, "both forms take as many columns");
+  const int n = L > 0 ? L : pl.n;
+  C2<T>* buf = lds_tile<T, (L > 0 ? L * TK : 0)>();
+  const int o = blockIdx.y, f = threadIdx.x % TK, j = threadIdx.x / TK;
+  const bool pair = MODE == FC_CONV && blockIdx.x == gridDim.x - 1;
+  if (pair && o * H > Ny / 2) return;
+  int kx = blockIdx.x * TK + f, row = o;
+  bool live = kx < ncols && !(MODE == FC_CONV && kx == 0), keep = live;
+  if (pair) {
+    const int k = o * H + f % H, m = k == 0 ? 0 : Ny - k;
+    kx = 0;
+    live = k <= Ny / 2;
+    row = f < H ? k : m;
+    keep = live && (f < H || m != k);  // a column that is its own mirror is held twice
+  }
+  const size_t stride = axis == 1 ? (size_t)ncols : (size_t)Ny * ncols;
+  C2<T>* col = S + (axis == 1 ? (size_t)row * Ny : (size_t)row) * ncols + kx;
+  auto get = [&](int e) { return live && e < nin ? col[e * stride] : C2<T>{0, 0}; };
+  auto times = [&](const C2<T>& v, int e) {
+    const double gg = live ? green[(col - S) + e * stride] : 0.0;
+    return C2<T>{(T)(v.x * gg), (T)(v.y * gg)};
+  };
+  // Element e of slot 0's column row with zm, element -e of the mirrored column. The pair takes the Green's function
+  // at its lower index, and one product of each sum is rounded, the same in both its elements.
+  auto times_pair = [&](const C2<T>& z, const C2<T>& zm, int e, int row) {
+    const size_t i = (size_t)e * Ny + row, m = (size_t)(e == 0 ? 0 : n - e) * Ny + (row == 0 ? 0 : Ny - row);
+    const size_t g = live ? min(i, m) : 0;
+    const double g0 = green[g * ncols], gn = green_n[g];
+    const double a = 0.5 * (g0 + gn), b = 0.5 * (g0 - gn), x = z.x, y = z.y, xm = zm.x, ym = zm.y;
+    return C2<T>{(T)(i <= m ? fma(a, x, b * xm) : fma(b, xm, a * x)), (T)fma(a, y, -(b * ym))};
+  };
+  if constexpr (REG) {
+    constexpr int NTH = CR::NTH, RPT = CR::RPT;
+    C2<T> v[16];
+    if (MODE == FC_INV) {
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+#pragma unroll
+        for (int k2 = 0; k2 < NTH; ++k2) v[i * NTH + k2] = get(j * RPT + i + 16 * k2);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 16; ++m) v[m] = get(j + NTH * m);
+      fft_a_to_b<T, NR, -1>(v, buf, tw, f, j);
+    }
+    if (MODE == FC_FWD) {
+      if (live)
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+#pragma unroll
+          for (int k2 = 0; k2 < NTH; ++k2) col[(j * RPT + i + 16 * k2) * stride] = v[i * NTH + k2];
+      return;
+    }
+    if (MODE == FC_CONV) {
+      if (live) hold(v);
+      else
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = C2<T>{0, 0};
+      __syncthreads();  // the forward transpose's reads of buf are done
+      if (pair) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+#pragma unroll
+          for (int k2 = 0; k2 < NTH; ++k2) buf[(j * RPT + i + 16 * k2) * TK + f] = v[i * NTH + k2];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+#pragma unroll
+          for (int k2 = 0; k2 < NTH; ++k2) {
+            const int e = j * RPT + i + 16 * k2;
+            v[i * NTH + k2] = times_pair(v[i * NTH + k2], buf[(e == 0 ? 0 : n - e) * TK + (f ^ H)], e, row);
+          }
+        __syncthreads();
+      } else {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+#pragma unroll
+          for (int k2 = 0; k2 < NTH; ++k2) v[i * NTH + k2] = times(v[i * NTH + k2], j * RPT + i + 16 * k2);
+      }
+    }
+    fft_b_to_a<T, NR, +1>(v, buf, tw, f, j);
+    if (keep) {
+      hold(v);
+#pragma unroll
+      for (int m = 0; m < 16; ++m)
+        if (j + NTH * m < nout) col[(j + NTH * m) * stride] = v[m];
+    }
+  } else {
+    auto transform = [&](auto dir) {
+      if constexpr (L > 0) lds_fft<(L > 0 ? L : 8), TK, dir.value>(buf, tw);
+      else lds_fft_rt<TK, dir.value, M>(buf, tw, pl);
+    };
+    for (int e = j; e < n; e += NT / TK) buf[f + e * TK] = get(e);
+    __syncthreads();
+    if constexpr (MODE != FC_INV) transform(std::integral_constant<int, -1>{});
+    if (MODE == FC_CONV) {
+      for (int e = j; e < n; e += NT / TK) {
+        if (!pair) {
+          buf[f + e * TK] = times(buf[f + e * TK], e);
+        } else if (f < H) {  // both of the pair
+          const int me = e == 0 ? 0 : n - e;
+          C2<T>&z = buf[f + e * TK], &zm = buf[f + H + me * TK];
+          const C2<T> z0 = z, m0 = zm;
+          z = times_pair(z0, m0, e, row);
+          zm = times_pair(m0, z0, me, row == 0 ? 0 : Ny - row);
+        }
+      }
+      __syncthreads();
+    }
+    if constexpr (MODE != FC_FWD) transform(std::integral_constant<int, +1>{});
+    for (int e = j; e < nout; e += NT / TK)
+      if (keep) col[e * stride] = buf[f + e * TK];
+  }
+}
+
 // ------------------------------------------------------------------ dispatch
 
 template <typename T, int N>
@@ -1116,52 +1229,62 @@ struct ColPass {
       hipLaunchKernelGGL(kern, grid, bt, lds, c.stream, spec, (const C2<T>*)c.tw[AXIS], ncols, AXIS,
                          mode == ZM_INV ? 1 : 0, c.N[1], norm, (const double*)c.cos4[0], (const double*)c.cos4[1],
                          (const double*)c.cos4[2], (const LowModes*)(force ? c.low_dev : nullptr),
-                         c.forcing, c.plan[AXIS], ColFree<T>{});
+                         c.forcing, c.plan[AXIS]);
     };
     if (mode == ZM_POISSON) go(k_fft_col<T, NN, M, true>);
     else go(k_fft_col<T, NN, M, false>);
-  }
-  // a pass of the free-space solve on the padded grid c: others = columns' rows or planes to take
-  static void free_pass(Ctx& c, int mode, int others, const ColFree<T>& fr)
-  {
-    if (c.N[AXIS] <= 256) free_launch<256>(c, mode, others, fr);
-    else if (c.N[AXIS] <= 512) free_launch<512>(c, mode, others, fr);
-    else free_launch<FFT_MAX_N>(c, mode, others, fr);
-  }
-  template <int M>
-  static void free_launch(Ctx& c, int mode, int others, const ColFree<T>& fr)
-  {
-    using CT = ColTile<T, M>;
-    const int ncols = c.N[0] / 2;
-    const dim3 grid((ncols + CT::TK - 1) / CT::TK + 1, others), bt(CT::BT);
-    const size_t lds = (size_t)c.N[AXIS] * CT::TK * sizeof(C2<T>);
-    auto kern = mode == ZM_POISSON ? k_fft_col<T, 0, M, true, true> : k_fft_col<T, 0, M, false, true>;
-    hipLaunchKernelGGL(kern, grid, bt, lds, c.stream, Three<C2<T>>{(C2<T>*)c.spec}, (const C2<T>*)c.tw[AXIS], ncols,
-                       AXIS, mode == ZM_INV ? 1 : 0, c.N[1], 0.0, (const double*)c.cos4[0], (const double*)c.cos4[1],
-                       (const double*)c.cos4[2], (const LowModes*)nullptr, ForcingArgs{}, c.plan[AXIS], fr);
   }
 };
 
 // The free-space solve's x passes on the padded grid: a field of the unpadded one and back.
 template <typename T, int N>
 struct GoXPad {
-  static void go(Ctx& c, const T* src, C2<T>* edge)
+  static void go(Ctx& c, const T* src)
   {
-    const size_t lds = XPass<T, N>::lds(c);
-    hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_PAD, false>), dim3(c.N[1] / 2 / BS, c.N[2] / 2), dim3(NT), lds, c.stream, src, src, src, Three<C2<T>>{(C2<T>*)c.spec},
+    hipLaunchKernelGGL((k_fft_x_fwd<T, N, XSRC_PAD, false>), dim3(c.N[1] / 2 / BS, c.N[2] / 2), dim3(NT),
+                       (XPass<T, N>::lds(c)), c.stream, src, src, src, Three<C2<T>>{(C2<T>*)c.spec},
                        (const C2<T>*)c.tw[0], c.grid(), c.sc, (const int*)nullptr, (const T*)nullptr,
-                       (double*)nullptr, c.plan[0], edge);
+                       (double*)nullptr, c.plan[0]);
   }
 };
 template <typename T, int N>
 struct GoXUnpad {
-  static void go(Ctx& c, T* dst, const C2<T>* edge)
+  static void go(Ctx& c, T* dst)
   {
-    const size_t lds = XPass<T, N>::lds(c);
-    hipLaunchKernelGGL((k_fft_x_inv<T, N, false, true>), dim3(c.N[1] / 2 / BS, c.N[2] / 2), dim3(NT), lds, c.stream, Three<C2<T>>{(C2<T>*)c.spec}, Three<T>{dst},
-                       (const C2<T>*)c.tw[0], c.grid(), c.plan[0], (T*)nullptr, edge);
+    hipLaunchKernelGGL((k_fft_x_inv<T, N, false, true>), dim3(c.N[1] / 2 / BS, c.N[2] / 2), dim3(NT),
+                       (XPass<T, N>::lds(c)), c.stream, Three<C2<T>>{(C2<T>*)c.spec}, Three<T>{dst},
+                       (const C2<T>*)c.tw[0], c.grid(), c.plan[0], (T*)nullptr);
   }
 };
+// A column pass of the free-space solve on the padded grid c, along axis 1 or 2.
+template <typename T, int N>
+struct GoFree {
+  static void go(Ctx& c, int axis, int mode, int others, int nin, int nout)
+  {
+    if constexpr (N >= 64) {
+      launch<N>(c, axis, mode, others, nin, nout);
+    } else {
+      const int n = c.N[axis];
+      if (n <= 256) launch<-256>(c, axis, mode, others, nin, nout);
+      else if (n <= 512) launch<-512>(c, axis, mode, others, nin, nout);
+      else launch<-FFT_MAX_N>(c, axis, mode, others, nin, nout);
+    }
+  }
+  template <int L>
+  static void launch(Ctx& c, int axis, int mode, int others, int nin, int nout)
+  {
+    constexpr int TK = FreeTile<T, L>::TK;
+    const int ncols = c.N[0] / 2;
+    const dim3 grid((ncols + TK - 1) / TK + (mode == FC_CONV ? 1 : 0), others);
+    const size_t lds = L > 0 ? 0 : (size_t)c.N[axis] * TK * sizeof(C2<T>);
+    const size_t nspec = (size_t)ncols * c.N[1] * c.N[2];
+    auto kern = mode == FC_FWD ? k_free_col<T, L, FC_FWD> : (mode == FC_INV ? k_free_col<T, L, FC_INV> : k_free_col<T, L, FC_CONV>);
+    hipLaunchKernelGGL(kern, grid, dim3(NT), lds, c.stream, (C2<T>*)c.spec, (const C2<T>*)c.tw[axis], ncols, axis,
+                       c.N[1], nin, nout, (const double*)c.ghat, (const double*)c.ghat + (mode == FC_CONV ? nspec : 0),
+                       c.plan[axis]);
+  }
+};
+
 // Runtime N -> template N.
 template <template <typename, int> class F, typename T, typename... A>
 static bool dispatch_n(int n, A&&... a)
@@ -1670,7 +1793,7 @@ void unbounded_free(Ctx& c)
 {
   if (!c.unb) return;
   Ctx& p = *c.unb;
-  void* bufs[] = {p.spec, p.spec2, p.rbuf, p.ghat, p.tw[0], p.tw[1], p.tw[2]};
+  void* bufs[] = {p.spec, p.rbuf, p.ghat, p.tw[0], p.tw[1], p.tw[2]};
   for (void* b : bufs)
     if (b) hipFree(b);
   for (auto* q : p.cos4)
@@ -1702,14 +1825,15 @@ static int unbounded_setup_t(Ctx& c)
   p->sc = c.sc;
   if (int rc = fft_setup(*p)) return set_error(c, rc, "poisson_unbounded: " + p->err);
   const size_t nlines = (size_t)p->N[1] * p->N[2], ncols = p->N[0] / 2, nspec = ncols * nlines;
-  // spec2: the kx = Nx/2 column; ghat: its spectrum behind the others'
+  // ghat: the kx = Nx/2 plane behind the others
   if (check_hip(c, hipMalloc(&p->spec, nspec * sizeof(C2<T>)), "hipMalloc unbounded spectrum") ||
-      check_hip(c, hipMalloc(&p->spec2, nlines * sizeof(C2<T>)), "hipMalloc unbounded spectrum") ||
       check_hip(c, hipMalloc(&p->rbuf, p->ncell * sizeof(T)), "hipMalloc unbounded kernel") ||
       check_hip(c, hipMalloc(&p->ghat, (nspec + nlines) * sizeof(double)), "hipMalloc unbounded kernel"))
     return CUP_E_NOMEM;
   hipLaunchKernelGGL((k_green<T>), dim3(p->nb), dim3(NT), 0, c.stream, (T*)p->rbuf, p->grid(), c.h);
-  if (int rc = launch_fft_forward_fields(*p, &p->rbuf, &p->spec, 1)) return set_error(c, rc, "poisson_unbounded: " + p->err);
+  dispatch_x<GoXFwdTo, T>(p->N[0], *p, Three<const T>{(const T*)p->rbuf}, Three<C2<T>>{(C2<T>*)p->spec}, 1);
+  dispatch_n<GoFree, T>(p->N[1], *p, 1, (int)FC_FWD, p->N[2], p->N[1], p->N[1]);
+  dispatch_n<GoFree, T>(p->N[2], *p, 2, (int)FC_FWD, p->N[1], p->N[2], p->N[2]);
   hipLaunchKernelGGL((k_green_real<T>), dim3((unsigned)std::min<size_t>(65536, (nspec + NT - 1) / NT)), dim3(NT), 0,
                      c.stream, (const C2<T>*)p->spec, (double*)p->ghat, (double*)p->ghat + nspec, (int)ncols, nspec,
                      1.0 / ((double)p->N[0] * p->N[1] * p->N[2]));
@@ -1723,10 +1847,9 @@ static int unbounded_setup_t(Ctx& c)
 
 // Only what the convolution needs: the RHS's rows forward along x (a quarter of the padded grid's
 // rows), their planes along y (half), every column along z, forward, times the Green's function and
-// back, the field's half of the planes along y and its quarter of the rows along x. The kx = Nx/2
-// values travel in a column of their own, since the Green's function differs from kx = 0's. Against
-// padding the RHS, transforming the whole padded grid, multiplying and copying the solution out, a
-// solve on 64^3 FP64 cells went from 71 to 47 us.
+// back, the field's half of the planes along y and its quarter of the rows along x. Against padding
+// the RHS, transforming the whole padded grid, multiplying and copying the solution out, a solve on
+// 64^3 cells takes 39 us for 69 in FP64 and 29 for 58 in FP32, on 96^3 133 for 396 and 88 for 262.
 template <typename T>
 static int poisson_unbounded_t(Ctx& c)
 {
@@ -1737,14 +1860,11 @@ static int poisson_unbounded_t(Ctx& c)
     }
   Ctx& p = *c.unb;
   p.stream = c.stream;
-  const size_t nspec = (size_t)(p.N[0] / 2) * p.N[1] * p.N[2];
-  C2<T>* edge = (C2<T>*)p.spec2;
-  const double* G = (const double*)p.ghat;
-  dispatch_x<GoXPad, T>(p.N[0], p, (const T*)c.rbuf, edge);
-  ColPass<T, 0, 1>::free_pass(p, (int)ZM_FWD, c.N[2], ColFree<T>{c.N[1], p.N[1], edge, nullptr, nullptr});
-  ColPass<T, 0, 2>::free_pass(p, (int)ZM_POISSON, p.N[1], ColFree<T>{c.N[2], c.N[2], edge, G, G + nspec});
-  ColPass<T, 0, 1>::free_pass(p, (int)ZM_INV, c.N[2], ColFree<T>{p.N[1], c.N[1], edge, nullptr, nullptr});
-  dispatch_x<GoXUnpad, T>(p.N[0], p, (T*)c.f[CUP_P], (const C2<T>*)edge);
+  dispatch_x<GoXPad, T>(p.N[0], p, (const T*)c.rbuf);
+  dispatch_n<GoFree, T>(p.N[1], p, 1, (int)FC_FWD, c.N[2], c.N[1], p.N[1]);
+  dispatch_n<GoFree, T>(p.N[2], p, 2, (int)FC_CONV, p.N[1], c.N[2], c.N[2]);
+  dispatch_n<GoFree, T>(p.N[1], p, 1, (int)FC_INV, c.N[2], p.N[1], c.N[1]);
+  dispatch_x<GoXUnpad, T>(p.N[0], p, (T*)c.f[CUP_P]);
   return check_hip(c, hipGetLastError(), "poisson_unbounded");
 }
 
