@@ -69,6 +69,7 @@ __device__ __forceinline__ void forcing_planes_wg(const double* __restrict__ row
                                                   void* lds)
 {
   static_assert(NT == 256, "16 slots x 16 row groups");
+  static_assert(LOW_KY == 2, "the sums below are those at ky = 0, 1, 2");
   double(*acc)[16][5] = reinterpret_cast<double(*)[16][5]>(lds);
   const int t = threadIdx.x, sl = t & 15, grp = t >> 4;
   const int ny = Ny / parts, y0 = part * ny;
@@ -100,7 +101,7 @@ __device__ __forceinline__ void forcing_planes_wg(const double* __restrict__ row
 // with a handful of FMAs per cell. Mode m (velocity coefficient c = scale times its mode sums red)
 // contributes c e^{2 pi i (ky y/Ny + kz z/Nz)} to the entries of |kx|: 2 Re at kx = 0, Re and
 // (sign kx) Im at |kx| = 1, 2. Taking a mode with kx < 0 as its conjugate (conj c, -ky, -kz; the
-// real parts are unchanged), the row value is a sum over ky of A_ky(z) e^{2 pi i ky y/Ny} with
+// real parts are unchanged), the row value is a sum over ky = -2 .. 2 (LOW_KY) of A_ky(z) e^{2 pi i ky y/Ny} with
 // A_ky(z) = sum over the modes of that ky of c e^{2 pi i kz z/Nz}: the workgroup of plane z forms
 // B_m = c_m e^{...z} per mode, then the 5 x 3 x 3 sums A (in mode order), then each thread the 16
 // entries of one row from two y twiddles. All in FP64; the phases are conjugates of the twiddles
@@ -113,6 +114,7 @@ __device__ __forceinline__ void forcing_rows_wg(const LowModes* __restrict__ lmp
   double(*B)[3][2] = reinterpret_cast<double(*)[3][2]>(lds);                      // [LOW_MAX][3][2]
   double(*A)[3][3][2] = reinterpret_cast<double(*)[3][3][2]>(B + LOW_MAX);        // [5][3][3][2]
   int(*mk)[3] = reinterpret_cast<int(*)[3]>(reinterpret_cast<double*>(A + 5));   // [LOW_MAX][3]
+  static_assert(LOW_KX == 2 && LOW_KY == 2, "ky = -2 .. 2 and |kx| = 0, 1, 2 below");
   const LowModes& lm = *lmp;
   const int n = lm.n, t = threadIdx.x;
   if (t < n) {

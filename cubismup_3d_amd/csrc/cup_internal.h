@@ -98,7 +98,8 @@ struct FftPlan {
 // Canonical low modes of the band-limited forcing (0 < |k|^2 <= 4, one member of each
 // conjugate pair) and their positions in the packed half spectrum; passed by value.
 constexpr int LOW_MAX = 32;  // modes supported by the fused forcing
-constexpr int LOW_KX = 2;    // largest |kx| among them
+constexpr int LOW_KX = 2;    // largest |kx| among them: the rows' DFTs and synthesis along x
+constexpr int LOW_KY = 2;    // largest |ky|: the planes' DFTs and the row stage's sums (kz: any)
 struct LowModes {
   int n;                  // canonical modes
   int k[LOW_MAX][3];      // (kx, ky, kz) integer wavenumbers
@@ -202,7 +203,7 @@ struct Ctx {
   double* host_red = nullptr;     // pinned scratch for reductions, HOST_RED values
   // forcing: canonical low modes and the fused path's device tables
   int nlow = 0;
-  bool low_fused_ok = false;   // modes fit LowModes (count, |kx|)
+  bool low_fused_ok = false;   // modes fit LowModes (count, |kx|, |ky|)
   LowModes low{};
   LowModes* low_dev = nullptr;  // device copy (kernels index it per lane)
   double* low_part = nullptr;  // x-pass row values [Nz][Ny][16]: per component the row's x-DFT at kx 0..2, |u|^2

@@ -608,7 +608,7 @@ int spectral_setup(Ctx& c)
   c.low = LowModes{};
   c.low_fused_ok = c.nlow > 0 && c.nlow <= LOW_MAX;
   for (int m = 0; m < c.nlow && c.low_fused_ok; ++m)
-    if (std::abs(ks[3 * m]) > LOW_KX) c.low_fused_ok = false;
+    if (std::abs(ks[3 * m]) > LOW_KX || std::abs(ks[3 * m + 1]) > LOW_KY) c.low_fused_ok = false;
   if (!c.low_fused_ok) return CUP_OK;
   LowModes& L = c.low;
   L.n = c.nlow;
