@@ -46,3 +46,28 @@ def test_noalloc_diagnostics_match_the_allocating_entry_point(cup, order):
         # the same kernels over the same partial-sum layout: identical bits
         assert np.array_equal(got, ref)
         G.close()
+
+
+@pytest.mark.parametrize("precision", [4, 8])
+def test_noalloc_diagnostics_of_fields_at_any_element(cup, precision):
+    """The caller's fields need no more alignment than one element."""
+    import torch
+    from cubismup_3d_amd import _lib as L
+    print(f"noalloc diagnostics off by one element: precision {precision}", flush=True)
+    G = cup.Grid((3, 2, 2), precision=precision, decomposition="fused")
+    _random_fields(G, np.random.default_rng(8))
+    ref = G.diagnostics(0.01)
+    ncell = int(np.prod(G.shape))
+    bufs = [torch.empty(ncell + 1, dtype=torch.float32 if precision == 4 else torch.float64, device="cuda")
+            for _ in range(5)]
+    out = torch.full((20,), float("nan"), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    ptrs = [b.data_ptr() + b.element_size() for b in bufs]
+    for n, p in zip(("chi", "u", "v", "w", "p"), ptrs):
+        G._c(L.lib().cup_get_field_device(G._h, L.FIELD_IDS[n], C.c_void_p(p)))
+    d = L.GridDesc((C.c_int * 3)(*G.bpd), float(G.extent.max()), precision, 1, 0)
+    rc = L.lib().cup_diagnostics_noalloc(C.byref(d), (C.c_void_p * 5)(*ptrs), 0.01, C.c_void_p(G.stream()),
+                                         C.c_void_p(out.data_ptr()))
+    assert rc == 0, L.lib().cup_last_error(None)
+    G.synchronize()
+    assert np.array_equal(out.cpu().numpy(), ref)
