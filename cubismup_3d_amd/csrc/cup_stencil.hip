@@ -201,7 +201,8 @@ __device__ __forceinline__ void lab_put(const LabRegs<T, NF>& r, T (*lab)[LabGeo
 // A walk's length trades the halo faces it saves against workgroups: with fewer than a few per CU
 // a launch lasts as long as its longest chain of blocks. Gradient, FP32, 1 / 2 / 4 blocks:
 // 8.3 / 8.8 / 10.8 us on 64^3, 10.6 / 10.9 / 11.5 on 96^3, 17.3 / 16.0 / 16.1 on 128^3,
-// 88.0 / 84.5 / 83.1 on 256^3.
+// 88.0 / 84.5 / 83.1 on 256^3; FP64: 7.4 / 7.8 / 10.1 on 64^3, 12.8 / 12.1 / 11.9 on 96^3, 22.2 / 21.9
+// / 21.6 on 128^3, 66.6 / 64.5 / 66.4 on 192^3.
 // The largest of most, most/2, .. 1 blocks that divides n and leaves at least wgs workgroups.
 inline int walk_blocks(int n, int nb, int most, int wgs)
 {
@@ -540,19 +541,13 @@ __global__ __launch_bounds__(NT) void k_advdiff_xwalk(const T* __restrict__ u, c
   }
 }
 
-template <typename T, int NBW>
+template <typename T, int NBW, bool BC>
 static void launch_advdiff_xwalk(Ctx& c, double nu, const double uinf[3], const StepFold& fold, const Fade6<T>& fd)
 {
-  if (c.periodic())
-    hipLaunchKernelGGL((k_advdiff_xwalk<T, NBW, ADV_PD, false>), dim3(c.nb / NBW), dim3(NT), 0, c.stream,
-                       (const T*)c.f[CUP_U], (const T*)c.f[CUP_V], (const T*)c.f[CUP_W], (T*)c.f[CUP_TMPU],
-                       (T*)c.f[CUP_TMPV], (T*)c.f[CUP_TMPW], c.grid(), c.sc, (T)uinf[0], (T)uinf[1], (T)uinf[2], nu,
-                       fold, fd);
-  else
-    hipLaunchKernelGGL((k_advdiff_xwalk<T, NBW, ADV_PD, true>), dim3(c.nb / NBW), dim3(NT), 0, c.stream,
-                       (const T*)c.f[CUP_U], (const T*)c.f[CUP_V], (const T*)c.f[CUP_W], (T*)c.f[CUP_TMPU],
-                       (T*)c.f[CUP_TMPV], (T*)c.f[CUP_TMPW], c.grid(), c.sc, (T)uinf[0], (T)uinf[1], (T)uinf[2], nu,
-                       fold, fd);
+  hipLaunchKernelGGL((k_advdiff_xwalk<T, NBW, ADV_PD, BC>), dim3(c.nb / NBW), dim3(NT), 0, c.stream,
+                     (const T*)c.f[CUP_U], (const T*)c.f[CUP_V], (const T*)c.f[CUP_W], (T*)c.f[CUP_TMPU],
+                     (T*)c.f[CUP_TMPV], (T*)c.f[CUP_TMPW], c.grid(), c.sc, (T)uinf[0], (T)uinf[1], (T)uinf[2], nu,
+                     fold, fd);
 }
 
 template <typename T>
@@ -577,14 +572,23 @@ static int advdiff_t(Ctx& c, double nu, const double uinf[3], const StepFold* fo
   // on 160 x 96 x 120, 18.5 / 15.8 / 15.6 / 16.5 on 128^3, 130 / 106 / 100 / 106 on 256^3. FP64,
   // whose x faces cost more sectors: 12.1 / 12.4 / 13.1 / 16.6 on 64^3, 19.1 / 17.7 / 14.8 on
   // 96^3, 33.8 / 26.4 / 24.9 / 23.4 on 128^3.
-  // Non-periodic grids take 8 or 2: the compiler keeps some of the 4 and 1 forms' state in scratch
-  // or LDS there (26 against 16 us for 4 against 8 on 128 x 96 x 64 FP64).
-  int nbw = sizeof(T) == 4 ? walk_blocks(c.bpd[0], c.nb, 4, 1024) : walk_blocks(c.bpd[0], c.nb, 8, 256);
-  if (!c.periodic()) nbw = c.bpd[0] % 8 == 0 && c.nb / 8 >= 128 ? 8 : (c.bpd[0] % 2 == 0 ? 2 : 1);
-  if (nbw == 8) launch_advdiff_xwalk<T, 8>(c, nu, uinf, fold, fd);
-  else if (nbw == 4) launch_advdiff_xwalk<T, 4>(c, nu, uinf, fold, fd);
-  else if (nbw == 2) launch_advdiff_xwalk<T, 2>(c, nu, uinf, fold, fd);
-  else launch_advdiff_xwalk<T, 1>(c, nu, uinf, fold, fd);
+  // Non-periodic grids take 2, FP64 ones 8 from 4096 blocks on, and odd block counts 1: the compiler
+  // keeps some of the 4 and 1 forms' state in scratch or LDS there. FP32, 1 / 2 / 4 / 8: 7.4 / 6.6 /
+  // 11.5 / 14.0 us on 64^3, 13.2 / 9.1 / 13.7 / 14.8 on 128 x 96 x 64, 24.8 / 15.0 / 18.8 / 17.1 on
+  // 128^3, 67 / 35.0 / 51 / 37.3 on 192^3; FP64: 19.6 / 7.8 / 18.5 / 15.2 on 64^3, 27.1 / 14.4 / 26.4 /
+  // 16.2 on 128 x 96 x 64, 43 / 27.1 / 36 / 21.6 on 128^3, 116 / 78 / 96 / 73 on 192^3.
+  if (!c.periodic()) {
+    if (sizeof(T) == 8 && c.bpd[0] % 8 == 0 && c.nb / 8 >= 512)
+      launch_advdiff_xwalk<T, sizeof(T) == 8 ? 8 : 2, true>(c, nu, uinf, fold, fd);
+    else if (c.bpd[0] % 2 == 0) launch_advdiff_xwalk<T, 2, true>(c, nu, uinf, fold, fd);
+    else launch_advdiff_xwalk<T, 1, true>(c, nu, uinf, fold, fd);
+    return check_hip(c, hipGetLastError(), "k_advdiff_xwalk");
+  }
+  const int nbw = sizeof(T) == 4 ? walk_blocks(c.bpd[0], c.nb, 4, 1024) : walk_blocks(c.bpd[0], c.nb, 8, 256);
+  if (nbw == 8) launch_advdiff_xwalk<T, 8, false>(c, nu, uinf, fold, fd);
+  else if (nbw == 4) launch_advdiff_xwalk<T, 4, false>(c, nu, uinf, fold, fd);
+  else if (nbw == 2) launch_advdiff_xwalk<T, 2, false>(c, nu, uinf, fold, fd);
+  else launch_advdiff_xwalk<T, 1, false>(c, nu, uinf, fold, fd);
   return check_hip(c, hipGetLastError(), "k_advdiff_xwalk");
 }
 

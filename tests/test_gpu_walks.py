@@ -32,7 +32,7 @@ def test_step(cup, oracle, bpd, scheme):
 BCS = [("dirichlet", "wall", "periodic"), ("wall", "dirichlet", "dirichlet"), ("dirichlet",) * 3]
 
 
-@pytest.mark.parametrize("bpd", [(8, 16, 8), (16, 12, 8), (8, 9, 12), (12, 8, 8), (9, 8, 5)])
+@pytest.mark.parametrize("bpd", [(8, 32, 16), (16, 12, 8), (8, 9, 12), (12, 8, 8), (9, 8, 5)])
 @pytest.mark.parametrize("bc", BCS)
 def test_advection_with_faces(cup, oracle, bpd, bc):
     """The advection's walks of 8, 2 and 1 blocks with open and wall faces, their fades and the inflow
