@@ -308,8 +308,9 @@ __device__ __forceinline__ const C2<T>* lds_twiddles(C2<T>* behind, const C2<T>*
 // --------------------------------------------------------------------- x passes
 
 // N: the row length, or for a length known at run time 0 (up to FFT_MAX_N) or X_SHORT (up to 256,
-// whose butterflies take half the registers, so twice the workgroups share a CU: 18.5 and 12.7 us
-// for the forward and inverse pass on 160 x 96 x 120 FP32 with the larger bound, 14.0 and 8.5 so).
+// whose butterflies take half the registers, so twice the workgroups share a CU: forward and inverse
+// pass in FP32 18.5 and 12.7 us on 160 x 96 x 120 with the larger bound, 14.0 and 8.5 so; 7.8 and 6.0
+// to 6.4 and 5.1 on 48^3, 53 and 35 to 35 and 20 on 192^3; FP64 18.1 and 11.8 to 15.1 and 7.8 on 96^3).
 constexpr int X_SHORT = -256;
 constexpr int x_max(int N) { return N < 0 ? -N : FFT_MAX_N; }
 constexpr int XROWS = 8;         // rows per workgroup = one block row of a z plane
@@ -873,8 +874,7 @@ __device__ __forceinline__ void fft_b_to_a(C2<T> (&v)[16], C2<T>* buf, const C2<
 
 // The column pass of k_fft_col in the register form (same arguments and modes). EXTRA: the
 // grid's first ex.ey rows are workgroups of the forcing's plane stage (1, beside the y forward
-// pass) or row stage (2, beside the z pass; coef is the forcing's coefficient table), in the
-// column tile's LDS.
+// pass) or row stage (2, beside the z pass), in the column tile's LDS.
 template <typename T, int N, int AXIS, int MODE, bool FORCE = false, int EXTRA = 0>
 __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>* __restrict__ tw, int ncols,
                                                  int Ny, int Nz, double norm, const double* __restrict__ cx,
@@ -1497,7 +1497,7 @@ int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_block
 // contraction over each line on the matrix cores; the coefficient (i, j, k) times
 // norm / (denX_i + denY_j + denZ_k) in FP64, the first one zeroed.
 //
-// One workgroup transforms LN lines of N cells: it stages them in LDS as X[j][line] and forms
+// One workgroup transforms LN (16 or 32) lines of N cells: it stages them in LDS as X[j][line] and forms
 // Y = M X in 16 x 16 tiles of the 16x16x4 matrix instruction (M's fragments from the cache, 16
 // columns of j ahead; X's from LDS, two line groups per fragment of M), then stores each tile
 // back over its lines. What bounds it is the latency of M's fragments in the cache, not the
@@ -1705,8 +1705,11 @@ static int mixed_setup(Ctx& c)
   return CUP_OK;
 }
 
-// Lines per workgroup: more of them share each fragment of the matrix, as long as the tile keeps
-// two workgroups on a CU (64 KiB) and the launch has two for every CU; 16 at least.
+// Lines per workgroup: 32 share each fragment of the matrix where the tile keeps two workgroups on a
+// CU (64 KiB) and the launch has two for every CU, 16 otherwise. 16 / 32 lines, x, y and z pass: FP64
+// 26.5 / 23.0, 24.4 / 23.4 and 28.5 / 26.8 us on 128^3, 14.0 / 17.8, 10.6 / 13.8 and 9.5 / 10.3 on
+// 128 x 96 x 64; FP32 16.3 / 17.6, 16.0 / 18.3 and 20.1 / 19.2 on 128^3, 55.8 / 58.6, 63.5 / 60.5 and
+// 68.3 / 67.8 on 192^3. 64 lines, where 64 KiB hold them, are slower (94, 90 and 109 there).
 template <typename T, int AXIS>
 static void r2r_pass(Ctx& c, const T* src, T* dst, int q, double norm, bool divide)
 {
@@ -1717,8 +1720,7 @@ static void r2r_pass(Ctx& c, const T* src, T* dst, int q, double norm, bool divi
                        (const double*)c.mden[2]);
   };
   constexpr size_t cap = 64 * 1024;
-  if (rows >= 512 && r2r_lds<T, 64, AXIS>(n) <= cap) go(k_r2r_axis<T, 64, AXIS>, 64, r2r_lds<T, 64, AXIS>(n));
-  else if (rows >= 256 && r2r_lds<T, 32, AXIS>(n) <= cap) go(k_r2r_axis<T, 32, AXIS>, 32, r2r_lds<T, 32, AXIS>(n));
+  if (rows >= 256 && r2r_lds<T, 32, AXIS>(n) <= cap) go(k_r2r_axis<T, 32, AXIS>, 32, r2r_lds<T, 32, AXIS>(n));
   else go(k_r2r_axis<T, 16, AXIS>, 16, r2r_lds<T, 16, AXIS>(n));
 }
 
@@ -1733,8 +1735,9 @@ static int poisson_mixed_t(Ctx& c)
   r2r_pass<T, 0>(c, (const T*)c.rbuf, a, 0, norm, false);
   r2r_pass<T, 1>(c, a, a, 0, norm, false);
   r2r_pass<T, 2>(c, a, a, 0, norm, true);
-  // the inverse passes go x, y, z: in the reverse order p's error against the
-  // 64-bit restatement after two steps on 128 x 96 x 64 is 5.8e-14, so it is 2.5e-14
+  // The order of the inverse passes is free up to rounding. On the one box where it was measured
+  // (dirichlet, wall, periodic, 128 x 96 x 64 in FP64, two steps) p is off by 2.5e-14 in the order
+  // x, y, z and by 5.8e-14 in the order z, y, x.
   r2r_pass<T, 0>(c, a, a, 1, norm, false);
   r2r_pass<T, 1>(c, a, a, 1, norm, false);
   r2r_pass<T, 2>(c, a, (T*)c.f[CUP_P], 1, norm, false);

@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 # cells per axis / 8. Lines per workgroup are chosen by the other axes' blocks: 16 below 256 of
-# them, 32 from 256, 64 from 512 (where the axis is short enough)
+# them, 32 from 256 (where the axis is short enough)
 CASES = [
     ((1, 1, 1), ("dirichlet", "wall", "periodic")),
     ((3, 5, 9), ("periodic", "dirichlet", "wall")),
