@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cmath>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace cup {
@@ -979,13 +980,6 @@ __global__ __launch_bounds__(NT) void k_fft_colr(Three<C2<T>> spec, const C2<T>*
 
 enum FreeMode { FC_FWD = 0, FC_INV = 1, FC_CONV = 2 };
 
-// L: a length (64 .. 256 in the register form, 512 or 1024 by lds_fft), or minus the bound of a
-// run-time length (lds_fft_rt). 16 elements per thread, or as many columns as 64 KiB of LDS hold.
-template <typename T, int L>
-struct FreeTile {
-  static constexpr int M = L > 0 ? L : -L, TK = L >= 512 ? 65536 / (M * (int)sizeof(C2<T>)) : 16 * NT / M;
-};
-
 // A transform's results, formed where this stands and not in the branches behind it: which product of
 // a sum is rounded depends on the block that the compiler forms the sum in.
 template <typename T>
@@ -1006,46 +1000,94 @@ __device__ __forceinline__ void hold(C2<T> (&v)[16])
 // its own, so the result is theirs bit for bit. After the inflow correction the RHS's sum is rounding
 // noise, and the solve returns it as most of the pressure's mean: another rounding of the solve changes
 // the next step's noise, in FP32 by several times the solve's own error (3e-7 to 1e-5 of |p|).
+struct FreeArgs {
+  int ncols, axis, Ny, nin, nout;
+  const double *green, *green_n;
+};
+
+// Thread (f, j) of a workgroup of TK columns: column f.
+template <typename T, int TK, int MODE>
+struct FreeCol {
+  static constexpr int H = TK / 2;
+  C2<T>* S;
+  C2<T>* col;
+  size_t stride;
+  FreeArgs a;
+  int n, f, row;
+  bool pair, live, keep;
+
+  // false: nothing to do for the workgroup
+  __device__ __forceinline__ bool init(C2<T>* spec, const FreeArgs& args, int length)
+  {
+    a = args;
+    S = spec;
+    n = length;
+    f = threadIdx.x % TK;
+    const int o = blockIdx.y;
+    pair = MODE == FC_CONV && blockIdx.x == gridDim.x - 1;
+    if (pair && o * H > a.Ny / 2) return false;
+    int kx = blockIdx.x * TK + f;
+    row = o;
+    live = keep = kx < a.ncols && !(MODE == FC_CONV && kx == 0);
+    if (pair) {
+      const int k = o * H + f % H, m = k == 0 ? 0 : a.Ny - k;
+      kx = 0;
+      live = k <= a.Ny / 2;
+      row = f < H ? k : m;
+      keep = live && (f < H || m != k);  // a column that is its own mirror is held twice
+    }
+    stride = a.axis == 1 ? (size_t)a.ncols : (size_t)a.Ny * a.ncols;
+    col = S + (a.axis == 1 ? (size_t)row * a.Ny : (size_t)row) * a.ncols + kx;
+    return true;
+  }
+  __device__ __forceinline__ C2<T> get(int e) const { return live && e < a.nin ? col[e * stride] : C2<T>{0, 0}; }
+  __device__ __forceinline__ C2<T> times(const C2<T>& v, int e) const
+  {
+    const double gg = live ? a.green[(col - S) + e * stride] : 0.0;
+    return C2<T>{(T)(v.x * gg), (T)(v.y * gg)};
+  }
+  // Element e of slot 0's column r with zm, element -e of the mirrored column. The pair takes the
+  // Green's function at its lower index, and of each sum one product is rounded, in both elements the
+  // same.
+  __device__ __forceinline__ C2<T> times_pair(const C2<T>& z, const C2<T>& zm, int e, int r) const
+  {
+    const size_t i = (size_t)e * a.Ny + r, m = (size_t)(e == 0 ? 0 : n - e) * a.Ny + (r == 0 ? 0 : a.Ny - r);
+    const size_t g = live ? min(i, m) : 0;
+    const double g0 = a.green[g * a.ncols], gn = a.green_n[g];
+    const double p = 0.5 * (g0 + gn), q = 0.5 * (g0 - gn), x = z.x, y = z.y, xm = zm.x, ym = zm.y;
+    return C2<T>{(T)(i <= m ? fma(p, x, q * xm) : fma(q, xm, p * x)), (T)fma(p, y, -(q * ym))};
+  }
+  // the product of a tile buf[f + e*TK] of slot 0's columns, elements j, j + step, ..
+  __device__ __forceinline__ void times_pairs(C2<T>* buf, int j, int step) const
+  {
+    if (f < H)
+      for (int e = j; e < n; e += step) {
+        const int me = e == 0 ? 0 : n - e;
+        C2<T>&z = buf[f + e * TK], &zm = buf[f + H + me * TK];
+        const C2<T> z0 = z, m0 = zm;
+        z = times_pair(z0, m0, e, row);
+        zm = times_pair(m0, z0, me, row == 0 ? 0 : a.Ny - row);
+      }
+  }
+};
+
+// Lengths L that are powers of two from 64 on: up to 256 in the register form, 512 and 1024 in LDS.
+template <typename T, int L>
+struct FreeTile {
+  static constexpr int TK = L >= 512 ? 65536 / (L * (int)sizeof(C2<T>)) : 16 * NT / L;
+};
+
 template <typename T, int L, int MODE>
-__global__ __launch_bounds__(NT) void k_free_col(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw, int ncols,
-                                                 int axis, int Ny, int nin, int nout,
-                                                 const double* __restrict__ green,
-                                                 const double* __restrict__ green_n, FftPlan pl)
+__global__ __launch_bounds__(NT) void k_free_col(C2<T>* __restrict__ S, const C2<T>* __restrict__ tw, FreeArgs a)
 {
-  constexpr bool REG = L > 0 && ColReg<T, (L > 0 ? L : 8)>::ok;
-  constexpr int M = FreeTile<T, L>::M, TK = FreeTile<T, L>::TK, H = TK / 2, NR = REG ? L : 64;
+  constexpr bool REG = ColReg<T, L>::ok;
+  constexpr int TK = FreeTile<T, L>::TK, NR = REG ? L : 64;
   using CR = ColReg<T, NR>;
   static_assert(!REG || CR::TK == TK, "both forms take as many columns");
-  const int n = L > 0 ? L : pl.n;
-  C2<T>* buf = lds_tile<T, (L > 0 ? L * TK : 0)>();
-  const int o = blockIdx.y, f = threadIdx.x % TK, j = threadIdx.x / TK;
-  const bool pair = MODE == FC_CONV && blockIdx.x == gridDim.x - 1;
-  if (pair && o * H > Ny / 2) return;
-  int kx = blockIdx.x * TK + f, row = o;
-  bool live = kx < ncols && !(MODE == FC_CONV && kx == 0), keep = live;
-  if (pair) {
-    const int k = o * H + f % H, m = k == 0 ? 0 : Ny - k;
-    kx = 0;
-    live = k <= Ny / 2;
-    row = f < H ? k : m;
-    keep = live && (f < H || m != k);  // a column that is its own mirror is held twice
-  }
-  const size_t stride = axis == 1 ? (size_t)ncols : (size_t)Ny * ncols;
-  C2<T>* col = S + (axis == 1 ? (size_t)row * Ny : (size_t)row) * ncols + kx;
-  auto get = [&](int e) { return live && e < nin ? col[e * stride] : C2<T>{0, 0}; };
-  auto times = [&](const C2<T>& v, int e) {
-    const double gg = live ? green[(col - S) + e * stride] : 0.0;
-    return C2<T>{(T)(v.x * gg), (T)(v.y * gg)};
-  };
-  // Element e of slot 0's column row with zm, element -e of the mirrored column. The pair takes the Green's function
-  // at its lower index, and one product of each sum is rounded, the same in both its elements.
-  auto times_pair = [&](const C2<T>& z, const C2<T>& zm, int e, int row) {
-    const size_t i = (size_t)e * Ny + row, m = (size_t)(e == 0 ? 0 : n - e) * Ny + (row == 0 ? 0 : Ny - row);
-    const size_t g = live ? min(i, m) : 0;
-    const double g0 = green[g * ncols], gn = green_n[g];
-    const double a = 0.5 * (g0 + gn), b = 0.5 * (g0 - gn), x = z.x, y = z.y, xm = zm.x, ym = zm.y;
-    return C2<T>{(T)(i <= m ? fma(a, x, b * xm) : fma(b, xm, a * x)), (T)fma(a, y, -(b * ym))};
-  };
+  C2<T>* buf = lds_tile<T, L * TK>();
+  FreeCol<T, TK, MODE> c;
+  if (!c.init(S, a, L)) return;
+  const int f = c.f, j = threadIdx.x / TK;
   if constexpr (REG) {
     constexpr int NTH = CR::NTH, RPT = CR::RPT;
     C2<T> v[16];
@@ -1053,27 +1095,27 @@ __global__ __launch_bounds__(NT) void k_free_col(C2<T>* __restrict__ S, const C2
 #pragma unroll
       for (int i = 0; i < RPT; ++i)
 #pragma unroll
-        for (int k2 = 0; k2 < NTH; ++k2) v[i * NTH + k2] = get(j * RPT + i + 16 * k2);
+        for (int k2 = 0; k2 < NTH; ++k2) v[i * NTH + k2] = c.get(j * RPT + i + 16 * k2);
     } else {
 #pragma unroll
-      for (int m = 0; m < 16; ++m) v[m] = get(j + NTH * m);
+      for (int m = 0; m < 16; ++m) v[m] = c.get(j + NTH * m);
       fft_a_to_b<T, NR, -1>(v, buf, tw, f, j);
     }
     if (MODE == FC_FWD) {
-      if (live)
+      if (c.live)
 #pragma unroll
         for (int i = 0; i < RPT; ++i)
 #pragma unroll
-          for (int k2 = 0; k2 < NTH; ++k2) col[(j * RPT + i + 16 * k2) * stride] = v[i * NTH + k2];
+          for (int k2 = 0; k2 < NTH; ++k2) c.col[(j * RPT + i + 16 * k2) * c.stride] = v[i * NTH + k2];
       return;
     }
     if (MODE == FC_CONV) {
-      if (live) hold(v);
+      if (c.live) hold(v);
       else
 #pragma unroll
         for (int q = 0; q < 16; ++q) v[q] = C2<T>{0, 0};
       __syncthreads();  // the forward transpose's reads of buf are done
-      if (pair) {
+      if (c.pair) {
 #pragma unroll
         for (int i = 0; i < RPT; ++i)
 #pragma unroll
@@ -1084,49 +1126,142 @@ __global__ __launch_bounds__(NT) void k_free_col(C2<T>* __restrict__ S, const C2
 #pragma unroll
           for (int k2 = 0; k2 < NTH; ++k2) {
             const int e = j * RPT + i + 16 * k2;
-            v[i * NTH + k2] = times_pair(v[i * NTH + k2], buf[(e == 0 ? 0 : n - e) * TK + (f ^ H)], e, row);
+            v[i * NTH + k2] = c.times_pair(v[i * NTH + k2], buf[(e == 0 ? 0 : L - e) * TK + (f ^ (TK / 2))], e, c.row);
           }
         __syncthreads();
       } else {
 #pragma unroll
         for (int i = 0; i < RPT; ++i)
 #pragma unroll
-          for (int k2 = 0; k2 < NTH; ++k2) v[i * NTH + k2] = times(v[i * NTH + k2], j * RPT + i + 16 * k2);
+          for (int k2 = 0; k2 < NTH; ++k2) v[i * NTH + k2] = c.times(v[i * NTH + k2], j * RPT + i + 16 * k2);
       }
     }
     fft_b_to_a<T, NR, +1>(v, buf, tw, f, j);
-    if (keep) {
+    if (c.keep) {
       hold(v);
 #pragma unroll
       for (int m = 0; m < 16; ++m)
-        if (j + NTH * m < nout) col[(j + NTH * m) * stride] = v[m];
+        if (j + NTH * m < a.nout) c.col[(j + NTH * m) * c.stride] = v[m];
     }
   } else {
-    auto transform = [&](auto dir) {
-      if constexpr (L > 0) lds_fft<(L > 0 ? L : 8), TK, dir.value>(buf, tw);
-      else lds_fft_rt<TK, dir.value, M>(buf, tw, pl);
-    };
-    for (int e = j; e < n; e += NT / TK) buf[f + e * TK] = get(e);
+    for (int e = j; e < L; e += NT / TK) buf[f + e * TK] = c.get(e);
     __syncthreads();
-    if constexpr (MODE != FC_INV) transform(std::integral_constant<int, -1>{});
+    if constexpr (MODE != FC_INV) lds_fft<L, TK, -1>(buf, tw);
     if (MODE == FC_CONV) {
-      for (int e = j; e < n; e += NT / TK) {
-        if (!pair) {
-          buf[f + e * TK] = times(buf[f + e * TK], e);
-        } else if (f < H) {  // both of the pair
-          const int me = e == 0 ? 0 : n - e;
-          C2<T>&z = buf[f + e * TK], &zm = buf[f + H + me * TK];
-          const C2<T> z0 = z, m0 = zm;
-          z = times_pair(z0, m0, e, row);
-          zm = times_pair(m0, z0, me, row == 0 ? 0 : Ny - row);
-        }
-      }
+      if (c.pair) c.times_pairs(buf, j, NT / TK);
+      else
+        for (int e = j; e < L; e += NT / TK) buf[f + e * TK] = c.times(buf[f + e * TK], e);
       __syncthreads();
     }
-    if constexpr (MODE != FC_FWD) transform(std::integral_constant<int, +1>{});
-    for (int e = j; e < nout; e += NT / TK)
-      if (keep) col[e * stride] = buf[f + e * TK];
+    if constexpr (MODE != FC_FWD) lds_fft<L, TK, +1>(buf, tw);
+    for (int e = j; e < a.nout; e += NT / TK)
+      if (c.keep) c.col[e * c.stride] = buf[f + e * TK];
   }
+}
+
+// Every other length, up to M, in ColTile's form: the first stage reads from global memory and the last
+// writes there, and the product is taken on the last forward stage's registers (slot 0's in LDS).
+// Staging whole columns in LDS took 133 us for a solve on 96^3 FP64 cells, this takes 100.
+template <typename T, int M, int MODE>
+struct FreeStages {
+  using CT = ColTile<T, M>;
+  static constexpr int TK = CT::TK, BT = CT::BT;
+  FreeCol<T, TK, MODE> c;
+  C2<T>* buf;
+  const C2<T>* tw;
+
+  template <int R, int DIR, bool FIRST, bool LAST>
+  __device__ __forceinline__ void stage(int Ns)
+  {
+    constexpr int IT = (CT::E + R - 1) / R;
+    constexpr bool MID = MODE == FC_CONV && DIR < 0 && LAST;  // the forward transform's end: into LDS
+    constexpr bool STORE = LAST && !MID, LOAD = FIRST && !(MODE == FC_CONV && DIR > 0);
+    const int m = c.n / R, NB = TK * m, st = c.n / (Ns * R), f = c.f;
+    const float rNs = 1.0f / (float)Ns;
+    C2<T> v[IT][R];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int t = threadIdx.x + it * BT;
+      if (t >= NB) continue;
+      const int j = t / TK;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[it][r] = LOAD ? c.get(j + r * m) : buf[f + (j + r * m) * TK];
+      if (!FIRST) {
+        const int k = mod_ns(j, Ns, rNs);
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          C2<T> w = tw[r * k * st];
+          if (DIR > 0) w.y = -w.y;
+          v[it][r] = cmul(v[it][r], w);
+        }
+      }
+      dftR<R, DIR>(v[it]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) asm volatile("" : "+v"(v[it][r].x), "+v"(v[it][r].y));  // as hold()
+      if (MID && !c.pair)
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[it][r] = c.times(v[it][r], j + r * m);
+    }
+    if (!LOAD && !STORE) __syncthreads();  // the stage's reads are done
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int t = threadIdx.x + it * BT;
+      if (t >= NB) continue;
+      const int j = t / TK;
+      if (STORE) {
+        if (c.keep)
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+            if (j + r * m < c.a.nout) c.col[(j + r * m) * c.stride] = v[it][r];
+      } else {
+        const int k = FIRST ? 0 : mod_ns(j, Ns, rNs), o = FIRST ? j * R : (j - k) * R + k;
+#pragma unroll
+        for (int r = 0; r < R; ++r) buf[f + (o + r * Ns) * TK] = v[it][r];
+      }
+    }
+    if (!STORE) __syncthreads();
+  }
+
+  template <int DIR, bool LAST>
+  __device__ __forceinline__ void stage_rt(int R, int Ns)
+  {
+    if (R == 8) stage<8, DIR, false, LAST>(Ns);
+    else if (R == 4) stage<4, DIR, false, LAST>(Ns);
+    else if (R == 5) stage<5, DIR, false, LAST>(Ns);
+    else if (R == 3) stage<3, DIR, false, LAST>(Ns);
+    else stage<2, DIR, false, LAST>(Ns);
+  }
+
+  // the plan's radices: the first is 8, and there are two at least (a padded length is 16 x blocks)
+  template <int DIR>
+  __device__ __forceinline__ void transform(const FftPlan& pl)
+  {
+    stage<8, DIR, true, false>(1);
+    int Ns = 8;
+    for (int s = 1; s < pl.ns - 1; ++s) {
+      stage_rt<DIR, false>(pl.r[s], Ns);
+      Ns *= pl.r[s];
+    }
+    stage_rt<DIR, true>(pl.r[pl.ns - 1], Ns);
+  }
+};
+
+template <typename T, int M, int MODE>
+__global__ __launch_bounds__((ColTile<T, M>::BT)) void k_free_col_rt(C2<T>* __restrict__ S,
+                                                                   const C2<T>* __restrict__ tw, FreeArgs a,
+                                                                   FftPlan pl)
+{
+  using FS = FreeStages<T, M, MODE>;
+  FS fs;
+  fs.buf = lds_tile<T, 0>();
+  fs.tw = tw;
+  if (!fs.c.init(S, a, pl.n)) return;
+  if constexpr (MODE != FC_INV) fs.template transform<-1>(pl);
+  if (MODE == FC_CONV && fs.c.pair) {
+    fs.c.times_pairs(fs.buf, threadIdx.x / FS::TK, FS::BT / FS::TK);
+    __syncthreads();
+  }
+  if constexpr (MODE != FC_FWD) fs.template transform<+1>(pl);
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -1261,27 +1396,26 @@ template <typename T, int N>
 struct GoFree {
   static void go(Ctx& c, int axis, int mode, int others, int nin, int nout)
   {
+    const int ncols = c.N[0] / 2, n = c.N[axis];
+    const double* G = (const double*)c.ghat;
+    const FreeArgs a{ncols, axis, c.N[1], nin, nout, G, G + (mode == FC_CONV ? (size_t)ncols * c.N[1] * c.N[2] : 0)};
+    auto grid = [&](int tk) { return dim3((ncols + tk - 1) / tk + (mode == FC_CONV ? 1 : 0), others); };
     if constexpr (N >= 64) {
-      launch<N>(c, axis, mode, others, nin, nout);
+      auto kern = mode == FC_FWD ? k_free_col<T, N, FC_FWD> : (mode == FC_INV ? k_free_col<T, N, FC_INV> : k_free_col<T, N, FC_CONV>);
+      hipLaunchKernelGGL(kern, grid(FreeTile<T, N>::TK), dim3(NT), 0, c.stream, (C2<T>*)c.spec,
+                         (const C2<T>*)c.tw[axis], a);
     } else {
-      const int n = c.N[axis];
-      if (n <= 256) launch<-256>(c, axis, mode, others, nin, nout);
-      else if (n <= 512) launch<-512>(c, axis, mode, others, nin, nout);
-      else launch<-FFT_MAX_N>(c, axis, mode, others, nin, nout);
+      auto launch = [&](auto bound) {
+        constexpr int M = decltype(bound)::value;
+        using CT = ColTile<T, M>;
+        auto kern = mode == FC_FWD ? k_free_col_rt<T, M, FC_FWD> : (mode == FC_INV ? k_free_col_rt<T, M, FC_INV> : k_free_col_rt<T, M, FC_CONV>);
+        hipLaunchKernelGGL(kern, grid(CT::TK), dim3(CT::BT), (size_t)n * CT::TK * sizeof(C2<T>), c.stream,
+                           (C2<T>*)c.spec, (const C2<T>*)c.tw[axis], a, c.plan[axis]);
+      };
+      if (n <= 256) launch(std::integral_constant<int, 256>{});
+      else if (n <= 512) launch(std::integral_constant<int, 512>{});
+      else launch(std::integral_constant<int, FFT_MAX_N>{});
     }
-  }
-  template <int L>
-  static void launch(Ctx& c, int axis, int mode, int others, int nin, int nout)
-  {
-    constexpr int TK = FreeTile<T, L>::TK;
-    const int ncols = c.N[0] / 2;
-    const dim3 grid((ncols + TK - 1) / TK + (mode == FC_CONV ? 1 : 0), others);
-    const size_t lds = L > 0 ? 0 : (size_t)c.N[axis] * TK * sizeof(C2<T>);
-    const size_t nspec = (size_t)ncols * c.N[1] * c.N[2];
-    auto kern = mode == FC_FWD ? k_free_col<T, L, FC_FWD> : (mode == FC_INV ? k_free_col<T, L, FC_INV> : k_free_col<T, L, FC_CONV>);
-    hipLaunchKernelGGL(kern, grid, dim3(NT), lds, c.stream, (C2<T>*)c.spec, (const C2<T>*)c.tw[axis], ncols, axis,
-                       c.N[1], nin, nout, (const double*)c.ghat, (const double*)c.ghat + (mode == FC_CONV ? nspec : 0),
-                       c.plan[axis]);
   }
 };
 
@@ -1852,7 +1986,7 @@ static int unbounded_setup_t(Ctx& c)
 // rows), their planes along y (half), every column along z, forward, times the Green's function and
 // back, the field's half of the planes along y and its quarter of the rows along x. Against padding
 // the RHS, transforming the whole padded grid, multiplying and copying the solution out, a solve on
-// 64^3 cells takes 39 us for 69 in FP64 and 29 for 58 in FP32, on 96^3 133 for 396 and 88 for 262.
+// 64^3 cells takes 39 us for 69 in FP64 and 30 for 58 in FP32, on 96^3 100 for 394 and 70 for 261.
 template <typename T>
 static int poisson_unbounded_t(Ctx& c)
 {
