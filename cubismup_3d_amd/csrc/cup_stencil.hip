@@ -1728,9 +1728,10 @@ __device__ __forceinline__ void star_pair(const T* F, int l, Star<T> (&o)[2])
 }
 
 // KernelDissipation (ComputeDissipation.cpp:46-115): 20 FP64 integrals. A workgroup sums
-// nbw consecutive blocks (one block reduction per workgroup) into part[20*wg], fetching the next
-// block's lab while the current one is summed: about 200 FP64 operations a cell bound it (37 us
-// at 128^3 FP32 with each block fetched, waited for and summed in turn, 34 so).
+// nbw consecutive blocks (one block reduction per workgroup) into part[20*wg]. About 200 FP64 operations
+// a cell and their registers bound it. A block is fetched, waited for and summed in turn: with the next
+// one's lab fetched ahead the FP64 form needs 256 registers, and the call took 162 and 416 us on 192^3 and
+// 200^3 for 125 and 288 so, in FP32 the same either way.
 template <typename T, bool BC>
 __global__ __launch_bounds__(NT) void k_diagnostics(const T* __restrict__ u, const T* __restrict__ v,
                                                     const T* __restrict__ w, const T* __restrict__ p,
@@ -1748,7 +1749,6 @@ __global__ __launch_bounds__(NT) void k_diagnostics(const T* __restrict__ u, con
     lab_fetch<BC>(r, src, s, g, b, {HK_VEL, HK_VEL, HK_VEL, HK_COPY});
     xc = *reinterpret_cast<const V2*>(chi + (size_t)b * BS3 + c0);
   };
-  fetch(b0);
   const double h = g.h, hCube = h * h * h, inv2h = .5 / h, invHh = 1 / (h * h);
   double R[20];
 #pragma unroll
@@ -1757,11 +1757,11 @@ __global__ __launch_bounds__(NT) void k_diagnostics(const T* __restrict__ u, con
     const int b = b0 + j;
     int bx, by, bz;
     block_coords(g, b, bx, by, bz);
+    fetch(b);
     if (j) __syncthreads();  // the previous block is done with the lab
     lab_put<PX_GRAD>(r, lab, s);
     const T xv[2] = {xc.x, xc.y};
     __syncthreads();
-    if (j + 1 < nbw) fetch(b + 1);
     Star<T> su[2], sv[2], sw[2], sp[2];
     star_pair<PX_GRAD>(lab[0], s.li, su);
     star_pair<PX_GRAD>(lab[1], s.li, sv);
@@ -1816,8 +1816,12 @@ __global__ __launch_bounds__(NT) void k_diagnostics(const T* __restrict__ u, con
   block_reduce<20>(R, 0u, part + 20 * (size_t)(b0 / nbw));
 }
 
-// Blocks per diagnostics workgroup: 8 where the x rows allow it and 1024 workgroups remain.
-inline int diag_nbw(int bpdx, long long nb) { return walk_blocks(bpdx, (int)std::min(nb, 1ll << 30), 8, 1024); }
+// Blocks per diagnostics workgroup: up to 8 where the x rows allow it and 256 workgroups remain, since a
+// workgroup's reduction of 20 sums costs as much as a block. The call with 1 / 2 / 4 / 8 blocks, FP32:
+// 24.7 / 25.9 us on 48^3, 28.4 / 26.1 / 28.8 / 34.4 on 64^3, 48.8 / 41.2 / 34.8 on 96^3, 86 / 64 / 52 / 46
+// on 128^3, 502 / 352 / 283 / 231 on 256^3; FP64 28.9 / 26.8 / 29.9 / 37.2 on 64^3, 52 / 43 / 37 on 96^3,
+// 254 / 186 / 152 / 126 on 192^3.
+inline int diag_nbw(int bpdx, long long nb) { return walk_blocks(bpdx, (int)std::min(nb, 1ll << 30), 8, 256); }
 inline int diag_nbw(const Ctx& c) { return diag_nbw(c.bpd[0], c.nb); }
 
 template <typename T>
