@@ -1575,13 +1575,14 @@ int launch_gradp_fused(Ctx& c, const double uinf[3], const int* skip_slot, bool 
 // ------------------------------------------------------------------- reductions
 
 // Component i of partial j at part[j*width + i]; grid (width, nchunk): workgroup (i, c) reduces
-// component i of chunk c of the partials into out[c*width + i]. Each thread keeps 8 loads in
+// component i of chunk c of the partials into out[c*width + i]. Each thread keeps U loads in
 // flight (a single workgroup is bound by the latency of its loads, about 1 ns per partial one
-// load at a time); the lanes' and chunks' order is fixed, so the result is deterministic.
+// load at a time): 8, or 2 where the partials are no more than that, since the 6 that find none cost
+// 0.3 us. The lanes' and chunks' order is fixed, so the result is deterministic.
+template <int U>
 __global__ __launch_bounds__(NT) void k_reduce(const double* __restrict__ part, int n, int width, unsigned maxmask,
                                                double* __restrict__ out)
 {
-  constexpr int U = 8;
   const int i = blockIdx.x;
   const bool ismax = (maxmask >> i) & 1;
   const double none = ismax ? -INFINITY : 0.0;
@@ -1602,6 +1603,8 @@ __global__ __launch_bounds__(NT) void k_reduce(const double* __restrict__ part, 
   block_reduce<1>(a, ismax ? 1u : 0u, out + (size_t)blockIdx.y * width + i);
 }
 
+static auto reduce_form(int n) { return n <= 2 * NT ? k_reduce<2> : k_reduce<8>; }
+
 // Above REDUCE_ONE partials a component is reduced by several workgroups of half as many
 // partials each (more with REDUCE_CHUNKS of them), whose results a second launch reduces: one workgroup
 // took 150 us over the 131072 energy partials of 256^3 and 1.7 ms over the 1048576 of 512^3.
@@ -1613,11 +1616,11 @@ int launch_reduce(Ctx& c, int n, int width, unsigned maxmask, double* out_dev, c
   if (!part) part = c.partials;
   if (n > REDUCE_ONE) {
     const int chunks = std::min(REDUCE_CHUNKS, (n + REDUCE_ONE / 2 - 1) / (REDUCE_ONE / 2));
-    hipLaunchKernelGGL(k_reduce, dim3(width, chunks), dim3(NT), 0, c.stream, part, n, width, maxmask, c.red_part);
+    hipLaunchKernelGGL(k_reduce<8>, dim3(width, chunks), dim3(NT), 0, c.stream, part, n, width, maxmask, c.red_part);
     part = c.red_part;
     n = chunks;
   }
-  hipLaunchKernelGGL(k_reduce, dim3(width), dim3(NT), 0, c.stream, part, n, width, maxmask, out_dev);
+  hipLaunchKernelGGL(reduce_form(n), dim3(width), dim3(NT), 0, c.stream, part, n, width, maxmask, out_dev);
   return check_hip(c, hipGetLastError(), "k_reduce");
 }
 
@@ -1933,7 +1936,7 @@ static int diagnostics_noalloc_t(const void* const fields[5], const GridArgs& g,
                      (const T*)fields[CUP_CHI], g, nu, half_extent[0], half_extent[1], half_extent[2], part, nbw);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_reduce, dim3(20), dim3(NT), 0, s, (const double*)part, g.nb / nbw, 20, 0u, out_dev);
+    hipLaunchKernelGGL(reduce_form(g.nb / nbw), dim3(20), dim3(NT), 0, s, (const double*)part, g.nb / nbw, 20, 0u, out_dev);
     e = hipGetLastError();
   }
   if (e != hipSuccess) return free_error(CUP_E_DEVICE, std::string("diagnostics_noalloc: launch: ") + hipGetErrorString(e));
