@@ -18,6 +18,9 @@
 //   x-inverse : 8 rows per workgroup, complex-to-real, written into a block-layout field.
 // Unnormalized in both directions like FFTW's r2c/c2r; the 1/N^3 and h factors live in the
 // division (PoissonSolverPeriodic.cpp:23-35).
+//
+// Compiled in two halves, for the build's time: the FP64 forms by cup_fft_f64.hip, which includes this
+// file, everything else here.
 #include "cup_internal.h"
 #include "cup_forcing_dev.h"
 
@@ -1511,7 +1514,7 @@ static double poisson_norm(const Ctx& c)
 }
 
 template <typename T>
-static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rate, bool xface)
+int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rate, bool xface)
 {
   const Three<C2<T>> S{(C2<T>*)c.spec};
   const double norm = poisson_norm(c);
@@ -1557,7 +1560,7 @@ static int poisson_fused_t(Ctx& c, bool force, double tke_target, double inj_rat
 
 // The RHS stays in rbuf; the solution goes to p.
 template <typename T>
-static int poisson_plain_t(Ctx& c)
+int poisson_plain_t(Ctx& c)
 {
   const Three<C2<T>> S{(C2<T>*)c.spec};
   const double norm = poisson_norm(c);
@@ -1569,21 +1572,8 @@ static int poisson_plain_t(Ctx& c)
   return check_hip(c, hipGetLastError(), "poisson_plain");
 }
 
-int launch_poisson_fused(Ctx& c, bool force, double tke_target, double inj_rate, bool xface)
-{
-  c.xface_ok = false;
-  if (force && !c.low_fused_ok) return set_error(c, CUP_E_INVALID, "fused forcing: low-mode set not supported");
-  return c.precision == 4 ? poisson_fused_t<float>(c, force, tke_target, inj_rate, xface)
-                          : poisson_fused_t<double>(c, force, tke_target, inj_rate, xface);
-}
-
-int launch_poisson_plain(Ctx& c)
-{
-  return c.precision == 4 ? poisson_plain_t<float>(c) : poisson_plain_t<double>(c);
-}
-
 template <typename T>
-static int fwd_fields_t(Ctx& c, const void* const* real_blocks, void* const* spec, int nf)
+int fwd_fields_t(Ctx& c, const void* const* real_blocks, void* const* spec, int nf)
 {
   Three<const T> s{};
   Three<C2<T>> S{};
@@ -1598,7 +1588,7 @@ static int fwd_fields_t(Ctx& c, const void* const* real_blocks, void* const* spe
 }
 
 template <typename T>
-static int inv_fields_t(Ctx& c, void* const* spec, void* const* real_blocks, int nf)
+int inv_fields_t(Ctx& c, void* const* spec, void* const* real_blocks, int nf)
 {
   Three<T> d{};
   Three<C2<T>> S{};
@@ -1610,18 +1600,6 @@ static int inv_fields_t(Ctx& c, void* const* spec, void* const* real_blocks, int
   dispatch_n<GoY, T>(c.N[1], c, S, nf, (int)ZM_INV, 0.0);
   dispatch_x<GoXInv, T>(c.N[0], c, S, d, nf);
   return check_hip(c, hipGetLastError(), "fft_inverse_fields");
-}
-
-int launch_fft_forward_fields(Ctx& c, const void* const* real_blocks, void* const* spec, int nf)
-{
-  return c.precision == 4 ? fwd_fields_t<float>(c, real_blocks, spec, nf)
-                          : fwd_fields_t<double>(c, real_blocks, spec, nf);
-}
-
-int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_blocks, int nf)
-{
-  return c.precision == 4 ? inv_fields_t<float>(c, spec, real_blocks, nf)
-                          : inv_fields_t<double>(c, spec, real_blocks, nf);
 }
 
 // ------------------------------------------------------- PoissonSolverMixed
@@ -1860,7 +1838,7 @@ static void r2r_pass(Ctx& c, const T* src, T* dst, int q, double norm, bool divi
 
 // The RHS stays in rbuf; the transforms work in the spectrum's buffer and end in p.
 template <typename T>
-static int poisson_mixed_t(Ctx& c)
+int poisson_mixed_t(Ctx& c)
 {
   if (int rc = mixed_setup<T>(c)) return rc;
   T* a = (T*)c.spec;
@@ -1878,13 +1856,6 @@ static int poisson_mixed_t(Ctx& c)
   return check_hip(c, hipGetLastError(), "poisson_mixed");
 }
 
-int launch_poisson_mixed(Ctx& c)
-{
-  return c.precision == 4 ? poisson_mixed_t<float>(c) : poisson_mixed_t<double>(c);
-}
-
-// Twiddle tables e^{-2 pi i t/N} (t < N) per axis and the Poisson cosine tables, built in
-// FP64 on the host.
 // ------------------------------------------------------ PoissonSolverUnbounded
 // PoissonSolverUnbounded::solve (PoissonSolverUnbounded.cpp:126-157): Eastwood and
 // Brownrigg's cyclic convolution of the zero-padded RHS with the free-space Green's function
@@ -1924,19 +1895,6 @@ __global__ void k_green_real(const C2<T>* __restrict__ S, double* __restrict__ G
     G[i] = (double)v.x * norm;
     if (i % ncols == 0) GE[i / ncols] = (double)v.y * norm;
   }
-}
-
-void unbounded_free(Ctx& c)
-{
-  if (!c.unb) return;
-  Ctx& p = *c.unb;
-  void* bufs[] = {p.spec, p.rbuf, p.ghat, p.tw[0], p.tw[1], p.tw[2]};
-  for (void* b : bufs)
-    if (b) hipFree(b);
-  for (auto* q : p.cos4)
-    if (q) hipFree(q);
-  delete c.unb;
-  c.unb = nullptr;
 }
 
 template <typename T>
@@ -1988,7 +1946,7 @@ static int unbounded_setup_t(Ctx& c)
 // the RHS, transforming the whole padded grid, multiplying and copying the solution out, a solve on
 // 64^3 cells takes 39 us for 69 in FP64 and 30 for 58 in FP32, on 96^3 100 for 394 and 70 for 261.
 template <typename T>
-static int poisson_unbounded_t(Ctx& c)
+int poisson_unbounded_t(Ctx& c)
 {
   if (!c.unb)
     if (int rc = unbounded_setup_t<T>(c)) {
@@ -2005,6 +1963,64 @@ static int poisson_unbounded_t(Ctx& c)
   return check_hip(c, hipGetLastError(), "poisson_unbounded");
 }
 
+#ifdef CUP_FFT_F64
+template int poisson_fused_t<double>(Ctx& c, bool force, double tke_target, double inj_rate, bool xface);
+template int poisson_plain_t<double>(Ctx& c);
+template int fwd_fields_t<double>(Ctx& c, const void* const* real_blocks, void* const* spec, int nf);
+template int inv_fields_t<double>(Ctx& c, void* const* spec, void* const* real_blocks, int nf);
+template int poisson_mixed_t<double>(Ctx& c);
+template int poisson_unbounded_t<double>(Ctx& c);
+#else
+extern template int poisson_fused_t<double>(Ctx& c, bool force, double tke_target, double inj_rate, bool xface);
+extern template int poisson_plain_t<double>(Ctx& c);
+extern template int fwd_fields_t<double>(Ctx& c, const void* const* real_blocks, void* const* spec, int nf);
+extern template int inv_fields_t<double>(Ctx& c, void* const* spec, void* const* real_blocks, int nf);
+extern template int poisson_mixed_t<double>(Ctx& c);
+extern template int poisson_unbounded_t<double>(Ctx& c);
+
+int launch_poisson_fused(Ctx& c, bool force, double tke_target, double inj_rate, bool xface)
+{
+  c.xface_ok = false;
+  if (force && !c.low_fused_ok) return set_error(c, CUP_E_INVALID, "fused forcing: low-mode set not supported");
+  return c.precision == 4 ? poisson_fused_t<float>(c, force, tke_target, inj_rate, xface)
+                          : poisson_fused_t<double>(c, force, tke_target, inj_rate, xface);
+}
+
+int launch_poisson_plain(Ctx& c)
+{
+  return c.precision == 4 ? poisson_plain_t<float>(c) : poisson_plain_t<double>(c);
+}
+
+int launch_fft_forward_fields(Ctx& c, const void* const* real_blocks, void* const* spec, int nf)
+{
+  return c.precision == 4 ? fwd_fields_t<float>(c, real_blocks, spec, nf)
+                          : fwd_fields_t<double>(c, real_blocks, spec, nf);
+}
+
+int launch_fft_inverse_fields(Ctx& c, void* const* spec, void* const* real_blocks, int nf)
+{
+  return c.precision == 4 ? inv_fields_t<float>(c, spec, real_blocks, nf)
+                          : inv_fields_t<double>(c, spec, real_blocks, nf);
+}
+
+int launch_poisson_mixed(Ctx& c)
+{
+  return c.precision == 4 ? poisson_mixed_t<float>(c) : poisson_mixed_t<double>(c);
+}
+
+void unbounded_free(Ctx& c)
+{
+  if (!c.unb) return;
+  Ctx& p = *c.unb;
+  void* bufs[] = {p.spec, p.rbuf, p.ghat, p.tw[0], p.tw[1], p.tw[2]};
+  for (void* b : bufs)
+    if (b) hipFree(b);
+  for (auto* q : p.cos4)
+    if (q) hipFree(q);
+  delete c.unb;
+  c.unb = nullptr;
+}
+
 int launch_poisson_unbounded(Ctx& c)
 {
   if (2 * std::max(c.N[0], std::max(c.N[1], c.N[2])) > FFT_MAX_N)
@@ -2012,6 +2028,8 @@ int launch_poisson_unbounded(Ctx& c)
   return c.precision == 4 ? poisson_unbounded_t<float>(c) : poisson_unbounded_t<double>(c);
 }
 
+// Twiddle tables e^{-2 pi i t/N} (t < N) per axis and the Poisson cosine tables, built in
+// FP64 on the host.
 int fft_setup(Ctx& c)
 {
   for (int a = 0; a < 3; ++a) {
@@ -2051,5 +2069,6 @@ int fft_setup(Ctx& c)
   }
   return CUP_OK;
 }
+#endif
 
 }  // namespace cup
