@@ -887,11 +887,12 @@ int cup_run_steps(cup_ctx* ctx, const cup_step_params* p, int nsteps)
     step0 = c.sc_host->step;
   }
   const bool body = c.body.present && p->has_body;
+  const bool masked = c.body.present;  // has_body: whether it is penalized; the RHS is masked whenever it exists
   // The band-limited forcing stays on the device when its low-mode set fits the fused
   // kernels; otherwise the reference decomposition of SpectralForcing runs (host round trip).
   // With a body the forced u* must be in place before the RHS masking reads it (the fused
   // forcing adds its modes after), so the reference decomposition runs then as well.
-  const bool force_fused = p->spectral_forcing && c.low_fused_ok && !body;
+  const bool force_fused = p->spectral_forcing && c.low_fused_ok && !masked;
   struct SkipReset {
     Ctx& c;
     ~SkipReset() { c.timing_skip = false; }
@@ -911,7 +912,7 @@ int cup_run_steps(cup_ctx* ctx, const cup_step_params* p, int nsteps)
       double st[5];
       if (int rc = forcing_plain(c, -1.0, -1.0, p->nu, p->tke_target, p->injection_rate, st)) return rc;
     }
-    if (body)
+    if (masked)
       if (int rc = launch_rhs_obstacle(c, nullptr)) return rc;
     if (int rc = launch_poisson_fused(c, force_fused, p->tke_target, p->injection_rate, true)) return rc;
     stage_mark(c, ST_GRADP, false);

@@ -141,3 +141,27 @@ def test_python_sphere_like_the_reference_test(cup):
     assert ob["mass"] > 0  # a radius of about one cell (h = 2 pi / 64)
     for name in ("u", "v", "w"):
         assert not S.field(name).any(), name
+
+
+@pytest.mark.parametrize("decomposition", ["plain", "fused"])
+@pytest.mark.parametrize("forced", [False, True])
+def test_steps_that_do_not_penalize(cup, oracle, decomposition, forced):
+    """cup_run_steps without has_body while a sphere exists: the RHS is masked, as by
+    cup_pressure_rhs, and nothing is penalized."""
+    print(f"steps without penalization {decomposition} forced={forced}", flush=True)
+    rng = np.random.default_rng(67)
+    bpd, ext = (4, 2, 2), 2 * np.pi
+    G = cup.Grid(bpd, maxextent=ext, precision=8, decomposition=decomposition)
+    O = oracle.OracleSim(bpd, maxextent=ext)
+    centre, R = (0.9 * np.pi, 0.5 * np.pi, 0.5 * np.pi), 0.3 * np.pi
+    G.chi_from_sphere(centre, R)
+    O.sphere_create(R, centre)
+    u = [0.3 * rng.standard_normal(G.shape) + m for m in (1.0, 0.8, -0.9)]
+    G.set_velocity(*u); O.set_velocity(*u)
+    dt, nu, U = 0.2 * G.h, 1e-3, (1.0, 0.0, 0.0)
+    fkw = dict(spectral_forcing=True, injection_rate=0.4) if forced else {}
+    G.run_steps(2, nu=nu, uinf=U, fixed_dt=dt, **fkw)
+    for _ in range(2):
+        O.timestep(dt, nu, uinf=U, **fkw)
+    for a, b in zip(G.velocity(), O.velocity()):
+        assert np.linalg.norm(a - b) < 1e-11 * np.linalg.norm(b)
